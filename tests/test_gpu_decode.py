@@ -52,6 +52,26 @@ def test_balanced_split_and_merge(gpu, workgroups):
     check(wl, workgroups, what=f"workgroups={workgroups}")
 
 
+@pytest.mark.parametrize("hq,hkv", [(24, 4), (10, 2), (20, 1)])
+@pytest.mark.parametrize("parts", [2, 3, 8, 9, 32, 33])
+def test_merge_row_edges(gpu, hq, hkv, parts):
+    """The merge takes one wave per (unit, head) row up to three partials per
+    unit and four waves above, eight partials of a wave at a time: units of
+    about 2, 3, 8, 9, 32 and 33 partials, with rows that do not fill the last
+    workgroup and heads past 16 in a second unit.  Outputs and out_amax (the
+    bits of the largest |out|)."""
+    lens = [1100, 16, 700]
+    wl = small_case(lens, [1] * 3, hq=hq, hkv=hkv, d=256, seed=hq + parts, device=gpu,
+                    dtype=torch.bfloat16)
+    units = 3 * hkv * -(-(hq // hkv) // 16)
+    amax = torch.zeros(1, dtype=torch.int32, device=gpu)
+    out = slot_based_attention(wl.q, wl.k_pool, wl.v_pool, wl.batch, scaling=wl.scale,
+                               decode_workgroups=parts * units + 1, out_amax=amax)
+    torch.cuda.synchronize()
+    assert_attn_close(out, restatement(wl), what=f"{parts} partials per unit")
+    assert int(amax) == int(out.abs().max().view(torch.int16))
+
+
 def test_empty_and_tiny_requests(gpu):
     """L = 1 units next to long ones; many units per workgroup."""
     lens = [1, 2, 4000, 1, 17, 33, 1, 900]

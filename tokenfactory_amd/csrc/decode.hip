@@ -536,31 +536,51 @@ decode_kernel(DecodeArgs a) {
 }
 
 // Merges the partials of every unit owned by more than one workgroup of the
-// streaming kernel; one workgroup per unit. Units of an empty request (L = 0)
-// get zeros, as the reference's fully masked scaled_dot_product_attention
-// returns them (torch's safe softmax: a row with no visible key is all zeros).
-template <bool FP8>
-__global__ void __launch_bounds__(kWaves * kWave)
+// streaming kernel.  WPR waves share one (unit, head) row, 256 dims = 4 per
+// lane: they take the row's partials in turn, kMergeAhead of them in flight per
+// wave, and combine through LDS.  Bound by the latency of those reads.  Few
+// units (a small batch) are cut into many partials each (B = 1, 4 kv heads: 64
+// per unit), so a row gets a whole workgroup; with many units a row has two or
+// three partials and one wave.  One workgroup per unit, each wave walking its
+// share of the partials with all heads in registers, took 19.5 us at B = 1
+// (1531 keys), 11.7 us at B = 16 (with gate and amax) and 6.2 us at B = 64;
+// this takes 6.1, 7.3 and 4.9 us.  Eight waves per workgroup: with four, the
+// amax atomics (one per workgroup on one word) took 1.7 us more at B = 16, with
+// sixteen a launch starts 2 us later.
+// Units of an empty request (L = 0) get zeros, as the reference's fully masked
+// scaled_dot_product_attention returns them (torch's safe softmax: a row with
+// no visible key is all zeros).
+constexpr int kMergeAhead = 8;
+constexpr int kMergeWaves = 8;
+
+template <bool FP8, int WPR>
+__global__ void __launch_bounds__(kMergeWaves * kWave)
 decode_merge_kernel(DecodeArgs a) {
-  __shared__ StateSlot slots[2];
-  __shared__ int32_t red[2][kWaves];
+  constexpr int kRows = kMergeWaves / WPR;   // (unit, head) rows per workgroup
+  __shared__ f32x4 so[kMergeWaves][kWave];   // a wave's O in the partials' order, then dim order
+  __shared__ float sm_m[kMergeWaves], sm_l[kMergeWaves];
+  __shared__ int32_t red[2][kMergeWaves];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = wave_id();
-  const int g = lane >> 4;
-  const int n = lane & 15;
+  const int gmax = min(a.group, 16);
 
   const int units_per_item = a.hkv * a.n_hg;
-  const int u = blockIdx.x;
+  const int64_t row0 = (int64_t)blockIdx.x * kRows;   // first row of the workgroup
+  const int64_t n_rows = (int64_t)a.n_items * units_per_item * gmax;
+  const int64_t row = min<int64_t>(row0 + w / WPR, n_rows - 1);
+  const bool live = row0 + w / WPR < n_rows;
+  const int u = (int)(row / gmax), n = (int)(row - (int64_t)u * gmax);
   const int item = u / units_per_item;
   const int j = u - item * units_per_item;
 
-  // Tiles before this item and in total (block reductions over items).
+  // Tiles before the workgroup's first item and in total (block reductions).
+  const int item0 = (int)(row0 / gmax) / units_per_item;
   int before = 0, total = 0;
-  for (int i = tid; i < a.n_items; i += kWaves * kWave) {
+  for (int i = tid; i < a.n_items; i += kMergeWaves * kWave) {
     const int t = item_tiles(a, i);
     total += t;
-    if (i < item) before += t;
+    if (i < item0) before += t;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -572,56 +592,124 @@ decode_merge_kernel(DecodeArgs a) {
     red[1][w] = total;
   }
   __syncthreads();
-  before = red[0][0] + red[0][1] + red[0][2] + red[0][3];
-  total = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+  before = total = 0;
+#pragma unroll
+  for (int k = 0; k < kMergeWaves; ++k) {
+    before += red[0][k];
+    total += red[1][k];
+  }
+  for (int i = item0; i < item; ++i) before += item_tiles(a, i);
 
   const int hk = j / a.n_hg;
   const int hg = j - hk * a.n_hg;
   const int qrow = a.q_rows ? a.q_rows[item] : (a.items ? a.items[item] : item);
   const int hl = hg * 16 + n;
-  const bool head_ok = hl < a.group;
-  const int hq = hk * a.group + (head_ok ? hl : 0);
-  const float vscale = FP8 ? a.v_scale[0] : 1.f;
+  const int hq = hk * a.group + hl;
   const int Ti = item_tiles(a, item);
 
-  WaveState st;
-  reset_state(st);
-  if (Ti == 0) {
-    // An empty context (seq_len 0) is a row of zeros (the reference's fully
-    // masked attention); padding entries write nothing.
-    if (w == 0) {
-      uint32_t m = 0;
-      if (head_ok && !item_is_padding(a, item)) {
-        st.m = 0.f;
-        st.l = 1.f;   // O = 0
-        m = write_output<FP8>(a, qrow, hq, g, st, 1.f);
-      }
-      amax_commit(a.amax, m);
-    }
-    return;
+  // What this wave does: nothing (a unit the streaming kernel wrote, a padding
+  // item, a head past the group), zeros (an empty context) or a merge.
+  bool write = live && hl < a.group;
+  const bool empty = Ti == 0;
+  int b0 = 0, b1 = -1;
+  if (empty) {
+    write = write && !item_is_padding(a, item);
+  } else {
+    const int64_t N = (int64_t)units_per_item * total;
+    const int64_t p = (int64_t)units_per_item * before + (int64_t)j * Ti;
+    const int P = (int)min<int64_t>(a.n_blocks, N);   // as in the streaming kernel
+    b0 = owner_of(p, N, P);
+    b1 = owner_of(p + Ti - 1, N, P);
+    if (b0 == b1) write = false;   // written directly by the streaming kernel
   }
-  const int64_t N = (int64_t)units_per_item * total;
-  const int64_t p = (int64_t)units_per_item * before + (int64_t)j * Ti;
-  const int P = (int)min<int64_t>(a.n_blocks, N);   // as in the streaming kernel
-  const int b0 = owner_of(p, N, P);
-  const int b1 = owner_of(p + Ti - 1, N, P);
-  if (b0 == b1) return;  // written directly by the streaming kernel
 
-  if (n < min(a.group, 16)) {
-    for (int bb = b0 + w; bb <= b1; bb += kWaves) {
-      const int64_t pp = (int64_t)bb + u;
-      const float* po = a.ws_o + ((pp * 16 + n) * 4 + g) * 64;
-      f32x4 acc2[kAcc];
+  // The row's gate comes in under the partials' latency.
+  u32x2 gv = {0u, 0u};
+  if (write && a.gate)
+    gv = ld_g8(a.gate + (int64_t)qrow * a.gate_stride + (int64_t)hq * a.gate_hstride + 4 * lane);
+  float m = -INFINITY, l = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  if (write && !empty) {
+    for (int bb = b0 + w % WPR; bb <= b1; bb += WPR * kMergeAhead) {
+      f32x4 o[kMergeAhead];
+      float2 ml[kMergeAhead];
 #pragma unroll
-      for (int i = 0; i < kAcc; ++i) acc2[i] = reinterpret_cast<const f32x4*>(po)[i];
-      merge_into(st, a.ws_ml[(pp * 16 + n) * 2 + 0], a.ws_ml[(pp * 16 + n) * 2 + 1], acc2);
+      for (int k = 0; k < kMergeAhead; ++k) {
+        const int64_t pr = ((int64_t)min(bb + WPR * k, b1) + u) * 16 + n;
+        o[k] = reinterpret_cast<const f32x4*>(a.ws_o + pr * kD)[lane];
+        ml[k] = reinterpret_cast<const float2*>(a.ws_ml)[pr];
+      }
+      float mn = m;
+#pragma unroll
+      for (int k = 0; k < kMergeAhead; ++k) {
+        if (bb + WPR * k > b1) ml[k] = float2{-INFINITY, 0.f};   // a repeat of the last one
+        mn = fmaxf(mn, ml[k].x);
+      }
+      if (mn == -INFINITY) continue;
+      const float a1 = fast_exp2(m - mn);
+      acc *= a1;
+      l *= a1;
+#pragma unroll
+      for (int k = 0; k < kMergeAhead; ++k) {
+        const float a2 = fast_exp2(ml[k].x - mn);
+        if (bb + WPR * k <= b1) acc += o[k] * a2;
+        l += ml[k].y * a2;
+      }
+      m = mn;
     }
   }
-  block_merge(slots, w, lane, st);
-  if (w == 0) {
-    const uint32_t m = head_ok ? write_output<FP8>(a, qrow, hq, g, st, vscale) : 0u;
-    amax_commit(a.amax, m);
+  if (WPR > 1) {
+    so[w][lane] = acc;
+    if (lane == 0) {
+      sm_m[w] = m;
+      sm_l[w] = l;
+    }
+    __syncthreads();
+    if (w % WPR) write = false;   // the row's first wave goes on alone
+    if (write) {
+#pragma unroll
+      for (int k = 1; k < WPR; ++k) {
+        const float m2 = sm_m[w + k], l2 = sm_l[w + k];
+        const float mn = fmaxf(m, m2);
+        const float a1 = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+        const float a2 = m2 == -INFINITY ? 0.f : fast_exp2(m2 - mn);
+        acc = acc * a1 + so[w + k][lane] * a2;
+        l = l * a1 + l2 * a2;
+        m = mn;
+      }
+    }
   }
+  uint32_t om = 0;
+  if (write) {
+    // Lane (g, i) = (lane / 16, lane % 16) holds accumulator i of lane group g
+    // (see DecodeArgs' partials); through LDS to dims 4 lane .. + 3.
+    const float inv = empty ? 0.f : (FP8 ? a.v_scale[0] : 1.f) / l;
+    const int g = lane >> 4, i = lane & 15;
+    float* row_f = reinterpret_cast<float*>(&so[w][0]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      row_f[FP8 ? 64 * g + 16 * r + i : 128 * (i >> 3) + 32 * g + 8 * r + (i & 7)] =
+          acc[r] * inv;
+    wave_lds_sync();
+    const f32x4 v = so[w][lane];
+    u32x2 o = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+    if (a.gate) {
+      o[0] = gate_pair(o[0], gv[0]);
+      o[1] = gate_pair(o[1], gv[1]);
+    }
+    om = max(max(o[0] & 0x7fffu, (o[0] >> 16) & 0x7fffu),
+             max(o[1] & 0x7fffu, (o[1] >> 16) & 0x7fffu));
+    *reinterpret_cast<u32x2*>(a.out + (int64_t)qrow * a.out_stride + (int64_t)hq * kD +
+                              4 * lane) = o;
+  }
+  // One atomic per workgroup.
+  if (!a.amax) return;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) om = max(om, (uint32_t)__shfl_xor((int)om, d, kWave));
+  __syncthreads();
+  if (lane == 0) red[0][w] = (int32_t)om;
+  __syncthreads();
+  if (w == 0) amax_commit(a.amax, lane < kMergeWaves ? (uint32_t)red[0][lane] : 0u);
 }
 
 }  // namespace
@@ -792,10 +880,20 @@ int decode_launch(const void* q, int64_t q_row_stride, const void* k_pool, const
     if (rc != TF_OK) return rc;
   }
   if (phases & kPhaseMerge) {
-    if (fp8)
-      hipLaunchKernelGGL(decode_merge_kernel<true>, dim3((unsigned)p.n_units), block, 0, s, a);
+    // kWaves waves per (unit, head) row when the units average more than
+    // three partials each, else one (measured: see decode_merge_kernel).
+    const int64_t rows = p.n_units * p.gmax;
+    const bool wide = (int64_t)p.n_blocks > 2 * p.n_units;
+    const int64_t per_wg = wide ? kMergeWaves / kWaves : kMergeWaves;
+    const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg)), mblock(kMergeWaves * kWave);
+    if (fp8 && wide)
+      hipLaunchKernelGGL((decode_merge_kernel<true, kWaves>), grid, mblock, 0, s, a);
+    else if (fp8)
+      hipLaunchKernelGGL((decode_merge_kernel<true, 1>), grid, mblock, 0, s, a);
+    else if (wide)
+      hipLaunchKernelGGL((decode_merge_kernel<false, kWaves>), grid, mblock, 0, s, a);
     else
-      hipLaunchKernelGGL(decode_merge_kernel<false>, dim3((unsigned)p.n_units), block, 0, s, a);
+      hipLaunchKernelGGL((decode_merge_kernel<false, 1>), grid, mblock, 0, s, a);
     rc = launch_status("tf_attn_decode merge launch");
   }
   return rc;
