@@ -383,9 +383,8 @@ int32_t tf_qk_norm_rope_kv_write(const void* q, int64_t q_token_stride, int64_t 
  * scales (weight_scale_inv None: every scale 1).  bias: bf16 [n] or NULL.
  * out: bf16 [m, n], row stride out_row_stride elements (a multiple of 4),
  * 8-byte aligned.
- * workspace (optional, NULL allowed): when m is small (up to 512) the output
- * tiles alone leave most compute units idle and the call splits K over
- * several workgroups per tile if it gets tf_fp8_block_gemm_workspace_bytes(m,
+ * workspace (optional, NULL allowed): when the output tiles alone leave most
+ * compute units idle the call splits K over several workgroups per tile if it gets tf_fp8_block_gemm_workspace_bytes(m,
  * n, k) bytes of 16-byte aligned scratch (fp32 partials, no initialisation
  * needed; the partials are summed in a fixed order, so results do not depend
  * on timing).  Without it (or when the size query returns 0) one workgroup
@@ -418,6 +417,36 @@ int32_t tf_fp8_block_gemm(const void* xq, int64_t xq_row_stride, const float* x_
                           void* workspace, int64_t workspace_bytes, tf_stream_t stream);
 
 int64_t tf_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
+
+/* tf_fp8_block_gemm_multi: tf_fp8_block_gemm of one activation matrix with up
+ * to TF_FP8_MAX_MATS weight matrices in one launch (a layer's projections of
+ * the same input: full_attention.py:122-139, linear_attention.py:309-314).
+ * Each matrix has its own weight, block scales, bias and output; k, block_h
+ * and block_w are common.  Outputs are those of one call per matrix except
+ * for the order of fp32 sums where the split over K differs.  mats is a host
+ * array, read during the call.  workspace: optional, as there,
+ * tf_fp8_block_gemm_multi_workspace_bytes(m, n of each matrix, n_mats, k).
+ */
+#define TF_FP8_MAX_MATS 4
+
+typedef struct tf_fp8_mat {
+  const void* w;             /* e4m3 [n, k] */
+  int64_t w_row_stride;
+  const float* w_scale;      /* fp32 block scales or NULL */
+  int64_t w_scale_row_stride, w_scale_col_stride;
+  const void* bias;          /* bf16 [n] or NULL */
+  int64_t n;
+  void* out;                 /* bf16 [m, n] */
+  int64_t out_row_stride;
+} tf_fp8_mat;
+
+int32_t tf_fp8_block_gemm_multi(const void* xq, int64_t xq_row_stride, const float* x_scale,
+                                const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h,
+                                int32_t block_w, int64_t m, int64_t k, void* workspace,
+                                int64_t workspace_bytes, tf_stream_t stream);
+
+int64_t tf_fp8_block_gemm_multi_workspace_bytes(int64_t m, const int64_t* n, int32_t n_mats,
+                                                int64_t k);
 
 /* ------------------------------------------------------------------ Gated DeltaNet decode
  * One-token step of the linear-attention (Gated DeltaNet) layers for a batch

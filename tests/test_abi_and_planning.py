@@ -157,3 +157,23 @@ def test_plan_decode_items_lists_single_token_requests():
     assert rows.tolist() == [4, 5, 13]
     with pytest.raises(ValueError):
         plan_decode_items([3, 0])
+
+
+def test_fp8_gemm_workspace_queries_agree():
+    """The size query of a one-matrix call is that of the plain call, a split
+    workspace holds whole fp32 partials of every matrix, and widths that are not
+    multiples of 4 never split."""
+    lib = _native.load()
+    for m in (1, 16, 48, 64, 100, 300, 512, 700, 2000, 9000):
+        for n in (128, 1024, 5120, 5122, 12288):
+            for k in (128, 256, 5120):
+                one = lib.tf_fp8_block_gemm_workspace_bytes(m, n, k)
+                cols = (ctypes.c_int64 * 1)(n)
+                assert lib.tf_fp8_block_gemm_multi_workspace_bytes(m, cols, 1, k) == one
+                assert one % (4 * m * n) == 0 and (n % 4 == 0 or one == 0)
+    cols = (ctypes.c_int64 * 3)(1024, 256, 130)
+    assert lib.tf_fp8_block_gemm_multi_workspace_bytes(48, cols, 3, 5120) == 0
+    cols[2] = 132
+    nbytes = lib.tf_fp8_block_gemm_multi_workspace_bytes(48, cols, 3, 5120)
+    assert nbytes > 0 and nbytes % (4 * 48 * (1024 + 256 + 132)) == 0
+    assert lib.tf_fp8_block_gemm_multi_workspace_bytes(48, cols, 5, 5120) < 0

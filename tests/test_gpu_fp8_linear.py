@@ -284,3 +284,37 @@ def test_gemm_split_k_repeats_bit_identically(gpu):
         else:
             outs[m] = got.clone()
     gemm_case(gpu, 64, 5120, 6144, seed=64)
+
+
+@pytest.mark.parametrize("m", [1, 33, 130, 300, 700, 1100])
+@pytest.mark.parametrize("bias", [False, True])
+def test_projections_of_one_input_in_one_launch(gpu, m, bias):
+    """``fp8_linears`` (one quantisation, one launch over several weights) against
+    the oracle per weight: widths that end inside a tile, split and whole
+    plans.  A linear with a forward hook is called by itself."""
+    ns, k = [1288, 256, 132], 768
+    lins, refs = [], []
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn((m, k), generator=g).to(torch.bfloat16)
+    for n in ns:
+        lin = fl.Fp8Linear(k, n, bias=bias).to(gpu)
+        lin.quantize_from(torch.randn((n, k), generator=g).to(gpu) * k ** -0.5)
+        if bias:
+            lin.bias.copy_(torch.randn(n, generator=g).to(torch.bfloat16))
+        lins.append(lin)
+        refs.append(ofl.block_fp8_linear(x, lin.weight.cpu(), lin.weight_scale_inv.cpu(),
+                                         lin.bias.cpu() if bias else None)[0])
+    print(f"[fp8 gemm] {len(ns)} weights, m={m} bias={bias}", flush=True)
+    outs = fl.fp8_linears(x.to(gpu), lins)
+    torch.cuda.synchronize()
+    for out, ref, n in zip(outs, refs, ns):
+        assert out.shape == (m, n) and out.is_contiguous()
+        # fp32 sums in another order (2^-24 per term) and one bf16 rounding
+        assert torch.allclose(out.cpu().float(), ref, atol=1e-3, rtol=2 ** -8)
+    seen = []
+    lins[1].register_forward_hook(lambda mod, args, out: seen.append(tuple(out.shape)))
+    again = fl.fp8_linears(x.to(gpu), lins)
+    torch.cuda.synchronize()
+    assert seen == [(m, ns[1])]
+    for out, ref in zip(again, refs):
+        assert torch.allclose(out.cpu().float(), ref, atol=1e-3, rtol=2 ** -8)

@@ -125,6 +125,13 @@ SIGNATURES = {
         _p, _i64, _p,                  # workspace, workspace_bytes, stream
     ]),
     "tf_fp8_block_gemm_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "tf_fp8_block_gemm_multi": (_i32, [
+        _p, _i64, _p,                  # xq, xq_row_stride, x_scale
+        _p, _i32, _i32, _i32,          # mats, n_mats, block_h, block_w
+        _i64, _i64,                    # m, k
+        _p, _i64, _p,                  # workspace, workspace_bytes, stream
+    ]),
+    "tf_fp8_block_gemm_multi_workspace_bytes": (_i64, [_i64, _p, _i32, _i64]),
     "tf_gdn_decode": (_i32, [
         _p, _i64, _p, _p, _i64,        # qkv, qkv_row_stride, a, b, ab_row_stride
         _p, _i64,                      # z, z_row_stride
@@ -158,6 +165,17 @@ SIGNATURES = {
 
 SIGNATURES["tf_attn_decode_partial"] = SIGNATURES["tf_attn_decode"]
 SIGNATURES["tf_attn_decode_merge"] = SIGNATURES["tf_attn_decode"]
+
+
+class Fp8Mat(ctypes.Structure):
+    """``tf_fp8_mat``: one weight matrix of ``tf_fp8_block_gemm_multi``."""
+
+    _fields_ = [("w", _p), ("w_row_stride", _i64), ("w_scale", _p),
+                ("w_scale_row_stride", _i64), ("w_scale_col_stride", _i64), ("bias", _p),
+                ("n", _i64), ("out", _p), ("out_row_stride", _i64)]
+
+
+TF_FP8_MAX_MATS = 4
 
 
 class NativeLibraryError(RuntimeError):

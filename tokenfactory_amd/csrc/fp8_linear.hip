@@ -19,9 +19,11 @@
 // v_mfma_f32_16x16x128_f8f6f4 (one instruction covers a whole 128-wide scale
 // block).  A workgroup of 2 x WN waves owns 64 WN output columns x 32 MT rows,
 // a wave holding 64 columns x 16 MT rows (4 x MT 16x16 tiles): 4 waves
-// (128 columns, three K slices in LDS, one wave per SIMD) up to M = 1024,
-// 8 waves (256 columns x 256 or 192 rows, two slices in LDS, two waves per
-// SIMD) above.  Each MFMA starts from zero and its product is folded into the
+// (128 columns x 32, 64, 128 or 256 rows, three K slices in LDS, one wave per
+// SIMD) or 8 waves (256 columns x 256 or 192 rows, two slices in LDS, two waves
+// per SIMD), chosen with the split over K by gemm_plan.  One launch takes up to
+// four weight matrices of the same input (a layer's projections), so a narrow
+// matrix fills the rounds of a wide one.  Each MFMA starts from zero and its product is folded into the
 // fp32 accumulator with that block's scale, acc += p * s, one FMA per
 // accumulator element per 128 of K; a row's folds run between the next row's
 // MFMAs, and each row's operand is read from LDS two rows ahead.  Per
@@ -35,6 +37,8 @@
 // c ^ swz(row) so the operand reads (16 rows x 16 bytes per 16 lanes) hit 16
 // distinct bank groups.  The transposed product makes each lane own four
 // consecutive output columns of a row: the epilogue stores 8 bytes per lane.
+#include <math.h>
+
 #include <algorithm>
 
 #include "tf_common.h"
@@ -172,21 +176,30 @@ struct Tile {
   static_assert(kBM % kRowsPerInst == 0 && kBN % kRowsPerInst == 0, "staging rows");
 };
 
-struct GemmArgs {
-  const uint8_t* xq;      // e4m3 [M, K], row stride xs bytes
-  int64_t xs;
-  const float* x_scale;   // device scalar
+// One weight matrix of a call, its output and its place among the call's
+// columns.
+struct GemmMat {
   const uint8_t* w;       // e4m3 [N, K], row stride wrs bytes
   int64_t wrs;
   const float* wsc;       // fp32 block scales (NULL: all 1)
   int64_t sn, sk;         // their strides (elements)
-  int32_t bh, bw_slices;  // block_h, block_w / 128
   const uint16_t* bias;   // bf16 [N] or NULL
   uint16_t* out;          // bf16 [M, N], row stride os elements
   int64_t os;
-  int32_t M, N, KB, tiles_m;
+  int32_t N, bh;          // columns, block_h
+  int32_t tn0, c0;        // first n-tile and first split-K column of the matrix
+};
+constexpr int kMaxMats = TF_FP8_MAX_MATS;
+
+struct GemmArgs {
+  const uint8_t* xq;      // e4m3 [M, K], row stride xs bytes
+  int64_t xs;
+  const float* x_scale;   // device scalar
+  GemmMat mat[kMaxMats];  // the matrices x is multiplied with (their n-tiles follow each other)
+  int32_t n_mats, bw_slices;   // bw_slices: block_w / 128
+  int32_t M, KB, tiles_m, n_cols;   // n_cols: columns of all matrices
   int32_t tiles, splits;  // split-K: workgroup = (split, tile), K slices split evenly
-  float* part;            // split-K: fp32 [splits, M, N] partial products (NULL: no split)
+  float* part;            // split-K: fp32 [splits, M, n_cols] partial products (NULL: no split)
 };
 
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
@@ -267,8 +280,13 @@ fp8_gemm_kernel(GemmArgs a) {
   const int split = blockIdx.x / a.tiles;
   int tm_i, tn_i;
   xcd_tile(blockIdx.x % a.tiles, a.tiles, a.tiles_m, kGroupM, &tm_i, &tn_i);
+  int mi = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxMats; ++i)
+    if (i < a.n_mats && tn_i >= a.mat[i].tn0) mi = i;
+  const GemmMat mat = a.mat[mi];
   const int m0 = tm_i * T::kBM;
-  const int n0 = tn_i * T::kBN;
+  const int n0 = (tn_i - mat.tn0) * T::kBN;
   // This workgroup's K slices [kb0, kb0 + KB) (all of them without split-K).
   const int kb0 = (int)((int64_t)a.KB * split / a.splits);
   const int KB = (int)((int64_t)a.KB * (split + 1) / a.splits) - kb0;
@@ -288,14 +306,14 @@ fp8_gemm_kernel(GemmArgs a) {
     xo[i] = (uint32_t)min(m0 + T::kRowsPerInst * i + srow, a.M - 1) * (uint32_t)a.xs + cb;
 #pragma unroll
   for (int i = 0; i < T::kWInst; ++i)
-    wo[i] = (uint32_t)min(n0 + T::kRowsPerInst * i + srow, a.N - 1) * (uint32_t)a.wrs + cb;
+    wo[i] = (uint32_t)min(n0 + T::kRowsPerInst * i + srow, mat.N - 1) * (uint32_t)mat.wrs + cb;
   // Without block scales every lane stages x_scale itself and the staged value
   // is used as is; otherwise the staged weight scale times x_scale.  Wave w
   // stages the scales of columns 64 (w % WN) ..; waves w >= WN stage a copy.
-  const bool ones = a.wsc == nullptr;
+  const bool ones = mat.wsc == nullptr;
   const float sfac = ones ? 1.f : xsc;
-  const int scol = min(n0 + 64 * wn + l, a.N - 1);
-  const uint32_t so = ones ? 0u : (uint32_t)((scol / a.bh) * a.sn) * 4u;
+  const int scol = min(n0 + 64 * wn + l, mat.N - 1);
+  const uint32_t so = ones ? 0u : (uint32_t)((scol / mat.bh) * mat.sn) * 4u;
   const uint32_t lds0 = lds_addr(smem);
 
   // Staging instruction idx of K slice kb into stage st: the X rows
@@ -306,9 +324,9 @@ fp8_gemm_kernel(GemmArgs a) {
       dma16(a.xq + (int64_t)kb * kKSlice, xo[idx], sb + idx * 16 * T::kThreads);
     } else if (idx < T::kXInst + T::kWInst) {
       const int i = idx - T::kXInst;
-      dma16(a.w + (int64_t)kb * kKSlice, wo[i], sb + T::kXBytes + i * 16 * T::kThreads);
+      dma16(mat.w + (int64_t)kb * kKSlice, wo[i], sb + T::kXBytes + i * 16 * T::kThreads);
     } else {
-      const float* sbase = ones ? a.x_scale : a.wsc + (int64_t)(kb / a.bw_slices) * a.sk;
+      const float* sbase = ones ? a.x_scale : mat.wsc + (int64_t)(kb / a.bw_slices) * mat.sk;
       dma4(sbase, so, lds0 + st * T::kStage + T::kXBytes + T::kWBytes + w * 256);
     }
   };
@@ -429,12 +447,12 @@ fp8_gemm_kernel(GemmArgs a) {
 #pragma unroll
     for (int tn = 0; tn < 4; ++tn) {
       const int n = n0 + scol4 + 16 * tn;
-      if (n >= a.N) continue;   // N % 4 == 0: four columns in or out together
+      if (n >= mat.N) continue;   // N % 4 == 0: four columns in or out together
 #pragma unroll
       for (int tm = 0; tm < MT; ++tm) {
         const int m = m0 + xrow + 16 * tm;
         if (m < a.M)
-          *reinterpret_cast<f32x4*>(a.part + ((int64_t)split * a.M + m) * a.N + n) = acc[tm][tn];
+          *reinterpret_cast<f32x4*>(a.part + ((int64_t)split * a.M + m) * a.n_cols + mat.c0 + n) = acc[tm][tn];
       }
     }
     return;
@@ -443,18 +461,18 @@ fp8_gemm_kernel(GemmArgs a) {
   for (int tn = 0; tn < 4; ++tn) {
     const int n = n0 + scol4 + 16 * tn;
     float b[4] = {0.f, 0.f, 0.f, 0.f};
-    if (a.bias) {
+    if (mat.bias) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (n + r < a.N) b[r] = __uint_as_float((uint32_t)a.bias[n + r] << 16);
+        if (n + r < mat.N) b[r] = __uint_as_float((uint32_t)mat.bias[n + r] << 16);
     }
 #pragma unroll
     for (int tm = 0; tm < MT; ++tm) {
       const int m = m0 + xrow + 16 * tm;
       if (m >= a.M) continue;
       const f32x4 v = acc[tm][tn];
-      uint16_t* o = a.out + (int64_t)m * a.os + n;
-      if (n + 3 < a.N) {
+      uint16_t* o = mat.out + (int64_t)m * mat.os + n;
+      if (n + 3 < mat.N) {
         u32x2 pk;
         pk[0] = pack_bf16(v[0] + b[0], v[1] + b[1]);
         pk[1] = pack_bf16(v[2] + b[2], v[3] + b[3]);
@@ -462,7 +480,7 @@ fp8_gemm_kernel(GemmArgs a) {
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (n + r < a.N) o[r] = (uint16_t)(pack_bf16(v[r] + b[r], 0.f) & 0xffffu);
+          if (n + r < mat.N) o[r] = (uint16_t)(pack_bf16(v[r] + b[r], 0.f) & 0xffffu);
       }
     }
   }
@@ -473,77 +491,227 @@ fp8_gemm_kernel(GemmArgs a) {
 // loaded before the first add, so the loads' latencies overlap.
 __global__ void __launch_bounds__(kThreads) splitk_reduce_kernel(GemmArgs a) {
   const int64_t e = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
-  const int64_t mn = (int64_t)a.M * a.N;
+  const int64_t mn = (int64_t)a.M * a.n_cols;
   if (e >= mn) return;
-  const int m = (int)(e / a.N), n = (int)(e - (int64_t)m * a.N);
+  const int m = (int)(e / a.n_cols), c = (int)(e - (int64_t)m * a.n_cols);
   f32x4 p[kMaxSplits];
 #pragma unroll
   for (int sp = 0; sp < kMaxSplits; ++sp)
     if (sp < a.splits) p[sp] = *reinterpret_cast<const f32x4*>(a.part + sp * mn + e);
+  int mi = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxMats; ++i)
+    if (i < a.n_mats && c >= a.mat[i].c0) mi = i;
+  const GemmMat& mat = a.mat[mi];
+  const int n = c - mat.c0;
   f32x4 v = p[0];
 #pragma unroll
   for (int sp = 1; sp < kMaxSplits; ++sp)
     if (sp < a.splits) v += p[sp];
   float b[4] = {0.f, 0.f, 0.f, 0.f};
-  if (a.bias) {
+  if (mat.bias) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) b[r] = __uint_as_float((uint32_t)a.bias[n + r] << 16);
+    for (int r = 0; r < 4; ++r) b[r] = __uint_as_float((uint32_t)mat.bias[n + r] << 16);
   }
   u32x2 pk;
   pk[0] = pack_bf16(v[0] + b[0], v[1] + b[1]);
   pk[1] = pack_bf16(v[2] + b[2], v[3] + b[3]);
-  *reinterpret_cast<u32x2*>(a.out + (int64_t)m * a.os + n) = pk;
+  *reinterpret_cast<u32x2*>(mat.out + (int64_t)m * mat.os + n) = pk;
 }
 
-// Tile shape by M: (MT, WN, STAGES).
+// Tile shape (MT, WN) and split-K factor of a call.
 struct Shape {
   int mt, wn;
 };
-Shape gemm_shape(int64_t m, int64_t n) {
-  if (m <= 32) return {1, 2};
-  if (m <= 64) return {2, 2};
-  if (m <= 128) return {4, 2};
-  if (m <= 1024) return {8, 2};
-  // 8 waves, 256 columns, 2 waves per SIMD: 256 or 192 rows, whichever ends
-  // sooner when the tiles run in rounds of one per CU; a 192-row tile takes
-  // 0.8 of a 256-row one (measured at m = 4096, 8320, 21938: 192 rows win at
-  // 4096, 256 at the other two).
-  const int64_t cus = device_cu_count(), tn = (n + 255) / 256;
-  const int64_t r256 = ((m + 255) / 256 * tn + cus - 1) / cus;
-  const int64_t r192 = ((m + 191) / 192 * tn + cus - 1) / cus;
-  return 5 * r256 <= 4 * r192 ? Shape{8, 4} : Shape{6, 4};
+struct GemmPlan {
+  Shape shape;    // with the split factor below
+  int splits;
+  Shape whole;    // without a workspace: no split
+};
+
+// The candidates' times in microseconds: a workgroup of a shape takes
+// fixed + per_slice x K slices, the workgroups run in rounds of one per CU (two
+// of the small ones fit on a CU and then take 1.5 times as long), and a split
+// adds the reduce launch and its partials' way through memory.  Fitted to a
+// sweep of every shape and 1 to 16 splits over M = 1 .. 2000 at N = 1024, 5120,
+// 12288 + 1024 + 1024 and 10240 + 6144, K = 5120 and 6144: the plan's choice is
+// within 9 % of the best one of the sweep everywhere.  A rule by M alone (split
+// only up to M = 512, 256 columns per workgroup above 1024) left most CUs idle
+// where N is small.  From the sweep, that rule's pick and this one's: M = 300,
+// N = 5120 30.1 and 24.9 us; M = 500, N = 5120 32.7 both; M = 1000,
+// N = 10240 + 6144 93.9 and 79.9; M = 128, N = 12288 + 1024 + 1024 34.8 and
+// 28.0.  Three projections (12288, 1024, 1024 columns) at M = 2000 took
+// 152 + 55 + 55 us in launches of their own (44 workgroups for 1024 columns),
+// 164 in one.
+struct ShapeCost {
+  Shape shape;
+  float fixed, per_slice;
+  bool two;        // two workgroups per CU
+};
+constexpr ShapeCost kShapes[] = {{{1, 2}, 3.0f, 0.45f, true},  {{2, 2}, 3.5f, 0.48f, true},
+                                 {{4, 2}, 5.0f, 0.65f, false}, {{8, 2}, 3.0f, 1.10f, false},
+                                 {{6, 4}, 3.0f, 1.62f, false}, {{8, 4}, 3.0f, 1.85f, false}};
+constexpr float kReduceUs = 3.0f, kPartialBytesPerUs = 5e6f;   // written, then read
+
+float gemm_rounds(const ShapeCost& c, int64_t wgs, int64_t cus) {
+  if (!c.two) return (float)((wgs + cus - 1) / cus);
+  const int64_t full = wgs / (2 * cus), rem = wgs - full * 2 * cus;
+  return 1.5f * (float)full + (rem == 0 ? 0.f : rem <= cus ? 1.f : 1.5f);
 }
 
-// Split-K factor: when the output tiles alone leave most CUs idle (M up to 512,
-// the weight-streaming regime), K is split so that the workgroups fill the
-// device's CUs (256 on MI355X) in one round (320 workgroups, one and a quarter
-// rounds, took 1.4 times as long at M = 64).
-int gemm_splits(int64_t m, int64_t n, int64_t k) {
-  const Shape sh = gemm_shape(m, n);
-  if (m > 512 || n % 4) return 1;
-  const int64_t cus = device_cu_count();
-  const int64_t tiles = ((m + 32 * sh.mt - 1) / (32 * sh.mt)) * ((n + 64 * sh.wn - 1) / (64 * sh.wn));
-  const int64_t kb = k / kKSlice;
-  if (tiles >= cus / 2 || kb < 4) return 1;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({kb / 2, cus / tiles, kMaxSplits}));
+GemmPlan gemm_plan(int64_t m, const int64_t* n, int32_t n_mats, int64_t k) {
+  const int64_t cus = device_cu_count(), kb = k / kKSlice;
+  int64_t cols = 0;
+  bool can_split = true;   // the reduce kernel takes four columns of one matrix at a time
+  for (int i = 0; i < n_mats; ++i) {
+    cols += n[i];
+    can_split = can_split && n[i] % 4 == 0;
+  }
+  GemmPlan p{kShapes[0].shape, 1, kShapes[0].shape};
+  float best = INFINITY, best_whole = INFINITY;
+  for (const ShapeCost& c : kShapes) {
+    const int64_t tm = (m + 32 * c.shape.mt - 1) / (32 * c.shape.mt);
+    int64_t tn = 0;
+    for (int i = 0; i < n_mats; ++i) tn += (n[i] + 64 * c.shape.wn - 1) / (64 * c.shape.wn);
+    for (int64_t sp = 1; sp <= kMaxSplits; ++sp) {
+      if (sp > 1 && (!can_split || kb / sp < 2 || tm * tn * sp > 2 * cus)) break;
+      const float us = gemm_rounds(c, tm * tn * sp, cus) *
+                           (c.fixed + c.per_slice * (float)((kb + sp - 1) / sp)) +
+                       (sp > 1 ? kReduceUs + (float)(sp * m * cols) * 8.f / kPartialBytesPerUs
+                               : 0.f);
+      if (us < best) {
+        best = us;
+        p.shape = c.shape;
+        p.splits = (int)sp;
+      }
+      if (sp == 1 && us < best_whole) {
+        best_whole = us;
+        p.whole = c.shape;
+      }
+    }
+  }
+  return p;
 }
 
 template <int MT, int WN, int STAGES>
-void launch_gemm(const GemmArgs& a, hipStream_t stream) {
+void launch_gemm(GemmArgs a, hipStream_t stream) {
   using T = Tile<MT, WN, STAGES>;
-  GemmArgs b = a;
-  b.tiles_m = (a.M + T::kBM - 1) / T::kBM;
-  const int tiles_n = (a.N + T::kBN - 1) / T::kBN;
-  b.tiles = b.tiles_m * tiles_n;
-  const dim3 grid(b.tiles * b.splits), block(T::kThreads);
-  if (a.wsc == nullptr || a.bh % 64 == 0)
-    hipLaunchKernelGGL((fp8_gemm_kernel<MT, WN, STAGES, true>), grid, block, 0, stream, b);
-  else
-    hipLaunchKernelGGL((fp8_gemm_kernel<MT, WN, STAGES, false>), grid, block, 0, stream, b);
-  if (b.part) {
-    const int64_t groups = ((int64_t)a.M * a.N / 4 + kThreads - 1) / kThreads;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((uint32_t)groups), dim3(kThreads), 0, stream, b);
+  a.tiles_m = (a.M + T::kBM - 1) / T::kBM;
+  int tiles_n = 0;
+  bool uni = true;
+  for (int i = 0; i < a.n_mats; ++i) {
+    a.mat[i].tn0 = tiles_n;
+    tiles_n += (a.mat[i].N + T::kBN - 1) / T::kBN;
+    uni = uni && (a.mat[i].wsc == nullptr || a.mat[i].bh % 64 == 0);
   }
+  a.tiles = a.tiles_m * tiles_n;
+  const dim3 grid(a.tiles * a.splits), block(T::kThreads);
+  if (uni)
+    hipLaunchKernelGGL((fp8_gemm_kernel<MT, WN, STAGES, true>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((fp8_gemm_kernel<MT, WN, STAGES, false>), grid, block, 0, stream, a);
+  if (a.part) {
+    const int64_t groups = ((int64_t)a.M * a.n_cols / 4 + kThreads - 1) / kThreads;
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((uint32_t)groups), dim3(kThreads), 0, stream, a);
+  }
+}
+
+void launch_shape(const GemmArgs& a, Shape sh, hipStream_t s) {
+  if (sh.mt == 1)
+    launch_gemm<1, 2, 3>(a, s);
+  else if (sh.mt == 2)
+    launch_gemm<2, 2, 3>(a, s);
+  else if (sh.mt == 4)
+    launch_gemm<4, 2, 3>(a, s);
+  else if (sh.wn == 2)
+    launch_gemm<8, 2, 3>(a, s);
+  else if (sh.mt == 6)
+    launch_gemm<6, 4, 2>(a, s);
+  else
+    launch_gemm<8, 4, 2>(a, s);
+}
+
+// Validates the arguments of both GEMM entry points and launches the call.
+int32_t gemm_call(const char* fn, const void* xq, int64_t xq_row_stride, const float* x_scale,
+                  const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h, int32_t block_w,
+                  int64_t m, int64_t k, void* workspace, int64_t workspace_bytes,
+                  tf_stream_t stream) {
+  if (n_mats < 1 || n_mats > kMaxMats || !mats)
+    return fail(TF_ERR_INVALID, "%s: n_mats=%d (1 to %d)", fn, n_mats, kMaxMats);
+  if (m < 0 || k <= 0 || k % kKSlice)
+    return fail(TF_ERR_INVALID, "%s: m=%lld k=%lld (k a multiple of 128)", fn, (long long)m,
+                (long long)k);
+  if (m > INT32_MAX / 2 || k > INT32_MAX / 2)
+    return fail(TF_ERR_UNSUPPORTED, "%s: dimensions too large", fn);
+  if (xq_row_stride < k || xq_row_stride % 16)
+    return fail(TF_ERR_INVALID, "%s: xq row stride %lld (a multiple of 16 from k up)", fn,
+                (long long)xq_row_stride);
+  if (!x_scale || (m > 0 && !xq)) return fail(TF_ERR_INVALID, "%s: null pointer", fn);
+  if (!aligned16(xq)) return fail(TF_ERR_INVALID, "%s: xq must be 16-byte aligned", fn);
+  if ((m - 1) * xq_row_stride + k > (int64_t)UINT32_MAX)
+    return fail(TF_ERR_UNSUPPORTED, "%s: xq spans more than 4 GiB", fn);
+  GemmArgs a{};
+  a.xq = static_cast<const uint8_t*>(xq);
+  a.xs = xq_row_stride;
+  a.x_scale = x_scale;
+  a.n_mats = n_mats;
+  a.M = (int32_t)m;
+  a.KB = (int32_t)(k / kKSlice);
+  a.bw_slices = 1;
+  int64_t n_of[kMaxMats], cols = 0;
+  for (int i = 0; i < n_mats; ++i) {
+    const tf_fp8_mat& t = mats[i];
+    if (t.n <= 0) return fail(TF_ERR_INVALID, "%s: n=%lld", fn, (long long)t.n);
+    if (t.n > INT32_MAX / 2) return fail(TF_ERR_UNSUPPORTED, "%s: dimensions too large", fn);
+    if (t.w_row_stride < k || t.out_row_stride < t.n || t.w_row_stride % 16 ||
+        t.out_row_stride % 4)
+      return fail(TF_ERR_INVALID,
+                  "%s: row strides %lld/%lld (fp8 rows 16-byte, out rows 8-byte multiples)", fn,
+                  (long long)t.w_row_stride, (long long)t.out_row_stride);
+    if (!t.w || (m > 0 && !t.out)) return fail(TF_ERR_INVALID, "%s: null pointer", fn);
+    if (!aligned16(t.w) || !aligned8(t.out) || (reinterpret_cast<uintptr_t>(t.bias) & 1u))
+      return fail(TF_ERR_INVALID, "%s: w 16-byte, out 8-byte aligned", fn);
+    if (t.w_scale && (block_h <= 0 || block_w <= 0 || block_w % kKSlice))
+      return fail(TF_ERR_UNSUPPORTED, "%s: block_h=%d block_w=%d (block_w a multiple of 128)",
+                  fn, block_h, block_w);
+    if ((t.n - 1) * t.w_row_stride + k > (int64_t)UINT32_MAX ||
+        (t.w_scale && ((t.n - 1) / block_h) * t.w_scale_row_stride > (int64_t)(UINT32_MAX / 4)))
+      return fail(TF_ERR_UNSUPPORTED, "%s: w or w_scale spans more than 4 GiB", fn);
+    GemmMat& g = a.mat[i];
+    g.w = static_cast<const uint8_t*>(t.w);
+    g.wrs = t.w_row_stride;
+    g.wsc = t.w_scale;
+    g.sn = t.w_scale_row_stride;
+    g.sk = t.w_scale_col_stride;
+    g.bh = t.w_scale ? block_h : 1;
+    if (t.w_scale) a.bw_slices = block_w / kKSlice;
+    g.bias = static_cast<const uint16_t*>(t.bias);
+    g.out = static_cast<uint16_t*>(t.out);
+    g.os = t.out_row_stride;
+    g.N = (int32_t)t.n;
+    g.c0 = (int32_t)cols;
+    n_of[i] = t.n;
+    cols += t.n;
+  }
+  if (cols > INT32_MAX / 2) return fail(TF_ERR_UNSUPPORTED, "%s: dimensions too large", fn);
+  if (m == 0) return TF_OK;
+  a.n_cols = (int32_t)cols;
+  a.splits = 1;
+  // Split-K when a large enough 16-byte aligned workspace comes with the call;
+  // otherwise (or when it does not pay) one workgroup per output tile.
+  const GemmPlan p = gemm_plan(m, n_of, n_mats, k);
+  Shape sh = p.shape;
+  if (p.splits > 1) {
+    if (workspace && !(reinterpret_cast<uintptr_t>(workspace) & 15u) &&
+        workspace_bytes >= (int64_t)p.splits * m * cols * 4) {
+      a.splits = p.splits;
+      a.part = static_cast<float*>(workspace);
+    } else {
+      sh = p.whole;
+    }
+  }
+  launch_shape(a, sh, reinterpret_cast<hipStream_t>(stream));
+  return launch_status("tf_fp8_block_gemm launch");
 }
 
 // Validates the arguments both quantisation entry points share and fills a.
@@ -629,6 +797,34 @@ int32_t tf_fp8_act_quant_amax(const void* x, int32_t x_dtype, int64_t rows, int6
   return launch_status("tf_fp8_act_quant_amax launch");
 }
 
+int32_t tf_fp8_block_gemm_multi(const void* xq, int64_t xq_row_stride, const float* x_scale,
+                                const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h,
+                                int32_t block_w, int64_t m, int64_t k, void* workspace,
+                                int64_t workspace_bytes, tf_stream_t stream) {
+  using namespace tfa;
+  clear_error();
+  return gemm_call("fp8_block_gemm_multi", xq, xq_row_stride, x_scale, mats, n_mats, block_h,
+                   block_w, m, k, workspace, workspace_bytes, stream);
+}
+
+int64_t tf_fp8_block_gemm_multi_workspace_bytes(int64_t m, const int64_t* n, int32_t n_mats,
+                                                int64_t k) {
+  using namespace tfa;
+  clear_error();
+  if (m < 0 || n_mats < 1 || n_mats > kMaxMats || !n || k <= 0 || k % kKSlice)
+    return fail(TF_ERR_INVALID, "fp8_block_gemm_multi_workspace_bytes: m=%lld n_mats=%d k=%lld",
+                (long long)m, n_mats, (long long)k);
+  int64_t cols = 0;
+  for (int i = 0; i < n_mats; ++i) {
+    if (n[i] <= 0 || n[i] > INT32_MAX / 2)
+      return fail(TF_ERR_INVALID, "fp8_block_gemm_multi_workspace_bytes: n[%d]=%lld", i,
+                  (long long)n[i]);
+    cols += n[i];
+  }
+  const int splits = gemm_plan(m, n, n_mats, k).splits;
+  return splits > 1 ? (int64_t)splits * m * cols * 4 : 0;
+}
+
 int32_t tf_fp8_block_gemm(const void* xq, int64_t xq_row_stride, const float* x_scale,
                           const void* w, int64_t w_row_stride, const float* w_scale,
                           int64_t w_scale_row_stride, int64_t w_scale_col_stride,
@@ -637,75 +833,10 @@ int32_t tf_fp8_block_gemm(const void* xq, int64_t xq_row_stride, const float* x_
                           void* workspace, int64_t workspace_bytes, tf_stream_t stream) {
   using namespace tfa;
   clear_error();
-  if (m < 0 || n <= 0 || k <= 0 || k % kKSlice)
-    return fail(TF_ERR_INVALID, "fp8_block_gemm: m=%lld n=%lld k=%lld (k a multiple of 128)",
-                (long long)m, (long long)n, (long long)k);
-  if (m > INT32_MAX / 2 || n > INT32_MAX / 2 || k > INT32_MAX / 2)
-    return fail(TF_ERR_UNSUPPORTED, "fp8_block_gemm: dimensions too large");
-  if (xq_row_stride < k || w_row_stride < k || out_row_stride < n || xq_row_stride % 16 ||
-      w_row_stride % 16 || out_row_stride % 4)
-    return fail(TF_ERR_INVALID,
-                "fp8_block_gemm: row strides %lld/%lld/%lld (fp8 rows 16-byte, out rows "
-                "8-byte multiples)",
-                (long long)xq_row_stride, (long long)w_row_stride, (long long)out_row_stride);
-  if (!w || !x_scale || (m > 0 && (!xq || !out)))
-    return fail(TF_ERR_INVALID, "fp8_block_gemm: null pointer");
-  if (!aligned16(xq) || !aligned16(w) || !aligned8(out) ||
-      (reinterpret_cast<uintptr_t>(bias) & 1u))
-    return fail(TF_ERR_INVALID, "fp8_block_gemm: xq / w 16-byte, out 8-byte aligned");
-  if (w_scale && (block_h <= 0 || block_w <= 0 || block_w % kKSlice))
-    return fail(TF_ERR_UNSUPPORTED,
-                "fp8_block_gemm: block_h=%d block_w=%d (block_w a multiple of 128)", block_h,
-                block_w);
-  if (m == 0) return TF_OK;
-  if ((m - 1) * xq_row_stride + k > (int64_t)UINT32_MAX ||
-      (n - 1) * w_row_stride + k > (int64_t)UINT32_MAX ||
-      (w_scale && ((n - 1) / block_h) * w_scale_row_stride > (int64_t)(UINT32_MAX / 4)))
-    return fail(TF_ERR_UNSUPPORTED, "fp8_block_gemm: xq, w or w_scale spans more than 4 GiB");
-  GemmArgs a;
-  a.xq = static_cast<const uint8_t*>(xq);
-  a.xs = xq_row_stride;
-  a.x_scale = x_scale;
-  a.w = static_cast<const uint8_t*>(w);
-  a.wrs = w_row_stride;
-  a.wsc = w_scale;
-  a.sn = w_scale_row_stride;
-  a.sk = w_scale_col_stride;
-  a.bh = w_scale ? block_h : 1;
-  a.bw_slices = w_scale ? block_w / kKSlice : 1;
-  a.bias = static_cast<const uint16_t*>(bias);
-  a.out = static_cast<uint16_t*>(out);
-  a.os = out_row_stride;
-  a.M = (int32_t)m;
-  a.N = (int32_t)n;
-  a.KB = (int32_t)(k / kKSlice);
-  a.tiles_m = 0;
-  a.tiles = 0;
-  a.splits = 1;
-  a.part = nullptr;
-  // Split-K when a large enough 16-byte aligned workspace comes with the call;
-  // otherwise (or when it does not pay) one workgroup per output tile.
-  const int splits = gemm_splits(m, n, k);
-  if (splits > 1 && workspace && !(reinterpret_cast<uintptr_t>(workspace) & 15u) &&
-      workspace_bytes >= (int64_t)splits * m * n * 4) {
-    a.splits = splits;
-    a.part = static_cast<float*>(workspace);
-  }
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const Shape sh = gemm_shape(m, n);
-  if (sh.mt == 1)
-    launch_gemm<1, 2, 3>(a, s);
-  else if (sh.mt == 2)
-    launch_gemm<2, 2, 3>(a, s);
-  else if (sh.mt == 4)
-    launch_gemm<4, 2, 3>(a, s);
-  else if (sh.wn == 2)
-    launch_gemm<8, 2, 3>(a, s);
-  else if (sh.mt == 6)
-    launch_gemm<6, 4, 2>(a, s);
-  else
-    launch_gemm<8, 4, 2>(a, s);
-  return launch_status("tf_fp8_block_gemm launch");
+  const tf_fp8_mat mat = {w, w_row_stride, w_scale, w_scale_row_stride, w_scale_col_stride,
+                          bias, n, out, out_row_stride};
+  return gemm_call("fp8_block_gemm", xq, xq_row_stride, x_scale, &mat, 1, block_h, block_w, m, k,
+                   workspace, workspace_bytes, stream);
 }
 
 int64_t tf_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
@@ -714,7 +845,7 @@ int64_t tf_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m < 0 || n <= 0 || k <= 0 || k % kKSlice)
     return fail(TF_ERR_INVALID, "fp8_block_gemm_workspace_bytes: m=%lld n=%lld k=%lld",
                 (long long)m, (long long)n, (long long)k);
-  const int splits = gemm_splits(m, n, k);
+  const int splits = gemm_plan(m, &n, 1, k).splits;
   return splits > 1 ? (int64_t)splits * m * n * 4 : 0;
 }
 

@@ -16,6 +16,7 @@ There is no non-native path: without the library every call raises.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import math
 from typing import Optional, Sequence
 
@@ -176,6 +177,63 @@ def block_fp8_linear(x: torch.Tensor, weight: torch.Tensor,
     out = block_fp8_gemm(xq, scale, weight, weight_scale_inv, bias, block_h, block_w,
                          stream=stream)
     return out.reshape(*x.shape[:-1], weight.shape[0])
+
+
+def _plain(linear) -> bool:
+    """Whether calling ``linear`` runs ``Fp8Linear.forward`` and nothing else (no
+    subclass, replaced forward or hook)."""
+    return (type(linear) is Fp8Linear and "forward" not in linear.__dict__
+            and not (linear._forward_hooks or linear._forward_pre_hooks
+                     or linear._backward_hooks or linear._backward_pre_hooks
+                     or nn.modules.module._has_any_global_hook()))
+
+
+def fp8_linears(x: torch.Tensor, linears: Sequence["Fp8Linear"]):
+    """``[lin(x) for lin in linears]`` for projections of the same input
+    (``full_attention.py:122-139``, ``linear_attention.py:309-314``): x is
+    quantised once and one ``tf_fp8_block_gemm_multi`` launch multiplies it with
+    every weight.  Linears that do not share a block size and a K that is a
+    multiple of 128, or that are more than plain ``Fp8Linear`` calls, are called
+    one by one."""
+    first = linears[0]
+    k = first.in_features
+    if (len(linears) > _native.TF_FP8_MAX_MATS or k % K_SLICE or x.shape[-1] != k
+            or not x.is_cuda or x.dtype != torch.bfloat16
+            or not all(_plain(m) and m.in_features == k and m.block_h == first.block_h
+                       and m.block_w == first.block_w and m.weight.is_contiguous()
+                       and m.weight.dtype == torch.float8_e4m3fn
+                       and m.weight.device == x.device
+                       and m.weight_scale_inv.dtype == torch.float32
+                       and m.weight_scale_inv.device == x.device
+                       and (m.bias is None or (m.bias.dtype == torch.bfloat16
+                                               and m.bias.is_contiguous()
+                                               and m.bias.device == x.device))
+                       for m in linears)):
+        return [m(x) for m in linears]
+    x2d = x.reshape(-1, k)
+    if x2d.stride(1) != 1:
+        x2d = x2d.contiguous()
+    rows = x2d.shape[0]
+    xq, scale = quantize_activations(x2d)
+    outs = [torch.empty((rows, m.out_features), dtype=torch.bfloat16, device=x.device)
+            for m in linears]
+    if rows:
+        n = len(linears)
+        mats = (_native.Fp8Mat * n)()
+        cols = (ctypes.c_int64 * n)()
+        for i, (m, out) in enumerate(zip(linears, outs)):
+            ws = m.weight_scale_inv
+            mats[i] = _native.Fp8Mat(_ptr(m.weight), k, _ptr(ws), ws.stride(0), ws.stride(1),
+                                     _ptr(m.bias), m.out_features, _ptr(out), m.out_features)
+            cols[i] = m.out_features
+        nbytes = _native.load().tf_fp8_block_gemm_multi_workspace_bytes(rows, cols, n, k)
+        if nbytes < 0:
+            raise ValueError("fp8_linears: bad shape")
+        scratch = torch.empty((nbytes,), dtype=torch.uint8, device=x.device) if nbytes else None
+        _native.call("tf_fp8_block_gemm_multi", _ptr(xq), xq.stride(0), _ptr(scale), mats, n,
+                     first.block_h, first.block_w, rows, k, _ptr(scratch), nbytes,
+                     _stream_ptr(None, x.device))
+    return [out.reshape(*x.shape[:-1], out.shape[1]) for out in outs]
 
 
 class Fp8Linear(nn.Module):

@@ -30,7 +30,7 @@ import torch
 import torch.nn as nn
 
 from .attention import qk_norm_rope_kv_write, slot_based_attention
-from .fp8_linear import Fp8Linear
+from .fp8_linear import Fp8Linear, fp8_linears
 
 
 def _fp8_block_size(config):
@@ -148,14 +148,18 @@ class FullAttention(nn.Module):
     def forward(self, hidden_states: torch.Tensor, positions: torch.Tensor, cache_pool,
                 forward_batch) -> torch.Tensor:
         n_tok = hidden_states.shape[0]
-        if self.attn_output_gate:
-            qg = self.q_proj(hidden_states).view(n_tok, self.num_heads, 2 * self.head_dim)
-            q, gate = qg.chunk(2, dim=-1)   # gate stays a [T, Hq, D] view of qg
+        projections = (self.q_proj, self.k_proj, self.v_proj)
+        if all(isinstance(p, Fp8Linear) for p in projections):
+            q, k, v = fp8_linears(hidden_states, projections)
         else:
-            q = self.q_proj(hidden_states).view(n_tok, self.num_heads, self.head_dim)
-            gate = None
-        k = self.k_proj(hidden_states).view(n_tok, self.num_kv_heads, self.head_dim)
-        v = self.v_proj(hidden_states).view(n_tok, self.num_kv_heads, self.head_dim)
+            q, k, v = (p(hidden_states) for p in projections)
+        if self.attn_output_gate:
+            # gate stays a [T, Hq, D] view of the q projection
+            q, gate = q.view(n_tok, self.num_heads, 2 * self.head_dim).chunk(2, dim=-1)
+        else:
+            q, gate = q.view(n_tok, self.num_heads, self.head_dim), None
+        k = k.view(n_tok, self.num_kv_heads, self.head_dim)
+        v = v.view(n_tok, self.num_kv_heads, self.head_dim)
 
         k_buf, v_buf = cache_pool.get_full_kv_buffers(self.layer_idx)
         scales = (cache_pool.get_full_kv_scales(self.layer_idx)

@@ -24,7 +24,7 @@ import torch
 import torch.nn as nn
 
 from . import _native
-from .fp8_linear import Fp8Linear, on_stream
+from .fp8_linear import Fp8Linear, fp8_linears, on_stream
 
 HEAD_DIM = 128      # the tuned kernels' head dims (key and value)
 MAX_OTHER_HEAD_DIM = 64   # other head dims: multiples of 4 up to this (one wave per head)
@@ -217,8 +217,11 @@ class LinearAttention(nn.Module):
         return self._packed
 
     def forward(self, hidden_states: torch.Tensor, cache_pool, forward_batch) -> torch.Tensor:
-        qkv = self.in_proj_qkv(hidden_states)
-        z = self.in_proj_z(hidden_states)
+        wide = (self.in_proj_qkv, self.in_proj_z)
+        if all(isinstance(p, Fp8Linear) for p in wide):
+            qkv, z = fp8_linears(hidden_states, wide)
+        else:
+            qkv, z = (p(hidden_states) for p in wide)
         b = self.in_proj_b(hidden_states)
         a = self.in_proj_a(hidden_states)
         conv_state, ssm_state = cache_pool.get_linear_states(self.layer_idx)
