@@ -270,6 +270,46 @@ int32_t tf_attn_plan_device(const int64_t* extend_lens, int32_t batch_size,
                             int32_t work_capacity, int32_t* dec_items, int32_t* dec_rows,
                             int32_t dec_capacity, int32_t* status, tf_stream_t stream);
 
+/* tf_attn_rows: the decode entry point's streaming kernel over blocks of query
+ * rows (several tokens of a request, or several heads of one token, side by
+ * side on one pass over its keys; full_attention.py:215-283), and over any
+ * head_dim that is a multiple of 8 up to 256 (of 16 for an fp8 pool).
+ * blocks: device int32 [n_items][4] = {b, q row of the request's first new
+ * token, ext, row0}, 16-byte aligned: rows row0 .. row0 + 16 row_groups - 1 of
+ * the request's ext * G (row = t * G + h, token t sees keys up to
+ * seq_lens[b] - ext + t); b = -1 is padding.  NULL: item i is request i with one
+ * token at q row i (at most 2048), every head of it.  row_groups: 1 without
+ * blocks; 1 or 2 (2 at head dims other than 256) with them.  The other arguments are tf_attn_decode's;
+ * workspace: tf_attn_rows_workspace_bytes of the same sizes, 16-byte aligned.
+ */
+int64_t tf_attn_rows_workspace_bytes(int32_t has_blocks, int32_t n_items, int32_t row_groups,
+                                     int32_t num_q_heads, int32_t num_kv_heads,
+                                     int32_t head_dim, int32_t kv_dtype,
+                                     int32_t num_workgroups);
+
+int32_t tf_attn_rows(
+    const void* q, int64_t q_row_stride, const void* k_pool, const void* v_pool,
+    int64_t pool_slots, int32_t kv_dtype, const float* k_scale, const float* v_scale,
+    const int64_t* req_to_token, int64_t rtt_rows, int64_t rtt_row_stride, int64_t rtt_cols,
+    const int64_t* req_pool_indices, const int64_t* seq_lens, int32_t seq_len_override,
+    const int32_t* blocks, int32_t n_items, int32_t row_groups, int32_t num_q_heads,
+    int32_t num_kv_heads, int32_t head_dim, float scale, void* out, int64_t out_row_stride,
+    void* workspace, int64_t workspace_bytes, int32_t num_workgroups, const void* gate,
+    int64_t gate_row_stride, int64_t gate_head_stride, uint32_t* out_amax, tf_stream_t stream);
+
+/* tf_attn_plan_blocks: the row blocks of a step, built on the device from its
+ * work list and decode items (of either planner, padding included): the decode
+ * items, and the requests of at most max_rows rows (ext * G), become blocks of 16
+ * row_groups rows for tf_attn_rows, padded with b = -1 up to
+ * n_blocks; the other work entries go to pieces [n_pieces][8] in their order,
+ * padded with zeros, for tf_attn_extend (n_pieces = n_work suffices).
+ */
+int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* dec_items,
+                            const int32_t* dec_rows, int32_t n_dec, int32_t num_q_heads,
+                            int32_t num_kv_heads, int32_t row_groups, int64_t max_rows,
+                            int32_t* blocks, int32_t n_blocks, int32_t* pieces,
+                            int32_t n_pieces, tf_stream_t stream);
+
 /* ------------------------------------------------------------------ req_to_token sync
  * Brings the resident device req_to_token table up to date for one batch: the
  * per-step incremental sync of engine/model_runner.py:147-167, which copies

@@ -80,6 +80,24 @@ SIGNATURES = {
         _p, _p, _i32,                  # dec_items, dec_rows, dec_capacity
         _p, _p,                        # status, stream
     ]),
+    "tf_attn_rows": (_i32, [
+        _p, _i64,
+        _p, _p, _i64, _i32, _p, _p,
+        _p, _i64, _i64, _i64,
+        _p, _p, _i32,
+        _p, _i32, _i32,                # blocks, n_items, row_groups
+        _i32, _i32, _i32, _f32,
+        _p, _i64,
+        _p, _i64, _i32,                # workspace, workspace_bytes, num_workgroups
+        _p, _i64, _i64,
+        _p, _p,
+    ]),
+    "tf_attn_rows_workspace_bytes": (_i64, [_i32] * 8),
+    "tf_attn_plan_blocks": (_i32, [
+        _p, _i32, _p, _p, _i32,        # work, n_work, dec_items, dec_rows, n_dec
+        _i32, _i32, _i32, _i64,        # heads, row_groups, max_rows
+        _p, _i32, _p, _i32, _p,        # blocks, n_blocks, pieces, n_pieces, stream
+    ]),
     "tf_attn_plan_decode_items": (_i32, [_p, _i32, _p, _p, _i32]),
     "tf_req_to_token_sync": (_i32, [
         _p, _i64, _i64, _i64,          # req_to_token, rtt_rows, rtt_row_stride, rtt_cols
@@ -248,6 +266,19 @@ def decode_workspace_bytes(n_items, num_q_heads, num_kv_heads, head_dim, max_seq
     lib = load()
     n = lib.tf_attn_decode_workspace_bytes(n_items, num_q_heads, num_kv_heads, head_dim,
                                            max_seq_len, num_workgroups)
+    if n < 0:
+        msg = lib.tf_attn_last_error().decode(errors="replace")
+        if n == TF_ERR_UNSUPPORTED:
+            raise NotImplementedError(msg)
+        raise ValueError(msg)
+    return int(n)
+
+
+def rows_workspace_bytes(has_blocks, n_items, row_groups, num_q_heads, num_kv_heads, head_dim,
+                         kv_dtype, num_workgroups=0) -> int:
+    lib = load()
+    n = lib.tf_attn_rows_workspace_bytes(int(has_blocks), n_items, row_groups, num_q_heads,
+                                         num_kv_heads, head_dim, kv_dtype, num_workgroups)
     if n < 0:
         msg = lib.tf_attn_last_error().decode(errors="replace")
         if n == TF_ERR_UNSUPPORTED:

@@ -159,20 +159,95 @@ def _plan_event(device: torch.device, stream: torch.cuda.Stream) -> torch.cuda.E
     return ev
 
 
+SHORT_ROWS = 64      # query rows per kv head up to which an extend takes the streaming kernel
+MAX_ROW_ITEMS = 2048
+
+
+class Route:
+    """Which kernels a step's rows take, from what the host knows of it.
+
+    At head_dim 256 decode rows run the streaming kernel and extends the extend
+    kernel, except that requests with few new tokens (2 <= ext, ext * G <=
+    ``SHORT_ROWS`` query rows per kv head, e.g. up to 10 tokens at G = 6) are row
+    blocks of the streaming kernel too: its work is spread evenly over the CUs,
+    where the extend kernel gives a request one workgroup per kv head with 256
+    rows to fill (20 requests of 2 to 4 tokens on 1k to 8k keys: 347 us there,
+    84 us here).  At other head dims every row runs the streaming kernel (2
+    prompts of 100 to 400 tokens beside 12 decodes, 32 / 8 heads of 128: 1660 us
+    on the one-wave-per-row kernel, 88 us here); fp8 pools need a head dim that
+    is a multiple of 16, whose rows keep the 16-byte alignment of its loads, and
+    stay on the one-wave-per-row kernel otherwise.
+
+    ``row_groups``: groups of 16 rows per unit, 0 = the streaming kernel takes no
+    blocks.  ``n_blocks`` / ``n_pieces``: capacities of the device lists
+    (``tf_attn_plan_blocks``).  ``exact``: the lengths are this step's own (not a
+    captured or reused call's), so launches without work can be left out."""
+
+    __slots__ = ("row_groups", "max_rows", "n_blocks", "n_pieces", "run_extend", "run_rows")
+
+    def __init__(self, ext_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, n_work, exact):
+        group, bsz = n_q // n_kv, len(ext_lens)
+        self.row_groups = self.n_blocks = self.n_pieces = 0
+        self.max_rows = SHORT_ROWS
+        self.run_extend = self.run_rows = True
+        fp8 = kv_dtype == _native.TF_DTYPE_FP8_E4M3
+        if head_dim != 256:
+            if fp8 and head_dim % 16:
+                return
+            self.max_rows = 1 << 62
+            self.row_groups = 2 if n_work else 1   # blocks whenever the step is planned
+            unit = 16 * self.row_groups
+            self.n_blocks = n_tok * group // unit + (n_work // n_kv if n_work else 0) + bsz
+            self.run_extend = False
+            return
+        short = [e for e in ext_lens if e > 1 and e * group <= SHORT_ROWS]
+        if short:
+            self.row_groups = 1 if max(short) * group <= 16 else 2
+            unit = 16 * self.row_groups
+            self.n_blocks = bsz * max(-(-SHORT_ROWS // unit), -(-group // unit))
+            self.n_pieces = n_work
+        if exact:
+            n_short, n_dec = len(short), sum(1 for e in ext_lens if e == 1)
+            self.run_extend = n_short + n_dec < bsz
+            self.run_rows = n_short + n_dec > 0
+            if not self.run_extend:
+                self.n_pieces = 0
+
+    @property
+    def planned(self) -> bool:
+        """Whether the step needs ``tf_attn_plan_blocks``."""
+        return self.row_groups > 0
+
+    def alloc(self, device) -> torch.Tensor:
+        """The device lists: blocks, then pieces."""
+        return torch.empty(4 * self.n_blocks + 8 * self.n_pieces, dtype=torch.int32,
+                           device=device)
+
+    def plan(self, lists: torch.Tensor, work: int, n_work: int, items, rows, n_dec: int,
+             n_q: int, n_kv: int, stream: torch.cuda.Stream) -> None:
+        base = lists.data_ptr()
+        _native.call("tf_attn_plan_blocks", work if n_work else None, n_work, _ptr(items),
+                     _ptr(rows), n_dec, n_q, n_kv, self.row_groups, self.max_rows, base,
+                     self.n_blocks, base + 16 * self.n_blocks if self.n_pieces else None,
+                     self.n_pieces, stream.cuda_stream)
+
+
 class StepPlan:
     """The work lists of one model step for one head layout: the extend work
     entries and the decode items / rows of a ``ForwardBatch``, planned on the
-    device (``tf_attn_plan_device``, from ``extend_lens_tensor``) by the first
+    device (``tf_attn_plan_device``, from ``extend_lens_tensor``, and
+    ``tf_attn_plan_blocks`` where the step's ``Route`` needs it) by the first
     attention call of the step and read by every later one.
 
     A model step runs every full-attention layer over the same batch
     (``decoder_layer.py:68-69`` calls the attention once per layer), so the
     lists do not change between layers; ``slot_based_attention`` keeps one
-    ``StepPlan`` per (device, T, q heads, kv heads) on the batch object itself.
-    Calls on another stream than the planning one wait for the plan (an event
-    recorded on the planning stream)."""
+    ``StepPlan`` per (device, T, q heads, kv heads, head dim, pool dtype) on the
+    batch object itself.  Calls on another stream than the planning one wait for
+    the plan (an event recorded on the planning stream)."""
 
-    def __init__(self, batch, n_tok: int, n_q: int, n_kv: int, device: torch.device):
+    def __init__(self, batch, n_tok: int, n_q: int, n_kv: int, head_dim: int, kv_dtype: int,
+                 device: torch.device):
         bsz = batch.batch_size
         ext_t = batch.extend_lens_tensor
         if ext_t is None or ext_t.device != device or ext_t.dtype != torch.long \
@@ -180,10 +255,14 @@ class StepPlan:
             raise ValueError("a device plan needs batch.extend_lens_tensor: contiguous int64 "
                              "[batch_size] on q's device")
         self.batch_size, self.n_q, self.n_kv = bsz, n_q, n_kv
+        self.head_dim, self.kv_dtype = head_dim, kv_dtype
         self.ext_t = ext_t
         self.n_work = _native.plan_device_capacity(n_tok, bsz, n_q, n_kv)
         self.n_dec = bsz
+        self.route = Route(batch.extend_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, self.n_work,
+                           exact=True)
         self.meta = torch.empty(self.n_work * 8 + 2 * bsz + 4, dtype=torch.int32, device=device)
+        self.lists = self.route.alloc(device) if self.route.planned else None
         base = self.meta.data_ptr() + 4 * self.n_work * 8
         self.items = _DevPtr(base)
         self.rows = _DevPtr(base + 4 * bsz)
@@ -202,6 +281,9 @@ class StepPlan:
                              self.n_q, self.n_kv, 1, self.meta.data_ptr(), self.n_work,
                              self.items.data_ptr(), self.rows.data_ptr(), self.n_dec,
                              self.status.data_ptr(), stream.cuda_stream)
+                if self.lists is not None:
+                    self.route.plan(self.lists, self.meta.data_ptr(), self.n_work, self.items,
+                                    self.rows, self.n_dec, self.n_q, self.n_kv, stream)
                 with _ws_lock:
                     self._event = _plan_event(self.device, stream)
                     self._event.record(stream)
@@ -215,9 +297,10 @@ class StepPlan:
 _STEP_PLANS = "_tf_attn_step_plans"
 
 
-def step_plan(batch, n_tok: int, n_q: int, n_kv: int, device: torch.device) -> StepPlan:
+def step_plan(batch, n_tok: int, n_q: int, n_kv: int, head_dim: int, kv_dtype: int,
+              device: torch.device) -> StepPlan:
     """The ``StepPlan`` of ``batch`` for this head layout (made on first use)."""
-    key = (device.index, n_tok, n_q, n_kv)
+    key = (device.index, n_tok, n_q, n_kv, head_dim, kv_dtype)
     with _ws_lock:
         plans = getattr(batch, _STEP_PLANS, None)
         if plans is None:
@@ -225,7 +308,7 @@ def step_plan(batch, n_tok: int, n_q: int, n_kv: int, device: torch.device) -> S
             setattr(batch, _STEP_PLANS, plans)
         plan = plans.get(key)
         if plan is None:
-            plan = StepPlan(batch, n_tok, n_q, n_kv, device)
+            plan = StepPlan(batch, n_tok, n_q, n_kv, head_dim, kv_dtype, device)
             plans[key] = plan
         return plan
 
@@ -386,14 +469,21 @@ class SlotAttentionCall:
         self._meta = None
         self._items = self._rows = None
         self._status = None
+        self.route = None
+        self._lists = None
+        self._lists_planned = False   # of a host-planned call (its lengths are fixed)
+        self.ws = None
+        self._n_rows_items = 0   # items of the tf_attn_rows launch (0: tf_attn_decode)
         if n_tok == 0:
             return
         if step_plan is not None:
-            if (step_plan.batch_size, step_plan.n_q, step_plan.n_kv) != (bsz, n_q, n_kv) \
+            if (step_plan.batch_size, step_plan.n_q, step_plan.n_kv, step_plan.head_dim,
+                    step_plan.kv_dtype) != (bsz, n_q, n_kv, head_dim, kv_dtype) \
                     or step_plan.device != q.device:
                 raise ValueError("step_plan was made for another batch layout or device")
             self.n_work, self.n_dec = step_plan.n_work, step_plan.n_dec
             self._ext_t = step_plan.ext_t
+            self.route, self._lists = step_plan.route, step_plan.lists
             self._meta = step_plan.meta
             self._items, self._rows, self._status = (step_plan.items, step_plan.rows,
                                                      step_plan.status)
@@ -435,7 +525,12 @@ class SlotAttentionCall:
             if self.n_dec:
                 self._items = _DevPtr(base)
                 self._rows = _DevPtr(base + 4 * self.n_dec)
-        if (self.decode_workgroups == 0 and self.n_work and self.n_dec
+        if self.route is None:
+            self.route = Route(ext_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, self.n_work,
+                               exact=not self.device_plan)
+            if self.route.planned and self.n_work:
+                self._lists = self.route.alloc(q.device)
+        if (self.decode_workgroups == 0 and self.n_work and self.n_dec and self.route.run_extend
                 and max(ext_lens) > 1 and min(ext_lens) == 1):
             # A mixed step's decode kernel runs beside the extend kernel, whose
             # workgroups hold whole CUs: three times as many, shorter decode
@@ -443,12 +538,21 @@ class SlotAttentionCall:
             # (mixed step 1350 -> 1310 us per layer).  The rule depends on the
             # batch alone, so a serial call gives the same bits.
             self.decode_workgroups = 3 * _cu_count(q.device)
-        self.ws = None
-        if self.n_dec:
+        nbytes = 0
+        if self.route.planned:
+            has_blocks = self._lists is not None
+            if not has_blocks and bsz > MAX_ROW_ITEMS:
+                raise NotImplementedError(f"decode: {bsz} requests in one call (at most "
+                                          f"{MAX_ROW_ITEMS})")
+            self._n_rows_items = self.route.n_blocks if has_blocks else bsz
+            nbytes = _native.rows_workspace_bytes(has_blocks, self._n_rows_items,
+                                                  self.route.row_groups, n_q, n_kv, head_dim,
+                                                  kv_dtype, self.decode_workgroups)
+        elif self.n_dec and self.route.run_rows:
             nbytes = _native.decode_workspace_bytes(self.n_dec, n_q, n_kv, head_dim,
                                                     self.max_len, self.decode_workgroups)
-            if nbytes:
-                self.ws = _workspace(q.device, self.stream, nbytes)
+        if nbytes:
+            self.ws = _workspace(q.device, self.stream, nbytes)
 
     @property
     def stream(self) -> torch.cuda.Stream:
@@ -466,12 +570,26 @@ class SlotAttentionCall:
             if self.n_work:
                 self._shared_plan.ensure(self.stream)
             return
-        if self.device_plan and self.n_work:
+        if not self.n_work:
+            return
+        if self.device_plan:
             base = self._meta.data_ptr()
             _native.call("tf_attn_plan_device", self._ext_t.data_ptr(), self.batch.batch_size,
                          self.n_q, self.n_kv, 1, base, self.n_work, self._items.data_ptr(),
                          self._rows.data_ptr(), self.n_dec, self._status.data_ptr(),
                          self.stream.cuda_stream)
+        self._plan_lists()
+
+    def _plan_lists(self) -> None:
+        if self._lists is not None:
+            self.route.plan(self._lists, self._meta.data_ptr(), self.n_work, self._items,
+                            self._rows, self.n_dec, self.n_q, self.n_kv, self.stream)
+            self._lists_planned = not self.device_plan
+
+    def _host_lists(self) -> None:
+        """The lists of a host-planned call whose phases are run one by one."""
+        if self._lists is not None and not self.device_plan and not self._lists_planned:
+            self._plan_lists()
 
     def plan_status(self):
         """(real work entries, real decode items, flags) of the last device plan:
@@ -482,10 +600,21 @@ class SlotAttentionCall:
         return tuple(int(x) for x in self._meta[n:n + 3].cpu())
 
     def _decode(self, entry: str, stream: Optional[torch.cuda.Stream] = None) -> None:
-        if not self.n_dec:
-            return
         ws = self.ws
         stream = stream if stream is not None else self.stream
+        if self._n_rows_items:
+            if entry == "tf_attn_decode_merge":
+                return   # part of the rows launch
+            self._host_lists()
+            _native.call("tf_attn_rows", self.q.data_ptr(), self.q.stride(0), *self._pool_args,
+                         _ptr(self._lists), self._n_rows_items, self.route.row_groups,
+                         self.n_q, self.n_kv, self.head_dim, self.scaling,
+                         self.out.data_ptr(), self.out.stride(0),
+                         _ptr(ws), 0 if ws is None else ws.numel(), self.decode_workgroups,
+                         *self._epilogue_args, stream.cuda_stream)
+            return
+        if not self.n_dec or not self.route.run_rows:
+            return
         _native.call(entry, self.q.data_ptr(), self.q.stride(0), *self._pool_args,
                      _ptr(self._items), _ptr(self._rows), self.n_dec,
                      self.n_q, self.n_kv, self.head_dim, self.scaling,
@@ -494,9 +623,14 @@ class SlotAttentionCall:
                      self.decode_workgroups, *self._epilogue_args, stream.cuda_stream)
 
     def run_extend(self) -> None:
-        if self.n_work:
+        if self.n_work and self.route.run_extend:
+            work, n_work = self._meta.data_ptr(), self.n_work
+            if self._lists is not None:
+                self._host_lists()
+                work = self._lists.data_ptr() + 16 * self.route.n_blocks
+                n_work = self.route.n_pieces
             _native.call("tf_attn_extend", self.q.data_ptr(), self.q.stride(0),
-                         *self._pool_args, self._meta.data_ptr(), self.n_work,
+                         *self._pool_args, work, n_work,
                          self.n_q, self.n_kv, self.head_dim, self.scaling,
                          self.out.data_ptr(), self.out.stride(0), *self._epilogue_args,
                          self.stream.cuda_stream)
@@ -509,7 +643,8 @@ class SlotAttentionCall:
 
     def run(self) -> torch.Tensor:
         self.run_plan()
-        if self.n_work and self.n_dec and self.overlap_decode:
+        if self.n_work and self.n_dec and self.overlap_decode and self.route.run_extend \
+                and self.route.run_rows:
             # Mixed step: the HBM-bound decode launches go to a second stream and
             # run beside the MFMA-bound extend kernel (they write disjoint rows
             # of out); the caller's stream waits for both.
@@ -518,6 +653,7 @@ class SlotAttentionCall:
             # the other's on a CU, so the decode workgroups take the CUs the
             # extend kernel's last round leaves idle, rather than the extend
             # kernel waiting for the decode kernel's persistent grid.
+            # (the lists of both launches are planned on the caller's stream)
             main, side = self.stream, _side_stream(self.q.device)
             fork, join = _fork_join_events(self.q.device, main)
             fork.record(main)
@@ -573,7 +709,10 @@ def slot_based_attention(
             # replay) and shares nothing with eager calls of the batch.
             device_plan = True
         else:
-            plan = step_plan(batch, q.shape[0], q.shape[1], layer_k_buffer.shape[1], q.device)
+            if sum(int(e) for e in batch.extend_lens) == q.shape[0] \
+                    and layer_k_buffer.dtype in _KV_DTYPES and q.shape[1] % layer_k_buffer.shape[1] == 0:
+                plan = step_plan(batch, q.shape[0], q.shape[1], layer_k_buffer.shape[1],
+                                 q.shape[2], _KV_DTYPES[layer_k_buffer.dtype], q.device)
     call = SlotAttentionCall(q, layer_k_buffer, layer_v_buffer, batch, scaling=scaling,
                              k_scale=k_scale, v_scale=v_scale,
                              decode_workgroups=decode_workgroups, out=out, gate=gate,

@@ -1,8 +1,8 @@
-// Slot attention for head dims other than 256: decode and extend rows of any
-// head_dim that is a multiple of 8, up to 256 (the reference's own test
-// configurations use head_dim 32).  tf_attn_decode / tf_attn_extend route
-// here when head_dim != 256; the 256-dim kernels (decode.hip, extend.hip) are
-// the tuned paths of the 27B model.
+// Slot attention for head dims other than 256, one wave per query row: decode and
+// extend rows of any head_dim that is a multiple of 8, up to 256.
+// tf_attn_decode / tf_attn_extend, which take no workspace at these head dims,
+// route here; so do fp8 pools whose head dim is not a multiple of 16.
+// tf_attn_rows (decode.hip) runs everything else on MFMAs.
 //
 // Same semantics as those kernels (qwen3_8/full_attention.py:163-283): row
 // (token t, q head h) of request b attends to context positions 0 .. P + t,

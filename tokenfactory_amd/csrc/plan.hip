@@ -195,6 +195,80 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(PlanArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Which kernel a request's rows take: the row blocks of the streaming kernel
+// (tf_attn_rows) and the work entries left to the extend kernel, from the work
+// list and the decode items of a step (host- or device-planned, padding
+// included).  Requests of at most max_rows rows (ext * G) go to the streaming
+// kernel, in blocks of a unit's rows.
+struct BlockArgs {
+  const int32_t* work;
+  int32_t n_work;
+  const int32_t* dec_items;
+  const int32_t* dec_rows;
+  int32_t n_dec;
+  int32_t group, unit_rows;
+  int64_t max_rows;       // entries of requests with at most this many rows go to blocks
+  RowItem* blocks;
+  int32_t n_blocks;
+  int32_t* pieces;
+  int32_t n_pieces;
+};
+
+__global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
+  __shared__ int64_t wsum[kPlanThreads / kWave];
+  const int tid = threadIdx.x;
+  const int R = a.unit_rows, G = a.group;
+  int64_t at = 0;   // blocks so far
+  auto emit = [&](int n, int64_t i0, const RowItem& first) {
+    for (int k = 0; k < n; ++k)
+      if (i0 + k < a.n_blocks)
+        a.blocks[i0 + k] = RowItem{first.b, first.qrow, first.ext, first.row0 + k * R};
+  };
+  for (int base = 0; base < a.n_dec; base += kPlanThreads) {
+    const int i = base + tid;
+    RowItem it{-1, 0, 1, 0};
+    if (i < a.n_dec) {
+      it.b = a.dec_items[i];
+      it.qrow = a.dec_rows[i];
+    }
+    const int n = it.b < 0 ? 0 : (G + R - 1) / R;
+    int64_t total;
+    const int64_t before = block_scan(n, wsum, total);
+    emit(n, at + before, it);
+    at += total;
+  }
+  int64_t kept = 0;   // pieces so far
+  for (int base = 0; base < a.n_work; base += kPlanThreads) {
+    const int i = base + tid;
+    int32_t wk[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (i < a.n_work) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) wk[q] = a.work[8 * (int64_t)i + q];
+    }
+    const int64_t rows = (int64_t)wk[4] * G;
+    const bool to_blocks = rows > 0 && (rows <= a.max_rows);
+    const RowItem it{wk[0], wk[3], wk[4], wk[2]};
+    const int n = to_blocks && wk[1] == 0
+                      ? (int)((min<int64_t>(kExtendItemRows, rows - wk[2]) + R - 1) / R) : 0;
+    int64_t total;
+    const int64_t before = block_scan(n, wsum, total);
+    emit(n, at + before, it);
+    at += total;
+    const bool keep = rows > 0 && !to_blocks;
+    int64_t n_keep;
+    const int64_t k0 = kept + block_scan(keep ? 1 : 0, wsum, n_keep);
+    if (keep && k0 < a.n_pieces) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) a.pieces[8 * k0 + q] = wk[q];
+    }
+    kept += n_keep;
+  }
+  for (int64_t i = at + tid; i < a.n_blocks; i += kPlanThreads)
+    a.blocks[i] = RowItem{-1, 0, 1, 0};
+  for (int64_t i = 8 * kept + tid; i < 8LL * a.n_pieces; i += kPlanThreads) a.pieces[i] = 0;
+}
+
+// ---------------------------------------------------------------------------
 // req_to_token sync: the per-step incremental update of the resident device
 // req_to_token table (engine/model_runner.py:147-167) as one kernel.  Request
 // b of the batch owns two runs of flat elements, its rewritten prefix positions
@@ -351,6 +425,39 @@ int32_t tf_attn_plan_device(const int64_t* extend_lens, int32_t batch_size,
   hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0,
                      reinterpret_cast<hipStream_t>(stream), a);
   return launch_status("tf_attn_plan_device launch");
+}
+
+int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* dec_items,
+                            const int32_t* dec_rows, int32_t n_dec, int32_t num_q_heads,
+                            int32_t num_kv_heads, int32_t row_groups, int64_t max_rows,
+                            int32_t* blocks, int32_t n_blocks, int32_t* pieces,
+                            int32_t n_pieces, tf_stream_t stream) {
+  using namespace tfa;
+  clear_error();
+  if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads)
+    return fail(TF_ERR_INVALID, "plan_blocks: heads %d/%d", num_q_heads, num_kv_heads);
+  if (row_groups != 1 && row_groups != 2)
+    return fail(TF_ERR_INVALID, "plan_blocks: row_groups=%d (1 or 2)", row_groups);
+  if (n_work < 0 || n_dec < 0 || n_blocks < 0 || n_pieces < 0 || (n_work > 0 && !work) ||
+      (n_dec > 0 && (!dec_items || !dec_rows)) || (n_blocks > 0 && !blocks) ||
+      (n_pieces > 0 && !pieces) || !aligned16(blocks) || !aligned16(pieces))
+    return fail(TF_ERR_INVALID, "plan_blocks: null or misaligned pointer or negative count");
+  BlockArgs a;
+  a.work = work;
+  a.n_work = n_work;
+  a.dec_items = dec_items;
+  a.dec_rows = dec_rows;
+  a.n_dec = n_dec;
+  a.group = num_q_heads / num_kv_heads;
+  a.unit_rows = 16 * row_groups;
+  a.max_rows = max_rows;
+  a.blocks = reinterpret_cast<RowItem*>(blocks);
+  a.n_blocks = n_blocks;
+  a.pieces = pieces;
+  a.n_pieces = n_pieces;
+  hipLaunchKernelGGL(blocks_kernel, dim3(1), dim3(kPlanThreads), 0,
+                     reinterpret_cast<hipStream_t>(stream), a);
+  return launch_status("tf_attn_plan_blocks launch");
 }
 
 int32_t tf_req_to_token_sync(int64_t* req_to_token, int64_t rtt_rows, int64_t rtt_row_stride,

@@ -20,11 +20,18 @@ int device_cu_count();
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 
+// A block of query rows of one request for the streaming kernel (decode.hip):
+// rows row0 .. of the request's ext * G rows (row = t * G + h), q row of its
+// first token.  b < 0: padding.
+struct RowItem {
+  int32_t b, qrow, ext, row0;
+};
+
 // Decode plan shared by the launcher and the workspace-size query.
 struct DecodePlan {
   int32_t n_blocks;     // workgroups of the streaming kernel (1 per CU by default)
-  int32_t n_hgroups;    // ceil(group / 16)
-  int32_t gmax;         // min(group, 16)
+  int32_t n_hgroups;    // units per kv head of an item
+  int32_t rows_used;    // query rows of a unit that can be real
   int64_t n_units;      // items * kv_heads * n_hgroups
   int64_t ml_bytes, o_bytes, total_bytes;  // split partials: (max, sum) and O
   bool generic;         // head_dim != 256: the one-wave-per-row kernel, no workspace
@@ -32,6 +39,9 @@ struct DecodePlan {
 int make_decode_plan(int32_t n_items, int32_t num_q_heads, int32_t num_kv_heads,
                      int32_t head_dim, int32_t max_seq_len, int32_t num_workgroups,
                      DecodePlan* plan);
+// Units and split workspace of a plan whose n_blocks is set.
+void plan_units(int32_t n_items, int32_t num_kv_heads, int32_t n_hgroups, int32_t unit_rows,
+                int32_t rows_used, int32_t row_floats, DecodePlan* plan);
 
 // Extend kernel arguments (validated by tf_attn_extend).  Work items cover
 // kExtendItemRows flattened (token, q-head-of-group) rows each.
