@@ -303,12 +303,38 @@ int32_t tf_attn_rows(
  * row_groups rows for tf_attn_rows, padded with b = -1 up to
  * n_blocks; the other work entries go to pieces [n_pieces][8] in their order,
  * padded with zeros, for tf_attn_extend (n_pieces = n_work suffices).
+ * merges not NULL (head_dim 256): where the entries leave compute units idle and
+ * the longest one sets the time, entries are cut into pieces over their keys
+ * ({b, kv head, row0, q_start, ext, first 32-key tile, end tile, 1 + partial slot};
+ * at most one piece per compute unit), for tf_attn_extend_split with the merge
+ * entries [n_merges][8], padded with zeros; n_pieces >= the compute units,
+ * n_merges >= half of them, and seq_lens, seq_len_override and rtt_cols are the
+ * launch's.
  */
 int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* dec_items,
                             const int32_t* dec_rows, int32_t n_dec, int32_t num_q_heads,
                             int32_t num_kv_heads, int32_t row_groups, int64_t max_rows,
                             int32_t* blocks, int32_t n_blocks, int32_t* pieces,
-                            int32_t n_pieces, tf_stream_t stream);
+                            int32_t n_pieces, int32_t* merges, int32_t n_merges,
+                            const int64_t* seq_lens, int32_t seq_len_override,
+                            int64_t rtt_cols, tf_stream_t stream);
+
+/* tf_attn_extend_split: tf_attn_extend (head_dim 256) over the pieces and merge
+ * entries of tf_attn_plan_blocks.  workspace: 16-byte aligned scratch of
+ * tf_attn_extend_split_workspace_bytes() (fp32 partials of a piece per compute
+ * unit of the current device; no initialisation needed).
+ */
+int64_t tf_attn_extend_split_workspace_bytes(void);
+
+int32_t tf_attn_extend_split(
+    const void* q, int64_t q_row_stride, const void* k_pool, const void* v_pool,
+    int64_t pool_slots, int32_t kv_dtype, const float* k_scale, const float* v_scale,
+    const int64_t* req_to_token, int64_t rtt_rows, int64_t rtt_row_stride, int64_t rtt_cols,
+    const int64_t* req_pool_indices, const int64_t* seq_lens, int32_t seq_len_override,
+    const int32_t* pieces, int32_t n_pieces, const int32_t* merges, int32_t n_merges,
+    void* workspace, int64_t workspace_bytes, int32_t num_q_heads, int32_t num_kv_heads,
+    float scale, void* out, int64_t out_row_stride, const void* gate, int64_t gate_row_stride,
+    int64_t gate_head_stride, uint32_t* out_amax, tf_stream_t stream);
 
 /* ------------------------------------------------------------------ req_to_token sync
  * Brings the resident device req_to_token table up to date for one batch: the

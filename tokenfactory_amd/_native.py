@@ -96,8 +96,22 @@ SIGNATURES = {
     "tf_attn_plan_blocks": (_i32, [
         _p, _i32, _p, _p, _i32,        # work, n_work, dec_items, dec_rows, n_dec
         _i32, _i32, _i32, _i64,        # heads, row_groups, max_rows
-        _p, _i32, _p, _i32, _p,        # blocks, n_blocks, pieces, n_pieces, stream
+        _p, _i32, _p, _i32, _p, _i32,  # blocks, n_blocks, pieces, n_pieces, merges, n_merges
+        _p, _i32, _i64, _p,            # seq_lens, seq_len_override, rtt_cols, stream
     ]),
+    "tf_attn_extend_split": (_i32, [
+        _p, _i64,
+        _p, _p, _i64, _i32, _p, _p,
+        _p, _i64, _i64, _i64,
+        _p, _p, _i32,
+        _p, _i32, _p, _i32,            # pieces, n_pieces, merges, n_merges
+        _p, _i64,                      # workspace, workspace_bytes
+        _i32, _i32, _f32,              # num_q_heads, num_kv_heads, scale
+        _p, _i64,
+        _p, _i64, _i64,
+        _p, _p,
+    ]),
+    "tf_attn_extend_split_workspace_bytes": (_i64, []),
     "tf_attn_plan_decode_items": (_i32, [_p, _i32, _p, _p, _i32]),
     "tf_req_to_token_sync": (_i32, [
         _p, _i64, _i64, _i64,          # req_to_token, rtt_rows, rtt_row_stride, rtt_cols

@@ -28,7 +28,7 @@ import numpy as np
 import torch
 
 from . import _native
-from .planning import plan_decode_items, plan_extend
+from .planning import EXTEND_TILE_ROWS, plan_decode_items, plan_extend
 
 _KV_DTYPES = {
     torch.bfloat16: _native.TF_DTYPE_BF16,
@@ -159,6 +159,7 @@ def _plan_event(device: torch.device, stream: torch.cuda.Stream) -> torch.cuda.E
     return ev
 
 
+SPLIT_KEYS = 896     # shortest context whose extend entries may be split over keys
 SHORT_ROWS = 64      # query rows per kv head up to which an extend takes the streaming kernel
 MAX_ROW_ITEMS = 2048
 
@@ -178,16 +179,25 @@ class Route:
     is a multiple of 16, whose rows keep the 16-byte alignment of its loads, and
     stay on the one-wave-per-row kernel otherwise.
 
+    Extend entries that leave CUs idle are cut over their keys
+    (``tf_attn_plan_blocks`` decides from the lengths on the device): ``split``
+    says that it may, i.e. there is at most one entry per CU and a context of at
+    least ``SPLIT_KEYS`` keys (a piece shorter than 12 tiles of 32 keys never
+    pays).
+
     ``row_groups``: groups of 16 rows per unit, 0 = the streaming kernel takes no
-    blocks.  ``n_blocks`` / ``n_pieces``: capacities of the device lists
-    (``tf_attn_plan_blocks``).  ``exact``: the lengths are this step's own (not a
+    blocks.  ``n_blocks`` / ``n_pieces`` / ``n_merges``: capacities of the device
+    lists (``tf_attn_plan_blocks``).  ``exact``: the lengths are this step's own (not a
     captured or reused call's), so launches without work can be left out."""
 
-    __slots__ = ("row_groups", "max_rows", "n_blocks", "n_pieces", "run_extend", "run_rows")
+    __slots__ = ("row_groups", "max_rows", "n_blocks", "n_pieces", "n_merges", "split",
+                 "run_extend", "run_rows")
 
-    def __init__(self, ext_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, n_work, exact):
+    def __init__(self, ext_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, n_work, exact,
+                 max_len=0, cus=0):
         group, bsz = n_q // n_kv, len(ext_lens)
-        self.row_groups = self.n_blocks = self.n_pieces = 0
+        self.row_groups = self.n_blocks = self.n_pieces = self.n_merges = 0
+        self.split = False
         self.max_rows = SHORT_ROWS
         self.run_extend = self.run_rows = True
         fp8 = kv_dtype == _native.TF_DTYPE_FP8_E4M3
@@ -206,6 +216,12 @@ class Route:
             unit = 16 * self.row_groups
             self.n_blocks = bsz * max(-(-SHORT_ROWS // unit), -(-group // unit))
             self.n_pieces = n_work
+        long_entries = sum(n_kv * -(-e * group // EXTEND_TILE_ROWS) for e in ext_lens
+                           if e > 1 and e * group > SHORT_ROWS)
+        if n_work and 0 < long_entries <= cus and max_len >= SPLIT_KEYS:
+            self.split = True
+            self.n_pieces = cus if exact else max(n_work, cus)
+            self.n_merges = cus // 2
         if exact:
             n_short, n_dec = len(short), sum(1 for e in ext_lens if e == 1)
             self.run_extend = n_short + n_dec < bsz
@@ -216,20 +232,27 @@ class Route:
     @property
     def planned(self) -> bool:
         """Whether the step needs ``tf_attn_plan_blocks``."""
-        return self.row_groups > 0
+        return self.row_groups > 0 or self.split
 
     def alloc(self, device) -> torch.Tensor:
-        """The device lists: blocks, then pieces."""
-        return torch.empty(4 * self.n_blocks + 8 * self.n_pieces, dtype=torch.int32,
-                           device=device)
+        """The device lists: blocks, pieces, merges."""
+        return torch.empty(4 * self.n_blocks + 8 * (self.n_pieces + self.n_merges),
+                           dtype=torch.int32, device=device)
 
     def plan(self, lists: torch.Tensor, work: int, n_work: int, items, rows, n_dec: int,
-             n_q: int, n_kv: int, stream: torch.cuda.Stream) -> None:
+             n_q: int, n_kv: int, batch, stream: torch.cuda.Stream) -> None:
         base = lists.data_ptr()
-        _native.call("tf_attn_plan_blocks", work if n_work else None, n_work, _ptr(items),
-                     _ptr(rows), n_dec, n_q, n_kv, self.row_groups, self.max_rows, base,
-                     self.n_blocks, base + 16 * self.n_blocks if self.n_pieces else None,
-                     self.n_pieces, stream.cuda_stream)
+        pieces = base + 16 * self.n_blocks
+        rows_too = self.row_groups > 0
+        _native.call("tf_attn_plan_blocks", work if n_work else None, n_work,
+                     _ptr(items) if rows_too else None, _ptr(rows) if rows_too else None,
+                     n_dec if rows_too else 0, n_q, n_kv, max(self.row_groups, 1),
+                     self.max_rows if rows_too else 0, base if self.n_blocks else None,
+                     self.n_blocks, pieces if self.n_pieces else None, self.n_pieces,
+                     pieces + 32 * self.n_pieces if self.split else None, self.n_merges,
+                     batch.seq_lens.data_ptr(),
+                     int(batch.max_seq_len) if batch.batch_size == 1 else 0,
+                     batch.req_to_token.shape[1], stream.cuda_stream)
 
 
 class StepPlan:
@@ -260,7 +283,7 @@ class StepPlan:
         self.n_work = _native.plan_device_capacity(n_tok, bsz, n_q, n_kv)
         self.n_dec = bsz
         self.route = Route(batch.extend_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, self.n_work,
-                           exact=True)
+                           exact=True, max_len=int(batch.max_seq_len), cus=_cu_count(device))
         self.meta = torch.empty(self.n_work * 8 + 2 * bsz + 4, dtype=torch.int32, device=device)
         self.lists = self.route.alloc(device) if self.route.planned else None
         base = self.meta.data_ptr() + 4 * self.n_work * 8
@@ -272,7 +295,7 @@ class StepPlan:
         self._planned_on: Optional[torch.cuda.Stream] = None
         self._event: Optional[torch.cuda.Event] = None
 
-    def ensure(self, stream: torch.cuda.Stream) -> None:
+    def ensure(self, batch, stream: torch.cuda.Stream) -> None:
         """Plan on ``stream`` if no call has yet; else order ``stream`` after
         the plan."""
         with self._lock:
@@ -283,7 +306,7 @@ class StepPlan:
                              self.status.data_ptr(), stream.cuda_stream)
                 if self.lists is not None:
                     self.route.plan(self.lists, self.meta.data_ptr(), self.n_work, self.items,
-                                    self.rows, self.n_dec, self.n_q, self.n_kv, stream)
+                                    self.rows, self.n_dec, self.n_q, self.n_kv, batch, stream)
                 with _ws_lock:
                     self._event = _plan_event(self.device, stream)
                     self._event.record(stream)
@@ -527,7 +550,8 @@ class SlotAttentionCall:
                 self._rows = _DevPtr(base + 4 * self.n_dec)
         if self.route is None:
             self.route = Route(ext_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, self.n_work,
-                               exact=not self.device_plan)
+                               exact=not self.device_plan, max_len=self.max_len,
+                               cus=_cu_count(q.device))
             if self.route.planned and self.n_work:
                 self._lists = self.route.alloc(q.device)
         if (self.decode_workgroups == 0 and self.n_work and self.n_dec and self.route.run_extend
@@ -539,7 +563,7 @@ class SlotAttentionCall:
             # batch alone, so a serial call gives the same bits.
             self.decode_workgroups = 3 * _cu_count(q.device)
         nbytes = 0
-        if self.route.planned:
+        if self.route.row_groups:
             has_blocks = self._lists is not None
             if not has_blocks and bsz > MAX_ROW_ITEMS:
                 raise NotImplementedError(f"decode: {bsz} requests in one call (at most "
@@ -568,7 +592,7 @@ class SlotAttentionCall:
         (with a shared step plan: only if no earlier call of the step planned)."""
         if self._shared_plan is not None:
             if self.n_work:
-                self._shared_plan.ensure(self.stream)
+                self._shared_plan.ensure(self.batch, self.stream)
             return
         if not self.n_work:
             return
@@ -583,7 +607,8 @@ class SlotAttentionCall:
     def _plan_lists(self) -> None:
         if self._lists is not None:
             self.route.plan(self._lists, self._meta.data_ptr(), self.n_work, self._items,
-                            self._rows, self.n_dec, self.n_q, self.n_kv, self.stream)
+                            self._rows, self.n_dec, self.n_q, self.n_kv, self.batch,
+                            self.stream)
             self._lists_planned = not self.device_plan
 
     def _host_lists(self) -> None:
@@ -629,6 +654,17 @@ class SlotAttentionCall:
                 self._host_lists()
                 work = self._lists.data_ptr() + 16 * self.route.n_blocks
                 n_work = self.route.n_pieces
+            if self.route.split:
+                # (allocated on the launch's stream, which orders its reuse)
+                with torch.cuda.stream(self.stream):
+                    ws = torch.empty(_native.load().tf_attn_extend_split_workspace_bytes(),
+                                     dtype=torch.uint8, device=self.q.device)
+                _native.call("tf_attn_extend_split", self.q.data_ptr(), self.q.stride(0),
+                             *self._pool_args, work, n_work, work + 32 * n_work,
+                             self.route.n_merges, ws.data_ptr(), ws.numel(), self.n_q, self.n_kv,
+                             self.scaling, self.out.data_ptr(), self.out.stride(0),
+                             *self._epilogue_args, self.stream.cuda_stream)
+                return
             _native.call("tf_attn_extend", self.q.data_ptr(), self.q.stride(0),
                          *self._pool_args, work, n_work,
                          self.n_q, self.n_kv, self.head_dim, self.scaling,

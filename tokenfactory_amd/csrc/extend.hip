@@ -396,7 +396,9 @@ __device__ __forceinline__ bool softmax_tile(const f32x16& s, Row& row, float sl
   return __ballot(grow) != 0;
 }
 
-template <bool FP8>
+// kSplit: the work list may hold pieces of entries (an instance of its own: as
+// one kernel, large prefills took 0.4 % and mixed steps 2 % longer).
+template <bool FP8, bool kSplit>
 __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
   __shared__ Smem<FP8> sm;
   constexpr int kKS = kStagesOf<FP8>, kVS = kVStagesOf<FP8>;
@@ -416,15 +418,19 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
   const int G = a.group;
 
   if (ext <= 0) return;   // padding entry of a device-built work list
+  // A piece of a split entry takes key tiles [wk[5], wk[6]) and writes slot
+  // wk[7] - 1 of the partials; positions below are relative to its first key.
+  const int part = kSplit ? wk[7] : 0;
+  const int key0 = part ? kBN * wk[5] : 0;
   int64_t len = a.seq_override > 0 ? (int64_t)a.seq_override : a.seq_lens[b];
   if (len > a.rtt_cols) len = a.rtt_cols;
-  const int L = (int)len;
+  const int L = (int)len - key0;
   const int P = L - ext;
   const int rows_total = ext * G;
   if (L <= 0 || row0 >= rows_total) return;
 
   const int64_t rrow = clamp_i64(a.rpi[b], 0, a.rtt_rows - 1);
-  const int64_t* rtt = a.rtt + rrow * a.rtt_stride;
+  const int64_t* rtt = a.rtt + rrow * a.rtt_stride + key0;
 
   // This lane's row; padding lanes compute a valid duplicate row and never
   // write it.
@@ -436,7 +442,8 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
   // row's limit are masked; key 0 is visible to every row, so each row's max
   // is finite after tile 0).
   const int blk_last_row = min(row0 + kExtendItemRows, rows_total) - 1;
-  const int kend = min(L, P + blk_last_row / G + 1);
+  const int keys = min(L, P + blk_last_row / G + 1);
+  const int kend = part ? min(keys, kBN * (wk[6] - wk[5])) : keys;
   if (kend <= 0) return;
   const int n_tiles = (kend + kBN - 1) / kBN;
   const int last = n_tiles - 1;
@@ -533,7 +540,9 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
 #pragma unroll
   for (int kk = 0; kk < 16; ++kk) asm volatile("" ::"v"(qf[kk]));
 
-  Row row{-INFINITY, 0.f, 0.f};
+  // (a piece's first tiles may hold no key a row sees: its maximum starts at a
+  // finite value that any score raises)
+  Row row{part ? -1e30f : -INFINITY, 0.f, 0.f};
   f32x16 acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = f32x16{};
@@ -657,6 +666,25 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
     rescale();
     pv_phase<false>(sm.v + (last % kVS) * kVStage, vaddr, acc, pt, st);
   }
+  if (kSplit && part) {
+    // fp32 partials in the accumulators' own order (1 KB per store), each
+    // row's reference maximum (log2 units) and sum.
+    const float l = row.l + __shfl_xor(row.l, 32, kWave);
+    if (w_first < rows_total) {
+      f32x4* po = reinterpret_cast<f32x4*>(a.part_o) + ((int64_t)(part - 1) * kWaves + w) * 32 * kWave + lane;
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq)
+          po[(4 * mt + rq) * kWave] = f32x4{acc[mt][4 * rq], acc[mt][4 * rq + 1],
+                                            acc[mt][4 * rq + 2], acc[mt][4 * rq + 3]};
+      if (lane < kRowsPerWave)
+        reinterpret_cast<float2*>(a.part_ml)[(int64_t)(part - 1) * kExtendItemRows +
+                                             kRowsPerWave * w + lane] = float2{row.moff, l};
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no staging load outlives its LDS
+    return;
+  }
   // Every wave must be done with the stages before the stage memory holds
   // the output rows (the prologue's stand-in tile of a one-tile item has
   // landed by the last step's wait).
@@ -701,8 +729,137 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
   amax_commit(a.amax, omax);
 }
 
+// Merges the partials of the split entries: grid (entry, wave block of 32 rows);
+// wave mt of the workgroup combines output dims 32 mt .. + 31 of the 32 rows in
+// the partials' own layout (kMergeAhead pieces in flight), then the rows leave
+// through LDS as in the extend kernel's output.  Bound by reading the partials,
+// 256 KB per piece.
+constexpr int kMergeAhead = 4;
+
+template <bool FP8>
+__global__ void __launch_bounds__(kThreads) extend_merge_kernel(ExtendArgs a, const int32_t* merges) {
+  __shared__ __attribute__((aligned(16))) uint8_t rows[kTileBytes];
+  const int32_t* mg = merges + 8 * (int64_t)blockIdx.x;
+  const int ext = mg[4], G = a.group;
+  const int rows_total = ext * G;
+  const int first = mg[2] + kRowsPerWave * blockIdx.y;
+  if (ext <= 0 || first >= rows_total) return;
+  const int hk = mg[1], q_start = mg[3], slot0 = mg[5], n_pieces = mg[6];
+  const int lane = threadIdx.x & 63, mt = wave_id();
+  const int g = lane >> 5, n = lane & 31;
+
+  float m = -INFINITY, l = 0.f;
+  f32x4 acc[4] = {};
+  for (int p = 0; p < n_pieces; p += kMergeAhead) {
+    f32x4 o[kMergeAhead][4];
+    float2 ml[kMergeAhead];
+#pragma unroll
+    for (int k = 0; k < kMergeAhead; ++k) {
+      const int64_t slot = slot0 + min(p + k, n_pieces - 1);
+      ml[k] = reinterpret_cast<const float2*>(a.part_ml)[slot * kExtendItemRows +
+                                                         kRowsPerWave * blockIdx.y + n];
+      const f32x4* po = reinterpret_cast<const f32x4*>(a.part_o) +
+                        ((slot * kWaves + blockIdx.y) * 32 + 4 * mt) * kWave + lane;
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) o[k][rq] = po[rq * kWave];
+    }
+    float mn = m;
+#pragma unroll
+    for (int k = 0; k < kMergeAhead; ++k)
+      if (p + k < n_pieces) mn = fmaxf(mn, ml[k].x);
+    const float a1 = fast_exp2(m - mn);
+    l *= a1;
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq) acc[rq] *= a1;
+#pragma unroll
+    for (int k = 0; k < kMergeAhead; ++k) {
+      if (p + k >= n_pieces) break;
+      const float a2 = fast_exp2(ml[k].x - mn);
+      l += ml[k].y * a2;
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) acc[rq] += o[k][rq] * a2;
+    }
+    m = mn;
+  }
+  const float inv = (FP8 ? a.v_scale[0] : 1.f) / l;
+#pragma unroll
+  for (int rq = 0; rq < 4; ++rq)
+    st_s8(rows + n * kRowBytes + 16 * swz_chunk(n, 4 * mt + rq) + 8 * g,
+          u32x2{pack_bf16(acc[rq][0] * inv, acc[rq][1] * inv),
+                pack_bf16(acc[rq][2] * inv, acc[rq][3] * inv)});
+  __syncthreads();
+  uint32_t omax = 0;
+#pragma unroll
+  for (int i = 0; i < kRowsPerWave * 32 / kThreads; ++i) {
+    const int r = (i * kThreads + threadIdx.x) >> 5, c = threadIdx.x & 31;
+    const int rho = first + r;
+    if (rho >= rows_total) continue;
+    u32x4 v = ld_s16(rows + r * kRowBytes + 16 * swz_chunk(r, c));
+    const int t = rho / G, h = rho - t * G;
+    if (a.gate) {
+      const u32x4 gv = ld_g16(a.gate + (int64_t)(q_start + t) * a.gate_stride +
+                              (int64_t)(hk * G + h) * a.gate_hstride + 8 * c);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = gate_pair(v[k], gv[k]);
+    }
+    omax = max(omax, abs_max8(v));
+    *reinterpret_cast<u32x4*>(a.out + (int64_t)(q_start + t) * a.out_stride +
+                              (int64_t)(hk * G + h) * kD + 8 * c) = v;
+  }
+  amax_commit(a.amax, omax);
+}
+
+// Bytes of split partials: max and sum, then O, of n pieces.
+int64_t part_ml_bytes(int64_t n) { return n * kExtendItemRows * 2 * 4; }
+int64_t part_bytes(int64_t n) { return part_ml_bytes(n) + n * kExtendItemRows * kD * 4; }
+
 }  // namespace
 }  // namespace tfa
+
+namespace {
+
+int32_t extend_launch(const void* q, int64_t q_row_stride, const void* k_pool,
+                      const void* v_pool, int64_t pool_slots, int32_t kv_dtype,
+                      const float* k_scale, const float* v_scale, const int64_t* req_to_token,
+                      int64_t rtt_rows, int64_t rtt_row_stride, int64_t rtt_cols,
+                      const int64_t* req_pool_indices, const int64_t* seq_lens,
+                      int32_t seq_len_override, const int32_t* work, int32_t n_work,
+                      const int32_t* merges, int32_t n_merges, void* workspace,
+                      int64_t workspace_bytes, int32_t num_q_heads, int32_t num_kv_heads,
+                      int32_t head_dim, float scale, void* out, int64_t out_row_stride,
+                      const void* gate, int64_t gate_row_stride, int64_t gate_head_stride,
+                      uint32_t* out_amax, tf_stream_t stream);
+
+}  // namespace
+
+extern "C" int64_t tf_attn_extend_split_workspace_bytes(void) {
+  tfa::clear_error();
+  return tfa::part_bytes(tfa::device_cu_count());
+}
+
+extern "C" int32_t tf_attn_extend_split(
+    const void* q, int64_t q_row_stride, const void* k_pool, const void* v_pool,
+    int64_t pool_slots, int32_t kv_dtype, const float* k_scale, const float* v_scale,
+    const int64_t* req_to_token, int64_t rtt_rows, int64_t rtt_row_stride, int64_t rtt_cols,
+    const int64_t* req_pool_indices, const int64_t* seq_lens, int32_t seq_len_override,
+    const int32_t* pieces, int32_t n_pieces, const int32_t* merges, int32_t n_merges,
+    void* workspace, int64_t workspace_bytes, int32_t num_q_heads, int32_t num_kv_heads,
+    float scale, void* out, int64_t out_row_stride, const void* gate, int64_t gate_row_stride,
+    int64_t gate_head_stride, uint32_t* out_amax, tf_stream_t stream) {
+  using namespace tfa;
+  clear_error();
+  const int64_t need = part_bytes(device_cu_count());
+  if (n_merges < 0 || !merges || !aligned16(merges))
+    return fail(TF_ERR_INVALID, "extend_split: n_merges=%d or merges null or misaligned", n_merges);
+  if (!workspace || !aligned16(workspace) || workspace_bytes < need)
+    return fail(TF_ERR_INVALID, "extend_split: workspace needs %lld bytes, got %lld",
+                (long long)need, (long long)workspace_bytes);
+  return extend_launch(q, q_row_stride, k_pool, v_pool, pool_slots, kv_dtype, k_scale, v_scale,
+                       req_to_token, rtt_rows, rtt_row_stride, rtt_cols, req_pool_indices,
+                       seq_lens, seq_len_override, pieces, n_pieces, merges, n_merges, workspace,
+                       workspace_bytes, num_q_heads, num_kv_heads, kD, scale, out,
+                       out_row_stride, gate, gate_row_stride, gate_head_stride, out_amax, stream);
+}
 
 extern "C" int32_t tf_attn_extend(const void* q, int64_t q_row_stride, const void* k_pool,
                                   const void* v_pool, int64_t pool_slots, int32_t kv_dtype,
@@ -716,8 +873,28 @@ extern "C" int32_t tf_attn_extend(const void* q, int64_t q_row_stride, const voi
                                   int64_t out_row_stride, const void* gate,
                                   int64_t gate_row_stride, int64_t gate_head_stride,
                                   uint32_t* out_amax, tf_stream_t stream) {
+  tfa::clear_error();
+  return extend_launch(q, q_row_stride, k_pool, v_pool, pool_slots, kv_dtype, k_scale, v_scale,
+                       req_to_token, rtt_rows, rtt_row_stride, rtt_cols, req_pool_indices,
+                       seq_lens, seq_len_override, work, n_work, nullptr, 0, nullptr, 0,
+                       num_q_heads, num_kv_heads, head_dim, scale, out, out_row_stride, gate,
+                       gate_row_stride, gate_head_stride, out_amax, stream);
+}
+
+namespace {
+
+int32_t extend_launch(const void* q, int64_t q_row_stride, const void* k_pool,
+                      const void* v_pool, int64_t pool_slots, int32_t kv_dtype,
+                      const float* k_scale, const float* v_scale, const int64_t* req_to_token,
+                      int64_t rtt_rows, int64_t rtt_row_stride, int64_t rtt_cols,
+                      const int64_t* req_pool_indices, const int64_t* seq_lens,
+                      int32_t seq_len_override, const int32_t* work, int32_t n_work,
+                      const int32_t* merges, int32_t n_merges, void* workspace,
+                      int64_t workspace_bytes, int32_t num_q_heads, int32_t num_kv_heads,
+                      int32_t head_dim, float scale, void* out, int64_t out_row_stride,
+                      const void* gate, int64_t gate_row_stride, int64_t gate_head_stride,
+                      uint32_t* out_amax, tf_stream_t stream) {
   using namespace tfa;
-  clear_error();
   if (n_work < 0) return fail(TF_ERR_INVALID, "extend: n_work=%d", n_work);
   if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads)
     return fail(TF_ERR_INVALID, "extend: num_q_heads=%d not a multiple of num_kv_heads=%d",
@@ -775,6 +952,8 @@ extern "C" int32_t tf_attn_extend(const void* q, int64_t q_row_stride, const voi
   a.gate_stride = gate_row_stride;
   a.gate_hstride = gate_head_stride;
   a.amax = out_amax;
+  a.part_ml = static_cast<float*>(workspace);
+  a.part_o = workspace ? a.part_ml + part_ml_bytes(device_cu_count()) / 4 : nullptr;
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (generic) {   // head_dim != 256: one wave per row of every work entry
@@ -808,10 +987,25 @@ extern "C" int32_t tf_attn_extend(const void* q, int64_t q_row_stride, const voi
     g.amax = out_amax;
     return launch_generic_attn(g, s);
   }
-  if (kv_dtype == TF_DTYPE_FP8_E4M3)
-    hipLaunchKernelGGL(extend_mfma_kernel<true>, dim3((unsigned)n_work), dim3(kThreads), 0, s, a);
+  const bool fp8 = kv_dtype == TF_DTYPE_FP8_E4M3;
+  const dim3 items((unsigned)n_work), block(kThreads);
+  if (merges && fp8)
+    hipLaunchKernelGGL((extend_mfma_kernel<true, true>), items, block, 0, s, a);
+  else if (merges)
+    hipLaunchKernelGGL((extend_mfma_kernel<false, true>), items, block, 0, s, a);
+  else if (fp8)
+    hipLaunchKernelGGL((extend_mfma_kernel<true, false>), items, block, 0, s, a);
   else
-    hipLaunchKernelGGL(extend_mfma_kernel<false>, dim3((unsigned)n_work), dim3(kThreads), 0, s, a);
-  return launch_status("tf_attn_extend launch");
+    hipLaunchKernelGGL((extend_mfma_kernel<false, false>), items, block, 0, s, a);
+  const int rc = launch_status("tf_attn_extend launch");
+  if (rc != TF_OK || n_merges == 0) return rc;
+  const dim3 grid((unsigned)n_merges, kWaves);
+  if (fp8)
+    hipLaunchKernelGGL(extend_merge_kernel<true>, grid, block, 0, s, a, merges);
+  else
+    hipLaunchKernelGGL(extend_merge_kernel<false>, grid, block, 0, s, a, merges);
+  return launch_status("tf_attn_extend merge launch");
 }
+
+}  // namespace
 

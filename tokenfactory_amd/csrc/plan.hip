@@ -212,10 +212,80 @@ struct BlockArgs {
   int32_t n_blocks;
   int32_t* pieces;
   int32_t n_pieces;
+  int32_t* merges;        // NULL: entries are not split
+  int32_t n_merges;
+  const int64_t* seq_lens;
+  int32_t seq_override;
+  int64_t rtt_cols;
+  int32_t cus;
 };
+
+// Key split of the extend kernel's entries.  A workgroup of that kernel fills a
+// CU and walks its entry's keys in order, so with fewer entries than CUs the
+// longest entry's keys set the time.  The entries are then cut into pieces of
+// about equal key counts, at most one per CU, whose fp32 partials a merge
+// launch combines.  In tiles of 32 keys (about 1.5 us each): an entry costs its
+// tiles + 15 (Q, first slots, output), a piece its tiles + 24 (it also writes
+// 256 KB of partials), the merge 3 + 0.047 per piece.  The shortest piece
+// length that gives no more pieces than CUs is taken when it beats the whole
+// entries by 8 %; short contexts (below about 900 keys) never do.  Measured
+// (24 / 4 heads): 3 requests of 37 to 211 new tokens on 1.5k to 6k keys, 36
+// entries of up to 180 tiles: 252 us whole, 48 + 14 (merge) in 252 pieces.  One
+// of 2000 tokens on 3000, 188 entries of 95 to 156 tiles, stays whole (the plan
+// would save a tenth of the kernel and pay it back in the merge).
+constexpr int kSplitMax = 512;      // entries a split is considered for (LDS)
+constexpr int kMinPiece = 12;       // tiles
+constexpr float kEntryCost = 15.f, kPieceCost = 24.f, kMergeCost = 3.f, kMergePiece = 0.047f;
+
+struct SplitSmem {
+  int32_t src[kSplitMax];     // index of the kept entry in the work list
+  int32_t tiles[kSplitMax];
+  int32_t piece;              // tiles per piece (0: no split)
+};
+
+// Tiles of 32 keys that the entry's rows see.
+__device__ __forceinline__ int entry_tiles(const BlockArgs& a, const int32_t* wk) {
+  int64_t len = a.seq_override > 0 ? (int64_t)a.seq_override : a.seq_lens[wk[0]];
+  if (len > a.rtt_cols) len = a.rtt_cols;
+  const int64_t last = min<int64_t>((int64_t)wk[2] + kExtendItemRows, (int64_t)wk[4] * a.group) - 1;
+  const int64_t kend = min(len, len - wk[4] + last / a.group + 1);
+  return kend > 0 ? (int)((kend + 31) / 32) : 0;
+}
+
+// Tiles per piece for n entries, by wave 0 (every lane gets it; 0: no split).
+__device__ int piece_tiles(const SplitSmem& sm, int n, int cus) {
+  const int lane = threadIdx.x & (kWave - 1);
+  auto wave_sum = [&](int v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, kWave);
+    return v;
+  };
+  int sum = 0, mx = 0;
+  for (int i = lane; i < n; i += kWave) {
+    sum += sm.tiles[i];
+    mx = max(mx, sm.tiles[i]);
+  }
+  sum = wave_sum(sum);
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) mx = max(mx, __shfl_xor(mx, d, kWave));
+  if (n > cus || mx < 2 * kMinPiece) return 0;
+  auto pieces = [&](int len) {
+    int k = 0;
+    for (int i = lane; i < n; i += kWave) k += (sm.tiles[i] + len - 1) / len;
+    return wave_sum(k);
+  };
+  int lo = kMinPiece, hi = mx;   // pieces(mx) <= n <= cus
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (pieces(mid) <= cus) hi = mid; else lo = mid + 1;
+  }
+  const float split = (float)hi + kPieceCost + kMergeCost + kMergePiece * (float)pieces(hi);
+  return split < 0.92f * ((float)mx + kEntryCost) ? hi : 0;
+}
 
 __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
   __shared__ int64_t wsum[kPlanThreads / kWave];
+  __shared__ SplitSmem sm;
   const int tid = threadIdx.x;
   const int R = a.unit_rows, G = a.group;
   int64_t at = 0;   // blocks so far
@@ -261,8 +331,54 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) a.pieces[8 * k0 + q] = wk[q];
     }
+    if (keep && a.merges && k0 < kSplitMax) {
+      sm.src[k0] = i;
+      sm.tiles[k0] = entry_tiles(a, wk);
+    }
     kept += n_keep;
   }
+  int64_t n_merge = 0;
+  if (a.merges && kept <= kSplitMax) {
+    __syncthreads();
+    if (tid < kWave) {
+      const int len = piece_tiles(sm, (int)kept, a.cus);
+      if (tid == 0) sm.piece = len;
+    }
+    __syncthreads();
+    const int len = sm.piece;
+    if (len > 0) {   // kSplitMax <= kPlanThreads: one entry per thread
+      const int t = tid < kept ? sm.tiles[tid] : 0;
+      const int n = tid < kept ? max(1, (t + len - 1) / len) : 0;
+      int64_t total, slots;
+      const int64_t p0 = block_scan(n, wsum, total);
+      const int64_t s0 = block_scan(n > 1 ? n : 0, wsum, slots);
+      const int64_t m0 = block_scan(n > 1 ? 1 : 0, wsum, n_merge);
+      if (tid < kept) {
+        int32_t wk[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) wk[q] = a.work[8 * (int64_t)sm.src[tid] + q];
+        for (int k = 0; k < n && p0 + k < a.n_pieces; ++k) {
+          int32_t* pc = a.pieces + 8 * (p0 + k);
+#pragma unroll
+          for (int q = 0; q < 5; ++q) pc[q] = wk[q];
+          pc[5] = n > 1 ? (int)((int64_t)t * k / n) : 0;
+          pc[6] = n > 1 ? (int)((int64_t)t * (k + 1) / n) : 0;
+          pc[7] = n > 1 ? (int32_t)(s0 + k + 1) : 0;
+        }
+        if (n > 1 && m0 < a.n_merges) {
+          int32_t* mg = a.merges + 8 * m0;
+#pragma unroll
+          for (int q = 0; q < 5; ++q) mg[q] = wk[q];
+          mg[5] = (int32_t)s0;
+          mg[6] = n;
+          mg[7] = 0;
+        }
+      }
+      kept = total;
+    }
+  }
+  if (a.merges)
+    for (int64_t i = 8 * n_merge + tid; i < 8LL * a.n_merges; i += kPlanThreads) a.merges[i] = 0;
   for (int64_t i = at + tid; i < a.n_blocks; i += kPlanThreads)
     a.blocks[i] = RowItem{-1, 0, 1, 0};
   for (int64_t i = 8 * kept + tid; i < 8LL * a.n_pieces; i += kPlanThreads) a.pieces[i] = 0;
@@ -431,7 +547,9 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
                             const int32_t* dec_rows, int32_t n_dec, int32_t num_q_heads,
                             int32_t num_kv_heads, int32_t row_groups, int64_t max_rows,
                             int32_t* blocks, int32_t n_blocks, int32_t* pieces,
-                            int32_t n_pieces, tf_stream_t stream) {
+                            int32_t n_pieces, int32_t* merges, int32_t n_merges,
+                            const int64_t* seq_lens, int32_t seq_len_override,
+                            int64_t rtt_cols, tf_stream_t stream) {
   using namespace tfa;
   clear_error();
   if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads)
@@ -440,8 +558,14 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
     return fail(TF_ERR_INVALID, "plan_blocks: row_groups=%d (1 or 2)", row_groups);
   if (n_work < 0 || n_dec < 0 || n_blocks < 0 || n_pieces < 0 || (n_work > 0 && !work) ||
       (n_dec > 0 && (!dec_items || !dec_rows)) || (n_blocks > 0 && !blocks) ||
-      (n_pieces > 0 && !pieces) || !aligned16(blocks) || !aligned16(pieces))
+      (n_pieces > 0 && !pieces) || !aligned16(blocks) || !aligned16(pieces) ||
+      !aligned16(merges) || n_merges < 0)
     return fail(TF_ERR_INVALID, "plan_blocks: null or misaligned pointer or negative count");
+  const int32_t cus = device_cu_count();
+  if (merges && (n_pieces < cus || n_merges < cus / 2 || rtt_cols < 1 ||
+                 (!seq_lens && seq_len_override <= 0)))
+    return fail(TF_ERR_INVALID, "plan_blocks: a split needs the lengths and room for %d pieces "
+                "and %d merges", cus, cus / 2);
   BlockArgs a;
   a.work = work;
   a.n_work = n_work;
@@ -455,6 +579,12 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
   a.n_blocks = n_blocks;
   a.pieces = pieces;
   a.n_pieces = n_pieces;
+  a.merges = merges;
+  a.n_merges = n_merges;
+  a.seq_lens = seq_lens;
+  a.seq_override = seq_len_override;
+  a.rtt_cols = rtt_cols;
+  a.cus = cus;
   hipLaunchKernelGGL(blocks_kernel, dim3(1), dim3(kPlanThreads), 0,
                      reinterpret_cast<hipStream_t>(stream), a);
   return launch_status("tf_attn_plan_blocks launch");

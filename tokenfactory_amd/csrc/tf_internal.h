@@ -67,6 +67,8 @@ struct ExtendArgs {
   const __bf16* gate;             // optional output gate (NULL: none)
   int64_t gate_stride, gate_hstride;
   uint32_t* amax;                 // optional: raised to max |out| (bf16 bits)
+  float* part_o;                  // split entries: fp32 partials (work[7] - 1 = slot)
+  float* part_ml;
 };
 
 // Slot attention for head dims other than 256 (attn_generic.hip): one wave per
