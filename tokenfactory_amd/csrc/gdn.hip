@@ -553,10 +553,15 @@ __device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t
 // 512-thread workgroup per (request, value head) whose state wave w (0-3) owns
 // state columns
 // 32 w .. + 31 as four 32 x 32 MFMA accumulator tiles (lane (g, n) = (lane /
-// 32, lane % 32): rows 32 ti + 8 (r / 4) + 4 g + r % 4 of column 32 w + n), so
+// 32, lane % 32): register r of tile ti is row 32 ti + 16 (r / 8) + 8 g + r % 8 of
+// column 32 w + n; the update's K^T operand puts its rows in that order), so
 // the state update is an MFMA into S and the products with S read it as an
-// MFMA operand in place.  Every product runs on v_mfma_f32_32x32x16_bf16 with
-// both fp32 operands split into bf16 high and low parts (hi*hi + hi*lo +
+// MFMA operand in place, against eight consecutive dims of a k or q row: one
+// 16-byte LDS read.  (In the accumulator's own row order, 8 (r / 4) + 4 g + r % 4,
+// the rows came in 8-byte reads, which take the LDS three times as long per
+// byte: one request of 1900 tokens, 48 workgroups, 197 -> 171 us.)
+// Every product runs on v_mfma_f32_32x32x16_bf16 with both fp32 operands split
+// into bf16 high and low parts (hi*hi + hi*lo +
 // lo*hi, about 2^-17 relative error, fp32 accumulation); q and k arrive
 // already split (gdn_qk_ext_kernel).  Chunk records are numbered
 // floor(t0_b / 32) + b + ci for chunk ci of request b (first token row t0_b),
@@ -713,19 +718,13 @@ struct ChunkIn {
   float rec[kRec];           // 9 KB: the chunk's record
 };
 
-// Dims d0 .. d0 + 3 and d0 + 8 .. d0 + 11 (d0 a multiple of 4, d0 % 8 < 4) of
-// swizzled row t, high and low parts, as two MFMA operands.
-__device__ __forceinline__ void row8(const uint32_t (*rows)[128], int t, int d0, u32x4& hi,
+// Dims 8 c .. 8 c + 7 of swizzled row t, high and low parts, as two MFMA
+// operands.
+__device__ __forceinline__ void row8(const uint32_t (*rows)[128], int t, int c, u32x4& hi,
                                      u32x4& lo) {
-  const uint32_t* row = rows[t];
-  const int c = d0 >> 3, e = (d0 & 7) >> 1;   // 16-B chunk, dword within it
-  const int p0 = 4 * ((c) ^ (t & 15)) + e, p1 = 4 * ((c + 1) ^ (t & 15)) + e;
-  const u32x2 h0 = *reinterpret_cast<const u32x2*>(row + p0);
-  const u32x2 h1 = *reinterpret_cast<const u32x2*>(row + p1);
-  const u32x2 l0 = *reinterpret_cast<const u32x2*>(row + 64 + p0);
-  const u32x2 l1 = *reinterpret_cast<const u32x2*>(row + 64 + p1);
-  hi = u32x4{h0[0], h0[1], h1[0], h1[1]};
-  lo = u32x4{l0[0], l0[1], l1[0], l1[1]};
+  const uint32_t* row = rows[t] + 4 * (c ^ (t & 15));
+  hi = *reinterpret_cast<const u32x4*>(row);
+  lo = *reinterpret_cast<const u32x4*>(row + 64);
 }
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4_t lds_i16x4;
@@ -777,12 +776,12 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_chunk_ext_kernel(GdnArgs a)
     const int j = 32 * w + n;   // this lane's state column
     f32x16 st[4];
     {
-      const float* my = stage + 4 * g * kDv + j;
+      const float* my = stage + 8 * g * kDv + j;
 #pragma unroll
       for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
         for (int rr = 0; rr < 16; ++rr)
-          st[ti][rr] = my[(32 * ti + 8 * (rr >> 2) + (rr & 3)) * kDv];
+          st[ti][rr] = my[(32 * ti + 16 * (rr >> 3) + (rr & 7)) * kDv];
     }
     __syncthreads();   // the staging area is free for chunk 0
 
@@ -791,7 +790,7 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_chunk_ext_kernel(GdnArgs a)
       __syncthreads();   // chunk ci is in; its output tile is free
 
       // P = K S0 and R = Q S0 over the state rows (k index 8 g + jj <-> state
-      // row 32 ti + 16 hh + 8 (jj / 4) + 4 g + jj % 4)
+      // row 32 ti + 16 hh + 8 g + jj)
       // (two accumulators each for P and R, one per half of the state rows:
       // four independent MFMA chains)
       // (step (ti, hh) + 1's operands are read from LDS while step (ti, hh)'s
@@ -799,9 +798,8 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_chunk_ext_kernel(GdnArgs a)
       f32x16 Pp[2] = {{}, {}}, Rp[2] = {{}, {}};
       u32x4 op[2][4];
       auto read_ops = [&](int step, u32x4 (&o)[4]) __attribute__((always_inline)) {
-        const int d0 = 32 * (step >> 1) + 16 * (step & 1) + 4 * g;
-        row8(I.k, n, d0, o[0], o[1]);
-        row8(I.q, n, d0, o[2], o[3]);
+        row8(I.k, n, 2 * step + g, o[0], o[1]);
+        row8(I.q, n, 2 * step + g, o[2], o[3]);
       };
       // (and step + 1's state operand is split while step's MFMAs run)
       u32x4 sh[2], sl[2];
@@ -867,15 +865,17 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_chunk_ext_kernel(GdnArgs a)
       split16(D, 0, dh[0], dl[0]);
       split16(D, 8, dh[1], dl[1]);
       const float cC = I.rec[kRecC + kChunk - 1];
-      // A operand: K^T row i = 32 ti + n at tokens s(jj) as for Delta, read
-      // from the token-major k rows with ds_read_b64_tr_b16, which hands lane
-      // i of each 16-lane group element i % 4 of the 8 bytes addressed by lane
-      // 4 k + (i % 16) / 4 as its element k: lane L addresses token
-      // 16 hh + 4 g + (L % 16) / 4 (+ 8), dims 32 ti + 16 ((L / 16) % 2) +
-      // 4 (L % 4) .. + 3 (step (ti, hh) + 1's read while step (ti, hh)'s
-      // MFMAs run)
+      // A operand: the row of K^T that accumulator row n of tile ti holds (see
+      // above: dim 32 ti + 16 (n / 16) + 8 ((n / 4) % 2) + 4 ((n / 8) % 2) + n % 4)
+      // at tokens s(jj) as for Delta, read from the token-major k rows with
+      // ds_read_b64_tr_b16, which hands lane i of each 16-lane group element
+      // i % 4 of the 8 bytes addressed by lane 4 k + (i % 16) / 4 as its element
+      // k: lane L addresses token 16 hh + 4 g + (L % 16) / 4 (+ 8), dims 32 ti +
+      // 16 ((L / 16) % 2) + 8 (L % 2) + 4 ((L / 2) % 2) .. + 3 (step (ti, hh) + 1's
+      // read while step (ti, hh)'s MFMAs run)
       u32x4 ka[2][2];
-      const int tq = (lane & 15) >> 2, dq = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+      const int tq = (lane & 15) >> 2;
+      const int dq = 16 * ((lane >> 4) & 1) + 8 * (lane & 1) + 4 * ((lane >> 1) & 1);
       auto read_kt = [&](int step, u32x4 (&o)[2]) __attribute__((always_inline)) {
         const int d = 32 * (step >> 1) + dq, c = d >> 3, e = (d & 7) >> 1;
         const int t0 = 16 * (step & 1) + 4 * g + tq, t1 = t0 + 8;
@@ -901,12 +901,12 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_chunk_ext_kernel(GdnArgs a)
       }
     }
     __syncthreads();   // the last chunk's output tile is complete
-    float* mine = stage + 4 * g * kDv + j;   // the chunk buffers are no longer read
+    float* mine = stage + 8 * g * kDv + j;   // the chunk buffers are no longer read
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr)
-        mine[(32 * ti + 8 * (rr >> 2) + (rr & 3)) * kDv] = st[ti][rr];
+        mine[(32 * ti + 16 * (rr >> 3) + (rr & 7)) * kDv] = st[ti][rr];
   } else {
     const int key0 = chunk_key(a, bi);
     // Chunk ci into buffer bf (tokens past the last one re-read the last
