@@ -475,6 +475,30 @@ int32_t tf_fp8_act_quant_amax(const void* x, int32_t x_dtype, int64_t rows, int6
                               int64_t x_row_stride, void* xq, int64_t xq_row_stride,
                               float* x_scale, const uint32_t* amax_bits, tf_stream_t stream);
 
+/* tf_fp8_act_quant_partials: tf_fp8_act_quant with max|x| known as npartial (at
+ * most TF_FP8_QUANT_WORKSPACE_BYTES / 4) maxima over parts of x, as
+ * tf_narrow_linear2 leaves them: the same x_scale and xq bit for bit.
+ */
+int32_t tf_fp8_act_quant_partials(const void* x, int32_t x_dtype, int64_t rows, int64_t cols,
+                                  int64_t x_row_stride, void* xq, int64_t xq_row_stride,
+                                  float* x_scale, const uint32_t* partials, int32_t npartial,
+                                  tf_stream_t stream);
+
+/* tf_narrow_linear2: out_i = bf16(x w_i^T) for two narrow bf16 weights of one
+ * input, fp32 accumulation (the in_proj_b / in_proj_a gate projections,
+ * linear_attention.py:311-314).  x: bf16 [rows, k], k a multiple of 32, 16-byte
+ * aligned with a row stride that is a multiple of 8; w_i: bf16 [n, k]
+ * contiguous, 16-byte aligned, n up to 64; out_i: bf16 [rows, n] with a common
+ * row stride.  amax_partials (NULL allowed): device uint32
+ * [tf_narrow_linear2_blocks(rows)], receives the largest |x| (bf16 bit pattern,
+ * sign cleared) of each workgroup's rows.
+ */
+int32_t tf_narrow_linear2_blocks(int64_t rows);
+
+int32_t tf_narrow_linear2(const void* x, int64_t x_row_stride, int64_t rows, int64_t k,
+                          const void* w0, const void* w1, int32_t n, void* out0, void* out1,
+                          int64_t out_row_stride, uint32_t* amax_partials, tf_stream_t stream);
+
 int32_t tf_fp8_block_gemm(const void* xq, int64_t xq_row_stride, const float* x_scale,
                           const void* w, int64_t w_row_stride, const float* w_scale,
                           int64_t w_scale_row_stride, int64_t w_scale_col_stride,

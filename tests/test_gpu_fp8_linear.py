@@ -318,3 +318,44 @@ def test_projections_of_one_input_in_one_launch(gpu, m, bias):
     assert seen == [(m, ns[1])]
     for out, ref in zip(again, refs):
         assert torch.allclose(out.cpu().float(), ref, atol=1e-3, rtol=2 ** -8)
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 48, 4095, 4113])
+@pytest.mark.parametrize("n,k", [(6, 128), (16, 64), (48, 5120), (33, 96), (64, 1024)])
+def test_narrow_linears(gpu, rows, n, k):
+    """Two narrow bf16 linears in one launch, on a strided input, against fp64,
+    and the quantisation from its maxima against the two-pass one bit for bit."""
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randn((rows, 2 * k), generator=g).to(torch.bfloat16).to(gpu)[:, :k]
+    lins = [torch.nn.Linear(k, n, bias=False, dtype=torch.bfloat16, device=gpu)
+            .requires_grad_(False) for _ in range(2)]
+    print(f"[narrow] rows={rows} n={n} k={k}", flush=True)
+    first, second, amax = fl.narrow_linears(x, *lins)
+    xq, scale = fl.quantize_activations(x, amax_partials=amax)
+    want_q, want_scale = fl.quantize_activations(x)
+    torch.cuda.synchronize()
+    for got, lin in zip((first, second), lins):
+        ref = x.double().cpu() @ lin.weight.double().cpu().t()
+        # one bf16 rounding (2^-9) and fp32 sums of k terms of about 1/sqrt(k) each
+        assert torch.allclose(got.double().cpu(), ref, rtol=2 ** -8, atol=1e-5)
+    assert torch.equal(scale, want_scale)
+    assert torch.equal(xq.view(torch.uint8), want_q.view(torch.uint8))
+
+
+def test_narrow_linears_call_what_is_not_plain(gpu):
+    """A bias, a hook, a recorded gradient or another dtype goes through the modules."""
+    x = torch.randn((5, 64), device=gpu).to(torch.bfloat16)
+    mk = lambda **kw: torch.nn.Linear(64, 8, dtype=torch.bfloat16, device=gpu, **kw)
+    with torch.no_grad():
+        for lins in ((mk(), mk()), (mk(bias=False), mk())):
+            out = fl.narrow_linears(x, *lins)
+            assert out[2] is None and torch.equal(out[0], lins[0](x))
+    lins = [mk(bias=False).requires_grad_(False) for _ in range(2)]
+    seen = []
+    handle = lins[0].register_forward_hook(lambda m, a, o: seen.append(1))
+    assert fl.narrow_linears(x, *lins)[2] is None and seen == [1]
+    handle.remove()
+    assert fl.narrow_linears(x, *lins)[2] is not None
+    lins[1].requires_grad_(True)
+    out = fl.narrow_linears(x, *lins)
+    assert out[2] is None and out[1].requires_grad

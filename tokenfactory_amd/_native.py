@@ -148,6 +148,17 @@ SIGNATURES = {
         _p, _i64, _p,                  # xq, xq_row_stride, x_scale
         _p, _p,                        # amax_bits, stream
     ]),
+    "tf_fp8_act_quant_partials": (_i32, [
+        _p, _i32, _i64, _i64, _i64,    # x, x_dtype, rows, cols, x_row_stride
+        _p, _i64, _p,                  # xq, xq_row_stride, x_scale
+        _p, _i32, _p,                  # partials, npartial, stream
+    ]),
+    "tf_narrow_linear2_blocks": (_i32, [_i64]),
+    "tf_narrow_linear2": (_i32, [
+        _p, _i64, _i64, _i64,          # x, x_row_stride, rows, k
+        _p, _p, _i32,                  # w0, w1, n
+        _p, _p, _i64, _p, _p,          # out0, out1, out_row_stride, amax_partials, stream
+    ]),
     "tf_fp8_block_gemm": (_i32, [
         _p, _i64, _p,                  # xq, xq_row_stride, x_scale
         _p, _i64,                      # w, w_row_stride

@@ -797,6 +797,27 @@ int32_t tf_fp8_act_quant_amax(const void* x, int32_t x_dtype, int64_t rows, int6
   return launch_status("tf_fp8_act_quant_amax launch");
 }
 
+int32_t tf_fp8_act_quant_partials(const void* x, int32_t x_dtype, int64_t rows, int64_t cols,
+                                  int64_t x_row_stride, void* xq, int64_t xq_row_stride,
+                                  float* x_scale, const uint32_t* partials, int32_t npartial,
+                                  tf_stream_t stream) {
+  using namespace tfa;
+  clear_error();
+  QuantArgs a;
+  const int32_t rc = quant_setup("fp8_act_quant_partials", x, x_dtype, rows, cols, x_row_stride,
+                                 xq, xq_row_stride, x_scale, &a);
+  if (rc != TF_OK) return rc;
+  if (!partials || (reinterpret_cast<uintptr_t>(partials) & 3u) || npartial < 1 ||
+      npartial > kQuantMaxBlocks)
+    return fail(TF_ERR_INVALID, "fp8_act_quant_partials: %d partials (1 to %d, 4-byte aligned)",
+                npartial, kQuantMaxBlocks);
+  a.partial = partials;
+  a.npartial = (uint32_t)npartial;
+  hipLaunchKernelGGL(act_quant_kernel, dim3(a.nblocks), dim3(kThreads), 0,
+                     reinterpret_cast<hipStream_t>(stream), a);
+  return launch_status("tf_fp8_act_quant_partials launch");
+}
+
 int32_t tf_fp8_block_gemm_multi(const void* xq, int64_t xq_row_stride, const float* x_scale,
                                 const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h,
                                 int32_t block_w, int64_t m, int64_t k, void* workspace,

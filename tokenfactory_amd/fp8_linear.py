@@ -63,7 +63,8 @@ def _pad_cols(t: torch.Tensor, cols: int) -> torch.Tensor:
 
 
 def quantize_activations(x2d: torch.Tensor, stream=None, padded_cols: Optional[int] = None,
-                         amax: Optional[torch.Tensor] = None):
+                         amax: Optional[torch.Tensor] = None,
+                         amax_partials: Optional[torch.Tensor] = None):
     """Dynamic per-tensor e4m3 quantisation of a bf16 ``[rows, cols]`` matrix
     (``fp8_triton.py:127-130``). Returns ``(xq, x_scale)``: float8_e4m3fn rows
     and a 1-element fp32 tensor holding ``bf16(max(amax|x|, 1e-12) / 448)``.
@@ -71,7 +72,8 @@ def quantize_activations(x2d: torch.Tensor, stream=None, padded_cols: Optional[i
     ``amax``: the max of ``|x|`` already computed by x's producer (a 1-element
     int32 device tensor holding the bf16 bit pattern, as the attention kernels'
     ``out_amax`` leaves it); the result is the same, with one launch
-    (``tf_fp8_act_quant_amax``) instead of two."""
+    (``tf_fp8_act_quant_amax``) instead of two.  ``amax_partials``: the same as
+    int32 maxima over parts of x (``narrow_linears``)."""
     if x2d.dtype != torch.bfloat16 or x2d.dim() != 2 or not x2d.is_cuda:
         raise ValueError("quantize_activations: x must be a 2-D bf16 CUDA tensor")
     if x2d.stride(1) != 1:
@@ -91,6 +93,16 @@ def quantize_activations(x2d: torch.Tensor, stream=None, padded_cols: Optional[i
                                  "on x's device")
             _native.call("tf_fp8_act_quant_amax", _ptr(x2d), _native.TF_DTYPE_BF16, rows, cols,
                          x2d.stride(0), _ptr(xq), xq.stride(0), _ptr(scale), _ptr(amax),
+                         _stream_ptr(stream, x2d.device))
+            return xq, scale
+        if amax_partials is not None:
+            if amax_partials.dtype != torch.int32 or amax_partials.device != x2d.device \
+                    or not amax_partials.is_contiguous():
+                raise ValueError("quantize_activations: amax_partials must be a contiguous int32 "
+                                 "tensor on x's device")
+            _native.call("tf_fp8_act_quant_partials", _ptr(x2d), _native.TF_DTYPE_BF16, rows,
+                         cols, x2d.stride(0), _ptr(xq), xq.stride(0), _ptr(scale),
+                         _ptr(amax_partials), amax_partials.numel(),
                          _stream_ptr(stream, x2d.device))
             return xq, scale
         ws = torch.empty((_native.TF_FP8_QUANT_WORKSPACE_BYTES,), dtype=torch.uint8,
@@ -179,27 +191,58 @@ def block_fp8_linear(x: torch.Tensor, weight: torch.Tensor,
     return out.reshape(*x.shape[:-1], weight.shape[0])
 
 
-def _plain(linear) -> bool:
-    """Whether calling ``linear`` runs ``Fp8Linear.forward`` and nothing else (no
+def _plain(linear, kind) -> bool:
+    """Whether calling ``linear`` runs ``kind.forward`` and nothing else (no
     subclass, replaced forward or hook)."""
-    return (type(linear) is Fp8Linear and "forward" not in linear.__dict__
+    return (type(linear) is kind and "forward" not in linear.__dict__
             and not (linear._forward_hooks or linear._forward_pre_hooks
                      or linear._backward_hooks or linear._backward_pre_hooks
                      or nn.modules.module._has_any_global_hook()))
 
 
-def fp8_linears(x: torch.Tensor, linears: Sequence["Fp8Linear"]):
+def narrow_linears(x: torch.Tensor, first: nn.Linear, second: nn.Linear):
+    """``(first(x), second(x), amax_partials)`` for two narrow bf16 linears of one
+    input (``linear_attention.py:311-314``) in one ``tf_narrow_linear2`` launch,
+    with max ``|x|`` per row block for ``quantize_activations`` of the same x.
+    Linears that are more than plain bf16 ``nn.Linear`` calls without a bias, that
+    autograd is to record or autocast to cast, or whose sizes the kernel does not
+    take are called one by one (``amax_partials`` is then None)."""
+    n, k = first.weight.shape
+    grad = torch.is_grad_enabled() and (x.requires_grad or first.weight.requires_grad
+                                        or second.weight.requires_grad)
+    if (grad or torch.is_autocast_enabled() or not x.is_cuda or x.dim() != 2
+            or x.dtype != torch.bfloat16 or x.shape[0] == 0 or n > 64 or k % 32
+            or x.shape[1] != k or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16
+            or not all(_plain(m, nn.Linear) and m.bias is None and m.weight.shape == (n, k)
+                       and m.weight.dtype == torch.bfloat16 and m.weight.device == x.device
+                       and m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 0
+                       for m in (first, second))):
+        return first(x), second(x), None
+    rows = x.shape[0]
+    outs = [torch.empty((rows, n), dtype=torch.bfloat16, device=x.device) for _ in range(2)]
+    blocks = _native.load().tf_narrow_linear2_blocks(rows)
+    partials = None
+    if 0 < blocks <= _native.TF_FP8_QUANT_WORKSPACE_BYTES // 4:
+        partials = torch.empty((blocks,), dtype=torch.int32, device=x.device)
+    _native.call("tf_narrow_linear2", _ptr(x), x.stride(0), rows, k, _ptr(first.weight),
+                 _ptr(second.weight), n, _ptr(outs[0]), _ptr(outs[1]), n, _ptr(partials),
+                 _stream_ptr(None, x.device))
+    return outs[0], outs[1], partials
+
+
+def fp8_linears(x: torch.Tensor, linears: Sequence["Fp8Linear"],
+                amax_partials: Optional[torch.Tensor] = None):
     """``[lin(x) for lin in linears]`` for projections of the same input
     (``full_attention.py:122-139``, ``linear_attention.py:309-314``): x is
     quantised once and one ``tf_fp8_block_gemm_multi`` launch multiplies it with
     every weight.  Linears that do not share a block size and a K that is a
     multiple of 128, or that are more than plain ``Fp8Linear`` calls, are called
-    one by one."""
+    one by one.  ``amax_partials``: see ``quantize_activations``."""
     first = linears[0]
     k = first.in_features
     if (len(linears) > _native.TF_FP8_MAX_MATS or k % K_SLICE or x.shape[-1] != k
             or not x.is_cuda or x.dtype != torch.bfloat16
-            or not all(_plain(m) and m.in_features == k and m.block_h == first.block_h
+            or not all(_plain(m, Fp8Linear) and m.in_features == k and m.block_h == first.block_h
                        and m.block_w == first.block_w and m.weight.is_contiguous()
                        and m.weight.dtype == torch.float8_e4m3fn
                        and m.weight.device == x.device
@@ -214,7 +257,7 @@ def fp8_linears(x: torch.Tensor, linears: Sequence["Fp8Linear"]):
     if x2d.stride(1) != 1:
         x2d = x2d.contiguous()
     rows = x2d.shape[0]
-    xq, scale = quantize_activations(x2d)
+    xq, scale = quantize_activations(x2d, amax_partials=amax_partials)
     outs = [torch.empty((rows, m.out_features), dtype=torch.bfloat16, device=x.device)
             for m in linears]
     if rows:

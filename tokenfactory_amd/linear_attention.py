@@ -24,7 +24,7 @@ import torch
 import torch.nn as nn
 
 from . import _native
-from .fp8_linear import Fp8Linear, fp8_linears, on_stream
+from .fp8_linear import Fp8Linear, fp8_linears, narrow_linears, on_stream
 
 HEAD_DIM = 128      # the tuned kernels' head dims (key and value)
 MAX_OTHER_HEAD_DIM = 64   # other head dims: multiples of 4 up to this (one wave per head)
@@ -217,13 +217,12 @@ class LinearAttention(nn.Module):
         return self._packed
 
     def forward(self, hidden_states: torch.Tensor, cache_pool, forward_batch) -> torch.Tensor:
+        b, a, amax = narrow_linears(hidden_states, self.in_proj_b, self.in_proj_a)
         wide = (self.in_proj_qkv, self.in_proj_z)
         if all(isinstance(p, Fp8Linear) for p in wide):
-            qkv, z = fp8_linears(hidden_states, wide)
+            qkv, z = fp8_linears(hidden_states, wide, amax)
         else:
             qkv, z = (p(hidden_states) for p in wide)
-        b = self.in_proj_b(hidden_states)
-        a = self.in_proj_a(hidden_states)
         conv_state, ssm_state = cache_pool.get_linear_states(self.layer_idx)
         conv_w, a_log, dt_bias, norm_w = self._kernel_params()
         if all(e == 1 for e in forward_batch.extend_lens):     # :316-326
