@@ -475,15 +475,6 @@ int32_t tf_fp8_act_quant_amax(const void* x, int32_t x_dtype, int64_t rows, int6
                               int64_t x_row_stride, void* xq, int64_t xq_row_stride,
                               float* x_scale, const uint32_t* amax_bits, tf_stream_t stream);
 
-/* tf_fp8_act_quant_partials: tf_fp8_act_quant with max|x| known as npartial (at
- * most TF_FP8_QUANT_WORKSPACE_BYTES / 4) maxima over parts of x, as
- * tf_narrow_linear2 leaves them: the same x_scale and xq bit for bit.
- */
-int32_t tf_fp8_act_quant_partials(const void* x, int32_t x_dtype, int64_t rows, int64_t cols,
-                                  int64_t x_row_stride, void* xq, int64_t xq_row_stride,
-                                  float* x_scale, const uint32_t* partials, int32_t npartial,
-                                  tf_stream_t stream);
-
 /* tf_narrow_linear2: out_i = bf16(x w_i^T) for two narrow bf16 weights of one
  * input, fp32 accumulation (the in_proj_b / in_proj_a gate projections,
  * linear_attention.py:311-314).  x: bf16 [rows, k], k a multiple of 32, 16-byte
@@ -508,14 +499,19 @@ int32_t tf_fp8_block_gemm(const void* xq, int64_t xq_row_stride, const float* x_
 
 int64_t tf_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 
-/* tf_fp8_block_gemm_multi: tf_fp8_block_gemm of one activation matrix with up
- * to TF_FP8_MAX_MATS weight matrices in one launch (a layer's projections of
- * the same input: full_attention.py:122-139, linear_attention.py:309-314).
- * Each matrix has its own weight, block scales, bias and output; k, block_h
- * and block_w are common.  Outputs are those of one call per matrix except
- * for the order of fp32 sums where the split over K differs.  mats is a host
- * array, read during the call.  workspace: optional, as there,
- * tf_fp8_block_gemm_multi_workspace_bytes(m, n of each matrix, n_mats, k).
+/* tf_fp8_linears: one to TF_FP8_MAX_MATS block-FP8 linears of one bf16 input (a
+ * layer's projections: full_attention.py:122-139, linear_attention.py:309-314):
+ * x [m, k] is quantised once (as tf_fp8_act_quant does; x 16-byte aligned with a
+ * row stride that is a multiple of 8, k a multiple of 128) and one GEMM launch
+ * multiplies it with every weight.  Each matrix has its own weight, block
+ * scales, bias and output; block_h and block_w are common.  Outputs are those of
+ * tf_fp8_block_gemm per matrix except for the order of fp32 sums where the
+ * split over K differs.  mats is a host array, read during the call.
+ * amax_partials (NULL: max|x| is computed here): n_partials (at most
+ * TF_FP8_QUANT_WORKSPACE_BYTES / 4) maxima over parts of x as bf16 bit patterns,
+ * as the attention kernels' out_amax (one) and tf_narrow_linear2 leave them.
+ * workspace: device, 16-byte aligned, tf_fp8_linears_workspace_bytes bytes (for
+ * the quantised rows and the split over K).
  */
 #define TF_FP8_MAX_MATS 4
 
@@ -530,13 +526,13 @@ typedef struct tf_fp8_mat {
   int64_t out_row_stride;
 } tf_fp8_mat;
 
-int32_t tf_fp8_block_gemm_multi(const void* xq, int64_t xq_row_stride, const float* x_scale,
-                                const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h,
-                                int32_t block_w, int64_t m, int64_t k, void* workspace,
-                                int64_t workspace_bytes, tf_stream_t stream);
+int32_t tf_fp8_linears(const void* x, int64_t x_row_stride, const uint32_t* amax_partials,
+                       int32_t n_partials, const tf_fp8_mat* mats, int32_t n_mats,
+                       int32_t block_h, int32_t block_w, int64_t m, int64_t k, void* workspace,
+                       int64_t workspace_bytes, tf_stream_t stream);
 
-int64_t tf_fp8_block_gemm_multi_workspace_bytes(int64_t m, const int64_t* n, int32_t n_mats,
-                                                int64_t k);
+int64_t tf_fp8_linears_workspace_bytes(int64_t m, const tf_fp8_mat* mats, int32_t n_mats,
+                                       int64_t k);
 
 /* ------------------------------------------------------------------ Gated DeltaNet decode
  * One-token step of the linear-attention (Gated DeltaNet) layers for a batch

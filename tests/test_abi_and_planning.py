@@ -160,20 +160,26 @@ def test_plan_decode_items_lists_single_token_requests():
 
 
 def test_fp8_gemm_workspace_queries_agree():
-    """The size query of a one-matrix call is that of the plain call, a split
-    workspace holds whole fp32 partials of every matrix, and widths that are not
-    multiples of 4 never split."""
+    """The split scratch of a one-matrix call is that of the plain GEMM, it holds
+    whole fp32 partials of every matrix, and widths that are not multiples of 4
+    never split."""
     lib = _native.load()
+    mats = (_native.Fp8Mat * 5)()
+
+    def scratch(m, ns, k):
+        for mat, n in zip(mats, ns):
+            mat.n = n
+        fixed = (m * k + 255) // 256 * 256 + 256 + _native.TF_FP8_QUANT_WORKSPACE_BYTES
+        return lib.tf_fp8_linears_workspace_bytes(m, mats, len(ns), k) - fixed
+
     for m in (1, 16, 48, 64, 100, 300, 512, 700, 2000, 9000):
         for n in (128, 1024, 5120, 5122, 12288):
             for k in (128, 256, 5120):
                 one = lib.tf_fp8_block_gemm_workspace_bytes(m, n, k)
-                cols = (ctypes.c_int64 * 1)(n)
-                assert lib.tf_fp8_block_gemm_multi_workspace_bytes(m, cols, 1, k) == one
+                assert scratch(m, [n], k) == one
                 assert one % (4 * m * n) == 0 and (n % 4 == 0 or one == 0)
-    cols = (ctypes.c_int64 * 3)(1024, 256, 130)
-    assert lib.tf_fp8_block_gemm_multi_workspace_bytes(48, cols, 3, 5120) == 0
-    cols[2] = 132
-    nbytes = lib.tf_fp8_block_gemm_multi_workspace_bytes(48, cols, 3, 5120)
+    assert scratch(48, [1024, 256, 130], 5120) == 0
+    nbytes = scratch(48, [1024, 256, 132], 5120)
     assert nbytes > 0 and nbytes % (4 * 48 * (1024 + 256 + 132)) == 0
-    assert lib.tf_fp8_block_gemm_multi_workspace_bytes(48, cols, 5, 5120) < 0
+    assert lib.tf_fp8_linears_workspace_bytes(48, mats, 5, 5120) < 0
+    assert lib.tf_fp8_linears_workspace_bytes(48, mats, 1, 5100) < 0

@@ -324,22 +324,43 @@ def test_projections_of_one_input_in_one_launch(gpu, m, bias):
 @pytest.mark.parametrize("n,k", [(6, 128), (16, 64), (48, 5120), (33, 96), (64, 1024)])
 def test_narrow_linears(gpu, rows, n, k):
     """Two narrow bf16 linears in one launch, on a strided input, against fp64,
-    and the quantisation from its maxima against the two-pass one bit for bit."""
+    and an FP8 linear from its maxima against one that takes its own."""
     g = torch.Generator().manual_seed(rows + n)
     x = torch.randn((rows, 2 * k), generator=g).to(torch.bfloat16).to(gpu)[:, :k]
     lins = [torch.nn.Linear(k, n, bias=False, dtype=torch.bfloat16, device=gpu)
             .requires_grad_(False) for _ in range(2)]
     print(f"[narrow] rows={rows} n={n} k={k}", flush=True)
     first, second, amax = fl.narrow_linears(x, *lins)
-    xq, scale = fl.quantize_activations(x, amax_partials=amax)
-    want_q, want_scale = fl.quantize_activations(x)
     torch.cuda.synchronize()
     for got, lin in zip((first, second), lins):
         ref = x.double().cpu() @ lin.weight.double().cpu().t()
         # one bf16 rounding (2^-9) and fp32 sums of k terms of about 1/sqrt(k) each
         assert torch.allclose(got.double().cpu(), ref, rtol=2 ** -8, atol=1e-5)
-    assert torch.equal(scale, want_scale)
-    assert torch.equal(xq.view(torch.uint8), want_q.view(torch.uint8))
+    assert amax.max().item() == x.abs().max().view(torch.int16).item()
+    if k % 128 == 0:
+        lin = fl.Fp8Linear(k, 132).to(gpu)
+        lin.quantize_from(torch.randn((132, k), generator=g).to(gpu) * k ** -0.5)
+        assert torch.equal(fl.fp8_linears(x, [lin], amax)[0], fl.fp8_linears(x, [lin])[0])
+
+
+@pytest.mark.parametrize("m", [1, 48, 300])
+def test_linear_is_its_quantisation_and_gemm(gpu, m):
+    """The one-call linear against the quantisation and the GEMM called apart, bit
+    for bit, with and without the input's amax; a scale tensor of the wrong
+    shape is refused by one linear and by several."""
+    g = torch.Generator().manual_seed(m)
+    lin = fl.Fp8Linear(768, 260, bias=True).to(gpu)
+    lin.quantize_from(torch.randn((260, 768), generator=g).to(gpu))
+    x = torch.randn((m, 2 * 768), generator=g).to(torch.bfloat16).to(gpu)[:, :768]
+    xq, scale = fl.quantize_activations(x)
+    want = fl.block_fp8_gemm(xq, scale, lin.weight, lin.weight_scale_inv, lin.bias)
+    amax = x.abs().max().view(torch.int16).to(torch.int32).reshape(1)
+    assert torch.equal(lin(x), want) and torch.equal(lin(x, x_amax=amax), want)
+    assert lin(x[:0]).shape == (0, 260)
+    lin.weight_scale_inv = lin.weight_scale_inv[:2].clone()
+    for call in (lambda: lin(x), lambda: fl.fp8_linears(x, [lin, lin])):
+        with pytest.raises(ValueError, match="weight_scale_inv"):
+            call()
 
 
 def test_narrow_linears_call_what_is_not_plain(gpu):

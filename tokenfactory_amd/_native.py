@@ -11,6 +11,8 @@ import threading
 from pathlib import Path
 from typing import Optional
 
+import torch
+
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libtf_attn.so"
 ABI_VERSION = 12
 
@@ -148,11 +150,6 @@ SIGNATURES = {
         _p, _i64, _p,                  # xq, xq_row_stride, x_scale
         _p, _p,                        # amax_bits, stream
     ]),
-    "tf_fp8_act_quant_partials": (_i32, [
-        _p, _i32, _i64, _i64, _i64,    # x, x_dtype, rows, cols, x_row_stride
-        _p, _i64, _p,                  # xq, xq_row_stride, x_scale
-        _p, _i32, _p,                  # partials, npartial, stream
-    ]),
     "tf_narrow_linear2_blocks": (_i32, [_i64]),
     "tf_narrow_linear2": (_i32, [
         _p, _i64, _i64, _i64,          # x, x_row_stride, rows, k
@@ -168,13 +165,12 @@ SIGNATURES = {
         _p, _i64, _p,                  # workspace, workspace_bytes, stream
     ]),
     "tf_fp8_block_gemm_workspace_bytes": (_i64, [_i64, _i64, _i64]),
-    "tf_fp8_block_gemm_multi": (_i32, [
-        _p, _i64, _p,                  # xq, xq_row_stride, x_scale
+    "tf_fp8_linears": (_i32, [
+        _p, _i64, _p, _i32,            # x, x_row_stride, amax_partials, n_partials
         _p, _i32, _i32, _i32,          # mats, n_mats, block_h, block_w
-        _i64, _i64,                    # m, k
-        _p, _i64, _p,                  # workspace, workspace_bytes, stream
+        _i64, _i64, _p, _i64, _p,      # m, k, workspace, workspace_bytes, stream
     ]),
-    "tf_fp8_block_gemm_multi_workspace_bytes": (_i64, [_i64, _p, _i32, _i64]),
+    "tf_fp8_linears_workspace_bytes": (_i64, [_i64, _p, _i32, _i64]),
     "tf_gdn_decode": (_i32, [
         _p, _i64, _p, _p, _i64,        # qkv, qkv_row_stride, a, b, ab_row_stride
         _p, _i64,                      # z, z_row_stride
@@ -211,7 +207,7 @@ SIGNATURES["tf_attn_decode_merge"] = SIGNATURES["tf_attn_decode"]
 
 
 class Fp8Mat(ctypes.Structure):
-    """``tf_fp8_mat``: one weight matrix of ``tf_fp8_block_gemm_multi``."""
+    """``tf_fp8_mat``: one weight matrix of ``tf_fp8_linears``."""
 
     _fields_ = [("w", _p), ("w_row_stride", _i64), ("w_scale", _p),
                 ("w_scale_row_stride", _i64), ("w_scale_col_stride", _i64), ("bias", _p),
@@ -240,6 +236,8 @@ _lib: Optional[ctypes.CDLL] = None
 def load(path: Optional[Path] = None) -> ctypes.CDLL:
     """Loads (once) and returns the library with every signature declared."""
     global _lib
+    if _lib is not None and path is None:
+        return _lib
     with _lock:
         if _lib is not None and path is None:
             return _lib
@@ -276,6 +274,13 @@ def call(name: str, *args) -> int:
             raise NotImplementedError(f"{name}: {msg}")
         raise NativeCallError(name, rc, msg)
     return rc
+
+
+def current_stream(device) -> int:
+    """The handle of ``device``'s current stream (0 = the default stream), without
+    the ``torch.cuda.Stream`` object that ``torch.cuda.current_stream`` makes
+    (about 2 us per launch)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def plan_device_capacity(total_tokens, batch_size, num_q_heads, num_kv_heads) -> int:

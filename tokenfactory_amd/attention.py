@@ -39,10 +39,9 @@ _ws_lock = threading.Lock()
 _workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
 
 
-def _workspace(device: torch.device, stream: torch.cuda.Stream, nbytes: int) -> torch.Tensor:
+def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
     """Decode split-partial scratch, one per (device, stream), grown on demand."""
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           stream.cuda_stream)
+    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     with _ws_lock:
         ws = _workspaces.get(key)
         if ws is None or ws.numel() < nbytes:
@@ -576,7 +575,7 @@ class SlotAttentionCall:
             nbytes = _native.decode_workspace_bytes(self.n_dec, n_q, n_kv, head_dim,
                                                     self.max_len, self.decode_workgroups)
         if nbytes:
-            self.ws = _workspace(q.device, self.stream, nbytes)
+            self.ws = _workspace(q.device, self._stream_handle, nbytes)
 
     @property
     def stream(self) -> torch.cuda.Stream:
@@ -585,6 +584,11 @@ class SlotAttentionCall:
         if self._fixed_stream is not None:
             return self._fixed_stream
         return torch.cuda.current_stream(self.q.device)
+
+    @property
+    def _stream_handle(self) -> int:
+        return (self._fixed_stream.cuda_stream if self._fixed_stream is not None
+                else _native.current_stream(self.q.device))
 
     # -- launches
     def run_plan(self) -> None:
@@ -626,7 +630,7 @@ class SlotAttentionCall:
 
     def _decode(self, entry: str, stream: Optional[torch.cuda.Stream] = None) -> None:
         ws = self.ws
-        stream = stream if stream is not None else self.stream
+        handle = stream.cuda_stream if stream is not None else self._stream_handle
         if self._n_rows_items:
             if entry == "tf_attn_decode_merge":
                 return   # part of the rows launch
@@ -636,7 +640,7 @@ class SlotAttentionCall:
                          self.n_q, self.n_kv, self.head_dim, self.scaling,
                          self.out.data_ptr(), self.out.stride(0),
                          _ptr(ws), 0 if ws is None else ws.numel(), self.decode_workgroups,
-                         *self._epilogue_args, stream.cuda_stream)
+                         *self._epilogue_args, handle)
             return
         if not self.n_dec or not self.route.run_rows:
             return
@@ -645,7 +649,7 @@ class SlotAttentionCall:
                      self.n_q, self.n_kv, self.head_dim, self.scaling,
                      self.out.data_ptr(), self.out.stride(0),
                      _ptr(ws), 0 if ws is None else ws.numel(), self.max_len,
-                     self.decode_workgroups, *self._epilogue_args, stream.cuda_stream)
+                     self.decode_workgroups, *self._epilogue_args, handle)
 
     def run_extend(self) -> None:
         if self.n_work and self.route.run_extend:
@@ -663,13 +667,13 @@ class SlotAttentionCall:
                              *self._pool_args, work, n_work, work + 32 * n_work,
                              self.route.n_merges, ws.data_ptr(), ws.numel(), self.n_q, self.n_kv,
                              self.scaling, self.out.data_ptr(), self.out.stride(0),
-                             *self._epilogue_args, self.stream.cuda_stream)
+                             *self._epilogue_args, self._stream_handle)
                 return
             _native.call("tf_attn_extend", self.q.data_ptr(), self.q.stride(0),
                          *self._pool_args, work, n_work,
                          self.n_q, self.n_kv, self.head_dim, self.scaling,
                          self.out.data_ptr(), self.out.stride(0), *self._epilogue_args,
-                         self.stream.cuda_stream)
+                         self._stream_handle)
 
     def run_decode_partial(self) -> None:
         self._decode("tf_attn_decode_partial")
@@ -785,7 +789,7 @@ def gather_kv(pool: torch.Tensor, req_to_token: torch.Tensor, req_pool_indices: 
     _native.call("tf_gather_kv", pool.data_ptr(), dtype_code, pool.shape[0], row_elems,
                  req_to_token.data_ptr(), req_to_token.shape[0], req_to_token.stride(0),
                  req_to_token.shape[1], rpi.data_ptr(), bsz, max_len,
-                 out.data_ptr(), torch.cuda.current_stream(pool.device).cuda_stream)
+                 out.data_ptr(), _native.current_stream(pool.device))
     return out
 
 
@@ -823,7 +827,14 @@ def write_kv(layer_k_buffer: torch.Tensor, layer_v_buffer: torch.Tensor,
                  loc.data_ptr(), loc.numel(), layer_k_buffer.data_ptr(),
                  layer_v_buffer.data_ptr(), layer_k_buffer.shape[0], kv_dtype,
                  _ptr(k_scale), _ptr(v_scale), n_kv, head_dim,
-                 torch.cuda.current_stream(k.device).cuda_stream)
+                 _native.current_stream(k.device))
+
+
+def _as(t: torch.Tensor, device: torch.device, dtype: torch.dtype) -> torch.Tensor:
+    """``t`` contiguous on ``device`` as ``dtype``; itself where it is that already."""
+    if t.dtype == dtype and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=dtype).contiguous()
 
 
 def qk_norm_rope_kv_write(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -868,18 +879,17 @@ def qk_norm_rope_kv_write(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             raise ValueError("an fp8 KV pool needs k_scale and v_scale")
         k_scale = k_scale.to(device=q.device, dtype=torch.float32).reshape(1).contiguous()
         v_scale = v_scale.to(device=q.device, dtype=torch.float32).reshape(1).contiguous()
-    loc = out_cache_loc.to(device=q.device, dtype=torch.int64).contiguous()
+    dev = q.device
+    loc = _as(out_cache_loc, dev, torch.int64)
     if loc.numel() != T:
         raise ValueError(f"out_cache_loc has {loc.numel()} slots for {T} tokens")
-    pos = positions.to(device=q.device, dtype=torch.int64)
-    if pos.dim() == 1:
-        pos = pos.reshape(1, -1)
+    pos = positions.reshape(1, -1) if positions.dim() == 1 else positions
     if pos.dim() != 2 or pos.shape[0] not in (1, 3) or pos.shape[1] != T:
         raise ValueError(f"positions {tuple(positions.shape)} for {T} tokens")
-    pos = pos.contiguous()
-    qw = q_norm_weight.to(device=q.device, dtype=torch.float32).contiguous()
-    kw = k_norm_weight.to(device=q.device, dtype=torch.float32).contiguous()
-    freqs = inv_freq.to(device=q.device, dtype=torch.float32).contiguous()
+    pos = _as(pos, dev, torch.int64)
+    qw = _as(q_norm_weight, dev, torch.float32)
+    kw = _as(k_norm_weight, dev, torch.float32)
+    freqs = _as(inv_freq, dev, torch.float32)
     if freqs.numel() != rotary_dim // 2:
         raise ValueError(f"inv_freq has {freqs.numel()} entries for rotary_dim {rotary_dim}")
     sec = list(mrope_section) if mrope_section is not None else [0, 0, 0]
@@ -892,5 +902,5 @@ def qk_norm_rope_kv_write(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                  int(bool(mrope_interleaved)), out.data_ptr(), out.stride(0), loc.data_ptr(),
                  layer_k_buffer.data_ptr(), layer_v_buffer.data_ptr(),
                  layer_k_buffer.shape[0], kv_dtype, _ptr(k_scale), _ptr(v_scale),
-                 torch.cuda.current_stream(q.device).cuda_stream)
+                 _native.current_stream(q.device))
     return out

@@ -631,11 +631,12 @@ void launch_shape(const GemmArgs& a, Shape sh, hipStream_t s) {
     launch_gemm<8, 4, 2>(a, s);
 }
 
-// Validates the arguments of both GEMM entry points and launches the call.
-int32_t gemm_call(const char* fn, const void* xq, int64_t xq_row_stride, const float* x_scale,
-                  const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h, int32_t block_w,
-                  int64_t m, int64_t k, void* workspace, int64_t workspace_bytes,
-                  tf_stream_t stream) {
+// Validates the GEMM arguments of both entry points and plans the launch (m == 0:
+// none, args is left alone).
+int32_t gemm_setup(const char* fn, const void* xq, int64_t xq_row_stride, const float* x_scale,
+                   const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h, int32_t block_w,
+                   int64_t m, int64_t k, void* workspace, int64_t workspace_bytes,
+                   GemmArgs* args, Shape* shape) {
   if (n_mats < 1 || n_mats > kMaxMats || !mats)
     return fail(TF_ERR_INVALID, "%s: n_mats=%d (1 to %d)", fn, n_mats, kMaxMats);
   if (m < 0 || k <= 0 || k % kKSlice)
@@ -710,8 +711,21 @@ int32_t gemm_call(const char* fn, const void* xq, int64_t xq_row_stride, const f
       sh = p.whole;
     }
   }
-  launch_shape(a, sh, reinterpret_cast<hipStream_t>(stream));
-  return launch_status("tf_fp8_block_gemm launch");
+  *args = a;
+  *shape = sh;
+  return TF_OK;
+}
+
+// tf_fp8_linears' workspace: quantised rows, x_scale, amax partials, split scratch.
+struct LinearsLayout {
+  int64_t scale, partial, gemm;
+};
+LinearsLayout linears_layout(int64_t m, int64_t k) {
+  LinearsLayout l;
+  l.scale = (m * k + 255) & ~255LL;
+  l.partial = l.scale + 256;
+  l.gemm = l.partial + TF_FP8_QUANT_WORKSPACE_BYTES;
+  return l;
 }
 
 // Validates the arguments both quantisation entry points share and fills a.
@@ -797,53 +811,65 @@ int32_t tf_fp8_act_quant_amax(const void* x, int32_t x_dtype, int64_t rows, int6
   return launch_status("tf_fp8_act_quant_amax launch");
 }
 
-int32_t tf_fp8_act_quant_partials(const void* x, int32_t x_dtype, int64_t rows, int64_t cols,
-                                  int64_t x_row_stride, void* xq, int64_t xq_row_stride,
-                                  float* x_scale, const uint32_t* partials, int32_t npartial,
-                                  tf_stream_t stream) {
+int32_t tf_fp8_linears(const void* x, int64_t x_row_stride, const uint32_t* amax_partials,
+                       int32_t n_partials, const tf_fp8_mat* mats, int32_t n_mats,
+                       int32_t block_h, int32_t block_w, int64_t m, int64_t k, void* workspace,
+                       int64_t workspace_bytes, tf_stream_t stream) {
   using namespace tfa;
-  clear_error();
-  QuantArgs a;
-  const int32_t rc = quant_setup("fp8_act_quant_partials", x, x_dtype, rows, cols, x_row_stride,
-                                 xq, xq_row_stride, x_scale, &a);
+  const int64_t need = tf_fp8_linears_workspace_bytes(m, mats, n_mats, k);   // clears the error
+  if (need < 0) return (int32_t)need;
+  if (m == 0) return TF_OK;
+  if (!workspace || !aligned16(workspace) || workspace_bytes < need)
+    return fail(TF_ERR_INVALID, "fp8_linears: workspace of %lld bytes (needs %lld, 16-byte aligned)",
+                (long long)workspace_bytes, (long long)need);
+  if (amax_partials && ((reinterpret_cast<uintptr_t>(amax_partials) & 3u) || n_partials < 1 ||
+                        n_partials > kQuantMaxBlocks))
+    return fail(TF_ERR_INVALID, "fp8_linears: %d partials (1 to %d, 4-byte aligned)", n_partials,
+                kQuantMaxBlocks);
+  uint8_t* w = static_cast<uint8_t*>(workspace);
+  const LinearsLayout l = linears_layout(m, k);
+  float* x_scale = reinterpret_cast<float*>(w + l.scale);
+  QuantArgs q;
+  int32_t rc = quant_setup("fp8_linears", x, TF_DTYPE_BF16, m, k, x_row_stride, w, k, x_scale, &q);
   if (rc != TF_OK) return rc;
-  if (!partials || (reinterpret_cast<uintptr_t>(partials) & 3u) || npartial < 1 ||
-      npartial > kQuantMaxBlocks)
-    return fail(TF_ERR_INVALID, "fp8_act_quant_partials: %d partials (1 to %d, 4-byte aligned)",
-                npartial, kQuantMaxBlocks);
-  a.partial = partials;
-  a.npartial = (uint32_t)npartial;
-  hipLaunchKernelGGL(act_quant_kernel, dim3(a.nblocks), dim3(kThreads), 0,
-                     reinterpret_cast<hipStream_t>(stream), a);
-  return launch_status("tf_fp8_act_quant_partials launch");
-}
-
-int32_t tf_fp8_block_gemm_multi(const void* xq, int64_t xq_row_stride, const float* x_scale,
-                                const tf_fp8_mat* mats, int32_t n_mats, int32_t block_h,
-                                int32_t block_w, int64_t m, int64_t k, void* workspace,
-                                int64_t workspace_bytes, tf_stream_t stream) {
-  using namespace tfa;
-  clear_error();
-  return gemm_call("fp8_block_gemm_multi", xq, xq_row_stride, x_scale, mats, n_mats, block_h,
-                   block_w, m, k, workspace, workspace_bytes, stream);
-}
-
-int64_t tf_fp8_block_gemm_multi_workspace_bytes(int64_t m, const int64_t* n, int32_t n_mats,
-                                                int64_t k) {
-  using namespace tfa;
-  clear_error();
-  if (m < 0 || n_mats < 1 || n_mats > kMaxMats || !n || k <= 0 || k % kKSlice)
-    return fail(TF_ERR_INVALID, "fp8_block_gemm_multi_workspace_bytes: m=%lld n_mats=%d k=%lld",
-                (long long)m, n_mats, (long long)k);
-  int64_t cols = 0;
-  for (int i = 0; i < n_mats; ++i) {
-    if (n[i] <= 0 || n[i] > INT32_MAX / 2)
-      return fail(TF_ERR_INVALID, "fp8_block_gemm_multi_workspace_bytes: n[%d]=%lld", i,
-                  (long long)n[i]);
-    cols += n[i];
+  GemmArgs g;
+  Shape sh;
+  rc = gemm_setup("fp8_linears", w, k, x_scale, mats, n_mats, block_h, block_w, m, k,
+                  need > l.gemm ? w + l.gemm : nullptr, need - l.gemm, &g, &sh);
+  if (rc != TF_OK) return rc;   // nothing is launched for arguments that any part refuses
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (amax_partials) {
+    q.partial = amax_partials;
+    q.npartial = (uint32_t)n_partials;
+  } else {
+    uint32_t* partial = reinterpret_cast<uint32_t*>(w + l.partial);
+    q.partial = partial;
+    q.npartial = q.nblocks;
+    hipLaunchKernelGGL(act_amax_kernel, dim3(q.nblocks), dim3(kThreads), 0, s, q, partial);
   }
-  const int splits = gemm_plan(m, n, n_mats, k).splits;
-  return splits > 1 ? (int64_t)splits * m * cols * 4 : 0;
+  hipLaunchKernelGGL(act_quant_kernel, dim3(q.nblocks), dim3(kThreads), 0, s, q);
+  launch_shape(g, sh, s);
+  return launch_status("tf_fp8_linears launch");
+}
+
+int64_t tf_fp8_linears_workspace_bytes(int64_t m, const tf_fp8_mat* mats, int32_t n_mats,
+                                       int64_t k) {
+  using namespace tfa;
+  clear_error();
+  if (m < 0 || m > INT32_MAX / 2 || n_mats < 1 || n_mats > kMaxMats || !mats || k <= 0 ||
+      k % kKSlice || k > INT32_MAX / 2)
+    return fail(TF_ERR_INVALID, "fp8_linears: m=%lld n_mats=%d (1 to %d) k=%lld (a multiple of %d)",
+                (long long)m, n_mats, kMaxMats, (long long)k, kKSlice);
+  int64_t n_of[kMaxMats], cols = 0;
+  for (int i = 0; i < n_mats; ++i) {
+    n_of[i] = mats[i].n;
+    if (n_of[i] <= 0 || n_of[i] > INT32_MAX / 2)
+      return fail(TF_ERR_INVALID, "fp8_linears: n[%d]=%lld", i, (long long)n_of[i]);
+    cols += n_of[i];
+  }
+  if (m == 0) return 0;
+  const int splits = gemm_plan(m, n_of, n_mats, k).splits;
+  return linears_layout(m, k).gemm + (splits > 1 ? (int64_t)splits * m * cols * 4 : 0);
 }
 
 int32_t tf_fp8_block_gemm(const void* xq, int64_t xq_row_stride, const float* x_scale,
@@ -856,8 +882,13 @@ int32_t tf_fp8_block_gemm(const void* xq, int64_t xq_row_stride, const float* x_
   clear_error();
   const tf_fp8_mat mat = {w, w_row_stride, w_scale, w_scale_row_stride, w_scale_col_stride,
                           bias, n, out, out_row_stride};
-  return gemm_call("fp8_block_gemm", xq, xq_row_stride, x_scale, &mat, 1, block_h, block_w, m, k,
-                   workspace, workspace_bytes, stream);
+  GemmArgs a;
+  Shape sh;
+  const int32_t rc = gemm_setup("fp8_block_gemm", xq, xq_row_stride, x_scale, &mat, 1, block_h,
+                                block_w, m, k, workspace, workspace_bytes, &a, &sh);
+  if (rc != TF_OK || m == 0) return rc;
+  launch_shape(a, sh, reinterpret_cast<hipStream_t>(stream));
+  return launch_status("tf_fp8_block_gemm launch");
 }
 
 int64_t tf_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {

@@ -16,7 +16,6 @@ There is no non-native path: without the library every call raises.
 from __future__ import annotations
 
 import contextlib
-import ctypes
 import math
 from typing import Optional, Sequence
 
@@ -33,8 +32,7 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
 
 
 def _stream_ptr(stream, device) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream(device)
-    return s.cuda_stream
+    return stream.cuda_stream if stream is not None else _native.current_stream(device)
 
 
 def on_stream(stream):
@@ -62,9 +60,15 @@ def _pad_cols(t: torch.Tensor, cols: int) -> torch.Tensor:
     return out.view(t.dtype)
 
 
+def _check_amax(amax: Optional[torch.Tensor], x2d: torch.Tensor, limit: int) -> None:
+    if amax is not None and (amax.dtype != torch.int32 or not 1 <= amax.numel() <= limit
+                             or amax.device != x2d.device or not amax.is_contiguous()):
+        raise ValueError(f"the amax of x must be a contiguous int32 tensor on x's device with "
+                         f"1 to {limit} elements")
+
+
 def quantize_activations(x2d: torch.Tensor, stream=None, padded_cols: Optional[int] = None,
-                         amax: Optional[torch.Tensor] = None,
-                         amax_partials: Optional[torch.Tensor] = None):
+                         amax: Optional[torch.Tensor] = None):
     """Dynamic per-tensor e4m3 quantisation of a bf16 ``[rows, cols]`` matrix
     (``fp8_triton.py:127-130``). Returns ``(xq, x_scale)``: float8_e4m3fn rows
     and a 1-element fp32 tensor holding ``bf16(max(amax|x|, 1e-12) / 448)``.
@@ -72,8 +76,7 @@ def quantize_activations(x2d: torch.Tensor, stream=None, padded_cols: Optional[i
     ``amax``: the max of ``|x|`` already computed by x's producer (a 1-element
     int32 device tensor holding the bf16 bit pattern, as the attention kernels'
     ``out_amax`` leaves it); the result is the same, with one launch
-    (``tf_fp8_act_quant_amax``) instead of two.  ``amax_partials``: the same as
-    int32 maxima over parts of x (``narrow_linears``)."""
+    (``tf_fp8_act_quant_amax``) instead of two."""
     if x2d.dtype != torch.bfloat16 or x2d.dim() != 2 or not x2d.is_cuda:
         raise ValueError("quantize_activations: x must be a 2-D bf16 CUDA tensor")
     if x2d.stride(1) != 1:
@@ -88,21 +91,9 @@ def quantize_activations(x2d: torch.Tensor, stream=None, padded_cols: Optional[i
             xq.view(torch.uint8)[:, cols:].zero_()
         scale = torch.empty((1,), dtype=torch.float32, device=x2d.device)
         if amax is not None:
-            if amax.dtype != torch.int32 or amax.numel() != 1 or amax.device != x2d.device:
-                raise ValueError("quantize_activations: amax must be a 1-element int32 tensor "
-                                 "on x's device")
+            _check_amax(amax, x2d, 1)
             _native.call("tf_fp8_act_quant_amax", _ptr(x2d), _native.TF_DTYPE_BF16, rows, cols,
                          x2d.stride(0), _ptr(xq), xq.stride(0), _ptr(scale), _ptr(amax),
-                         _stream_ptr(stream, x2d.device))
-            return xq, scale
-        if amax_partials is not None:
-            if amax_partials.dtype != torch.int32 or amax_partials.device != x2d.device \
-                    or not amax_partials.is_contiguous():
-                raise ValueError("quantize_activations: amax_partials must be a contiguous int32 "
-                                 "tensor on x's device")
-            _native.call("tf_fp8_act_quant_partials", _ptr(x2d), _native.TF_DTYPE_BF16, rows,
-                         cols, x2d.stride(0), _ptr(xq), xq.stride(0), _ptr(scale),
-                         _ptr(amax_partials), amax_partials.numel(),
                          _stream_ptr(stream, x2d.device))
             return xq, scale
         ws = torch.empty((_native.TF_FP8_QUANT_WORKSPACE_BYTES,), dtype=torch.uint8,
@@ -171,6 +162,55 @@ def block_fp8_gemm(xq: torch.Tensor, x_scale: torch.Tensor, weight: torch.Tensor
     return out
 
 
+def _takes(x2d: torch.Tensor) -> bool:
+    """Whether x is what ``tf_fp8_linears`` takes (else: the calls step by step,
+    which pad a K that is not a multiple of 128, or say what is wrong)."""
+    return x2d.is_cuda and x2d.dtype == torch.bfloat16 and x2d.shape[1] % K_SLICE == 0
+
+
+def _shared(x2d: torch.Tensor, w: torch.Tensor, scale: Optional[torch.Tensor],
+            bias: Optional[torch.Tensor], block_h: int, block_w: int) -> bool:
+    """Whether one weight of block size (block_h, block_w) is what
+    ``tf_fp8_linears`` takes with x."""
+    dev = x2d.device
+    if (w.dtype != torch.float8_e4m3fn or w.dim() != 2 or w.device != dev
+            or not w.is_contiguous() or scale is None or scale.dtype != torch.float32
+            or scale.device != dev):
+        return False
+    n, k = w.shape
+    return (k == x2d.shape[1] and scale.shape == (-(-n // block_h), -(-k // block_w))
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.shape == (n,)
+                                  and bias.device == dev and bias.is_contiguous())))
+
+
+def _linears(x2d: torch.Tensor, weights, block_h: int, block_w: int,
+             amax: Optional[torch.Tensor] = None, stream=None):
+    """``[x2d w^T + bias]`` for (weight, scales, bias) triples that pass
+    ``_takes`` and ``_shared``, in one ``tf_fp8_linears`` call: one entry and
+    one workspace for the quantisation and the GEMM, since at decode sizes the
+    host's calls and allocations take longer than the kernels (full-attention
+    layer, 16 decodes: host 150 -> 109 us a call, kernels 97)."""
+    rows, k = x2d.shape
+    dev = x2d.device
+    n = len(weights)
+    mats = (_native.Fp8Mat * n)()
+    lib = _native.load()
+    with on_stream(stream):
+        outs = [torch.empty((rows, w.shape[0]), dtype=torch.bfloat16, device=dev)
+                for w, _, _ in weights]
+        for i, (w, scale, bias) in enumerate(weights):
+            cols = w.shape[0]
+            mats[i] = (w.data_ptr(), k, scale.data_ptr(), scale.stride(0), scale.stride(1),
+                       _ptr(bias), cols, outs[i].data_ptr(), cols)
+        if rows:
+            nbytes = lib.tf_fp8_linears_workspace_bytes(rows, mats, n, k)
+            ws = torch.empty((max(nbytes, 0),), dtype=torch.uint8, device=dev)
+            _native.call("tf_fp8_linears", x2d.data_ptr(), x2d.stride(0), _ptr(amax),
+                         0 if amax is None else amax.numel(), mats, n, block_h, block_w, rows, k,
+                         ws.data_ptr(), nbytes, _stream_ptr(stream, dev))
+    return outs
+
+
 def block_fp8_linear(x: torch.Tensor, weight: torch.Tensor,
                      weight_scale_inv: Optional[torch.Tensor], bias: Optional[torch.Tensor],
                      block_h: int = 128, block_w: int = 128, stream=None,
@@ -184,6 +224,11 @@ def block_fp8_linear(x: torch.Tensor, weight: torch.Tensor,
     x2d = x.reshape(-1, in_features)
     if x2d.stride(1) != 1:
         x2d = x2d.contiguous()
+    if x2d.shape[0] and _takes(x2d) and _shared(x2d, weight, weight_scale_inv, bias, block_h,
+                                                block_w):
+        _check_amax(x_amax, x2d, 1)
+        out, = _linears(x2d, ((weight, weight_scale_inv, bias),), block_h, block_w, x_amax, stream)
+        return out.reshape(*x.shape[:-1], weight.shape[0])
     xq, scale = quantize_activations(x2d, stream, padded_cols=_padded_k(in_features),
                                      amax=x_amax)
     out = block_fp8_gemm(xq, scale, weight, weight_scale_inv, bias, block_h, block_w,
@@ -203,7 +248,7 @@ def _plain(linear, kind) -> bool:
 def narrow_linears(x: torch.Tensor, first: nn.Linear, second: nn.Linear):
     """``(first(x), second(x), amax_partials)`` for two narrow bf16 linears of one
     input (``linear_attention.py:311-314``) in one ``tf_narrow_linear2`` launch,
-    with max ``|x|`` per row block for ``quantize_activations`` of the same x.
+    with max ``|x|`` per row block for ``fp8_linears`` of the same x.
     Linears that are more than plain bf16 ``nn.Linear`` calls without a bias, that
     autograd is to record or autocast to cast, or whose sizes the kernel does not
     take are called one by one (``amax_partials`` is then None)."""
@@ -234,49 +279,26 @@ def fp8_linears(x: torch.Tensor, linears: Sequence["Fp8Linear"],
                 amax_partials: Optional[torch.Tensor] = None):
     """``[lin(x) for lin in linears]`` for projections of the same input
     (``full_attention.py:122-139``, ``linear_attention.py:309-314``): x is
-    quantised once and one ``tf_fp8_block_gemm_multi`` launch multiplies it with
-    every weight.  Linears that do not share a block size and a K that is a
-    multiple of 128, or that are more than plain ``Fp8Linear`` calls, are called
-    one by one.  ``amax_partials``: see ``quantize_activations``."""
+    quantised once and one GEMM launch multiplies it with every weight
+    (``tf_fp8_linears``).  Linears that do not share a block size and a K that is
+    a multiple of 128, or that are more than plain ``Fp8Linear`` calls, are called
+    one by one.  ``amax_partials``: int32 maxima of ``|x|`` over parts of x, as
+    ``narrow_linears`` leaves them (the result is the same, a pass over x less)."""
     first = linears[0]
-    k = first.in_features
-    if (len(linears) > _native.TF_FP8_MAX_MATS or k % K_SLICE or x.shape[-1] != k
-            or not x.is_cuda or x.dtype != torch.bfloat16
-            or not all(_plain(m, Fp8Linear) and m.in_features == k and m.block_h == first.block_h
-                       and m.block_w == first.block_w and m.weight.is_contiguous()
-                       and m.weight.dtype == torch.float8_e4m3fn
-                       and m.weight.device == x.device
-                       and m.weight_scale_inv.dtype == torch.float32
-                       and m.weight_scale_inv.device == x.device
-                       and (m.bias is None or (m.bias.dtype == torch.bfloat16
-                                               and m.bias.is_contiguous()
-                                               and m.bias.device == x.device))
-                       for m in linears)):
-        return [m(x) for m in linears]
-    x2d = x.reshape(-1, k)
-    if x2d.stride(1) != 1:
-        x2d = x2d.contiguous()
-    rows = x2d.shape[0]
-    xq, scale = quantize_activations(x2d, amax_partials=amax_partials)
-    outs = [torch.empty((rows, m.out_features), dtype=torch.bfloat16, device=x.device)
-            for m in linears]
-    if rows:
-        n = len(linears)
-        mats = (_native.Fp8Mat * n)()
-        cols = (ctypes.c_int64 * n)()
-        for i, (m, out) in enumerate(zip(linears, outs)):
-            ws = m.weight_scale_inv
-            mats[i] = _native.Fp8Mat(_ptr(m.weight), k, _ptr(ws), ws.stride(0), ws.stride(1),
-                                     _ptr(m.bias), m.out_features, _ptr(out), m.out_features)
-            cols[i] = m.out_features
-        nbytes = _native.load().tf_fp8_block_gemm_multi_workspace_bytes(rows, cols, n, k)
-        if nbytes < 0:
-            raise ValueError("fp8_linears: bad shape")
-        scratch = torch.empty((nbytes,), dtype=torch.uint8, device=x.device) if nbytes else None
-        _native.call("tf_fp8_block_gemm_multi", _ptr(xq), xq.stride(0), _ptr(scale), mats, n,
-                     first.block_h, first.block_w, rows, k, _ptr(scratch), nbytes,
-                     _stream_ptr(None, x.device))
-    return [out.reshape(*x.shape[:-1], out.shape[1]) for out in outs]
+    k = x.shape[-1]
+    bh, bw = first.block_h, first.block_w
+    if len(linears) <= _native.TF_FP8_MAX_MATS \
+            and all(_plain(m, Fp8Linear) and m.block_h == bh and m.block_w == bw
+                    for m in linears):
+        x2d = x.reshape(-1, k)
+        if x2d.stride(1) != 1:
+            x2d = x2d.contiguous()
+        weights = [(m.weight, m.weight_scale_inv, m.bias) for m in linears]
+        if _takes(x2d) and all(_shared(x2d, *t, bh, bw) for t in weights):
+            _check_amax(amax_partials, x2d, _native.TF_FP8_QUANT_WORKSPACE_BYTES // 4)
+            outs = _linears(x2d, weights, bh, bw, amax_partials)
+            return outs if x.dim() == 2 else [o.reshape(*x.shape[:-1], o.shape[1]) for o in outs]
+    return [m(x) for m in linears]
 
 
 class Fp8Linear(nn.Module):

@@ -100,7 +100,7 @@ def gdn_decode_step(qkv: torch.Tensor, b: torch.Tensor, a: torch.Tensor, z: torc
                            layer_conv_state, layer_ssm_state, req_indices, num_v_heads)
     value_dim = num_v_heads * dv
     cs, ss = layer_conv_state, layer_ssm_state
-    s = stream if stream is not None else torch.cuda.current_stream(qkv.device)
+    s = stream.cuda_stream if stream is not None else _native.current_stream(qkv.device)
     with on_stream(stream):
         out = torch.empty((bsz, value_dim), dtype=torch.bfloat16, device=qkv.device)
         core = torch.empty_like(out) if return_core else None
@@ -113,7 +113,7 @@ def gdn_decode_step(qkv: torch.Tensor, b: torch.Tensor, a: torch.Tensor, z: torc
                      _ptr(ss), ss.stride(0), _ptr(req_indices), bsz, cs.shape[0], num_k_heads,
                      num_v_heads, dk, dv, CONV_KERNEL, _ptr(out), out.stride(0),
                      _ptr(core), 0 if core is None else core.stride(0), _ptr(ws),
-                     ws.numel(), s.cuda_stream)
+                     ws.numel(), s)
     return (out, core) if return_core else out
 
 
@@ -141,7 +141,7 @@ def gdn_extend_step(qkv: torch.Tensor, b: torch.Tensor, a: torch.Tensor, z: torc
                                                            num_v_heads)
     if ws_bytes < 0:
         raise ValueError("gdn_extend_step: bad head counts")
-    s = stream if stream is not None else torch.cuda.current_stream(qkv.device)
+    s = stream.cuda_stream if stream is not None else _native.current_stream(qkv.device)
     cs, ss = layer_conv_state, layer_ssm_state
     with on_stream(stream):
         tok = torch.tensor(offsets, dtype=torch.int32).to(qkv.device, non_blocking=True)
@@ -154,7 +154,7 @@ def gdn_extend_step(qkv: torch.Tensor, b: torch.Tensor, a: torch.Tensor, z: torc
                      _ptr(ss), ss.stride(0), _ptr(req_indices), _ptr(tok), len(lens), n_tok,
                      max(lens), cs.shape[0], num_k_heads, num_v_heads, dk, dv,
                      CONV_KERNEL, _ptr(out), out.stride(0), _ptr(core),
-                     0 if core is None else core.stride(0), _ptr(ws), ws.numel(), s.cuda_stream)
+                     0 if core is None else core.stride(0), _ptr(ws), ws.numel(), s)
     return (out, core) if return_core else out
 
 
