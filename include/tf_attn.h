@@ -585,7 +585,8 @@ int32_t tf_gdn_decode(const void* qkv, int64_t qkv_row_stride, const void* a, co
  * _gated_delta_rule_step, then the gated norm).  Request b owns the token rows
  * token_offsets[b] .. token_offsets[b + 1] - 1 of qkv, a, b, z and out
  * (device int32 [batch_size + 1], non-decreasing, clamped into [0, n_tokens]);
- * max_extend_len: the largest extend length (host int, validated only);
+ * max_extend_len: the largest extend length (host int; it only chooses how the
+ * work is split, the offsets decide what is done);
  * each request's conv runs over [conv_state, its tokens] and its state is
  * carried through its tokens in order.  The state update is the reference's
  * chunk-wise WY form (:194-242) with 32-token chunks (the same recurrence as
@@ -596,7 +597,9 @@ int32_t tf_gdn_decode(const void* qkv, int64_t qkv_row_stride, const void* a, co
  * slot), the state-independent part of every chunk in parallel, the
  * one-token requests' update (as in tf_gdn_decode) and the chunked recurrence
  * with the gated norm of its rows (one workgroup per request of two or more
- * tokens and value head, its state in registers from first chunk to last).
+ * tokens and value head, its state in registers from first chunk to last; for
+ * few long prompts two workgroups per value head and the norm in a launch of
+ * its own).
  * When the
  * batch can hold both kinds of request (batch_size > 1, max_extend_len > 1),
  * the one-token update of a call that is not under graph capture runs on a

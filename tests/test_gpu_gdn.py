@@ -196,6 +196,46 @@ def test_extend_matches_oracle(gpu, lens, hk, hv):
         check_chunked_outputs(out.cpu(), want_out, f"{what}: normed output", True)
 
 
+@pytest.mark.parametrize("lens", [[237], [236], [1, 300, 1], [1, 31, 512], [512, 512],
+                                  [3] * 20 + [600] + [2] * 20 + [1] * 5])
+def test_split_columns_match_oracle(gpu, lens):
+    """Few long prompts (two workgroups per value head) at the rule's edge, beside
+    short requests, and with more (request, head) items than workgroups; the
+    second call of each case, with half the lengths, is the other kernel's."""
+    test_extend_matches_oracle(gpu, lens, 4, 12)
+
+
+@pytest.mark.parametrize("n", [256, 290, 545])
+def test_split_columns_match_whole_heads(gpu, n):
+    """Twelve prompts as one batch (a workgroup per value head) and one by one
+    (two): the same sums in another order, on views with row strides of their
+    own, beside a slot outside the pool."""
+    hk, hv, bsz = 4, 12, 12
+    conv_dim = 2 * hk * 128 + hv * 128
+    g = torch.Generator().manual_seed(n)
+    cs = torch.randn((bsz, conv_dim, 3), generator=g).to(torch.bfloat16).to(gpu)
+    ss = (torch.randn((bsz, hv, 128, 128), generator=g) * 0.2).to(gpu)
+    cs2, ss2 = cs.clone(), ss.clone()
+    gp = [p.to(gpu) for p in make_params(hk, hv, 8)]
+    qkv, a, b, z = (torch.cat((x, x[:, :8]), dim=1).to(gpu)[:, :x.shape[1]]
+                    for x in make_step(n * bsz, hk, hv, n))
+    req = torch.arange(bsz, device=gpu)
+    req[5] = bsz
+    print(f"[gdn extend] {bsz} x {n} tokens, whole heads and split columns", flush=True)
+    out, core = gdn_extend_step(qkv, b, a, z, *gp, 1e-6, cs, ss, req, [n] * bsz, hk, hv,
+                                return_core=True)
+    for i in range(bsz):
+        r = slice(n * i, n * (i + 1))
+        one, one_core = gdn_extend_step(qkv[r], b[r], a[r], z[r], *gp, 1e-6, cs2, ss2,
+                                        req[i:i + 1], [n], hk, hv, return_core=True)
+        torch.cuda.synchronize()
+        check_chunked_outputs(one_core.cpu(), core[r].cpu(), f"request {i}: pre-norm", False)
+        check_chunked_outputs(one.cpu(), out[r].cpu(), f"request {i}: normed", True)
+    assert torch.equal(cs, cs2)
+    scale = float(ss.abs().max())
+    close_fraction(ss2.cpu(), ss.cpu(), 1e-5 * scale, 1e-4 * scale, 1e-3, "ssm state")
+
+
 def test_extend_of_single_tokens_equals_decode(gpu):
     hk, hv, bsz = 16, 48, 6
     conv_dim = 2 * hk * 128 + hv * 128

@@ -70,6 +70,7 @@ struct GdnArgs {
   int32_t* owner;        // extend: int32 [rows] request of each token row (-1: none / skipped)
   uint16_t* silu_tab;    // extend: bf16 SiLU of the bf16 values 2^-25 <= |y| < 2^7
   float* wrec;           // extend: fp32 [chunk slots, Hv, 2304] chunk records
+  int32_t* multi;        // extend: [0] = requests with two or more tokens, then their indices
   const int32_t* tok;    // extend: request b owns token rows tok[b] .. tok[b + 1] - 1
   int32_t rows;          // token rows of qkv / a / b / z / out (offsets are clamped to it)
   uint16_t* ws;          // bf16 [rows, conv_dim]: conv + SiLU outputs
@@ -313,8 +314,28 @@ __device__ __forceinline__ uint32_t silu_lookup(float y, const uint16_t* tab) {
 
 // owner[tt] = the request whose rows hold tt, or -1 when none does or the
 // request's slot is outside the pool (those rows are skipped everywhere).
-// Threads 0 .. kSiluTab - 1 also fill the SiLU table.
+// Threads 0 .. kSiluTab - 1 also fill the SiLU table.  With a.multi one more
+// workgroup lists the requests with two or more tokens and a slot in the pool
+// (in batch order) for gdn_cols_ext_kernel.
 __global__ void __launch_bounds__(kThreads) gdn_owner_kernel(GdnArgs a) {
+  if (a.multi && blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x >= kWave) return;
+    int n = 0;
+    for (int b0 = 0; b0 < a.batch; b0 += kWave) {
+      const int b = b0 + threadIdx.x;
+      bool in = false;
+      if (b < a.batch) {
+        const int t0 = min(max(a.tok[b], 0), a.rows);
+        const int64_t r = a.req[b];
+        in = min(max(a.tok[b + 1], t0), a.rows) - t0 >= 2 && r >= 0 && r < a.n_slots;
+      }
+      const uint64_t mask = __ballot(in);
+      if (in) a.multi[1 + n + __popcll(mask & ((1ull << threadIdx.x) - 1))] = b;
+      n += __popcll(mask);
+    }
+    if (threadIdx.x == 0) a.multi[0] = n;
+    return;
+  }
   const int tt = blockIdx.x * kThreads + threadIdx.x;
   if (tt < kSiluTab) {
     const uint32_t u = ((uint32_t)(tt >> 12) << 15) | ((uint32_t)(kSiluELo + ((tt >> 7) & 31)) << 7) |
@@ -550,7 +571,8 @@ __device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t
 // depend on S - T, Bm, e^gamma, e^(gamma_C - gamma), beta - for every chunk
 // of every request in parallel into a 9 KB record per (chunk, value head).
 // gdn_chunk_ext_kernel then carries S through a request's chunks, one
-// 512-thread workgroup per (request, value head) whose state wave w (0-3) owns
+// 512-thread workgroup per (request, value head) (few long requests: two,
+// gdn_cols_ext_kernel) whose state wave w (0-3) owns
 // state columns
 // 32 w .. + 31 as four 32 x 32 MFMA accumulator tiles (lane (g, n) = (lane /
 // 32, lane % 32): register r of tile ti is row 32 ti + 16 (r / 8) + 8 g + r % 8 of
@@ -1043,6 +1065,377 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_chunk_ext_kernel(GdnArgs a)
   }
 }
 
+// ---- the recurrence, two workgroups per (request, value head)
+constexpr int kColGroups = 2;                 // workgroups per value head
+constexpr int kCols = kDv / kColGroups;       // state columns per workgroup, 16 per state wave
+constexpr int kColBufs = 3;                   // chunk inputs in LDS: in use, landed, in flight
+
+// A chunk's inputs: q and k rows (512 B per token: 16-B chunks 0-15 high parts,
+// 16-31 low parts, chunk c of either half stored at c ^ (t & 15) of that half),
+// the workgroup's columns of v, and the record (T and Bm, split into operand
+// halves in place; then e^gamma, e^(gamma_C - gamma), beta).
+struct ColsIn {
+  uint32_t q[kChunk][128];
+  uint32_t k[kChunk][128];
+  uint16_t v[kChunk][kCols];
+  float rec[kRecBeta + kChunk];
+};
+struct ColsSmem {
+  ColsIn in[kColBufs];
+  uint16_t o[2][kChunk][kCols];   // output rows (o rounded to bf16) by chunk parity
+};
+static_assert(sizeof(ColsSmem) <= 160 * 1024, "LDS");
+
+// c + a b on 16 x 16 x 32 MFMAs, split operands as in mma3.
+__device__ __forceinline__ f32x4 mma3s(f32x4 c, const u32x4& ah, const u32x4& al, const u32x4& bh,
+                                       const u32x4& bl) {
+  c = mfma_16x16x32(al, bh, c);
+  c = mfma_16x16x32(ah, bl, c);
+  return mfma_16x16x32(ah, bh, c);
+}
+
+// As gdn_chunk_ext_kernel, for batches whose (request, value head) pairs leave
+// half of the CUs idle: two workgroups of 64 columns per pair, waves 0-3 with 16
+// columns each as eight 16 x 16 MFMA accumulator tiles (lane (g, n) = (lane / 16,
+// lane % 16): register r of tile 2 kk + u is row 32 kk + 8 g + 4 u + r of column n).
+// What bounds the pass is each wave's own chain from one chunk's state to the
+// next (K S0, T X and K^T Delta follow each other, with their operand splits and
+// LDS reads), so the fewer columns a wave has the shorter the chunk.  Waves 4-7,
+// the helpers, keep the inputs ahead: while the state waves work on chunk ci
+// they move chunk ci + 2 into LDS, split chunk ci + 1's T and Bm into operand
+// halves and write chunk ci - 1's output rows.  One barrier per chunk hands the
+// buffers over.  The gated norm needs whole rows: a launch of its own
+// (gdn_norm_ext_kernel).
+// One request of 1900 tokens, 48 value heads: 120 us + 16 for the norm (171 with
+// whole heads); four of 2048, more workgroups than CUs: 290 us (186 whole).
+// Workgroups take (key head, value head of it, column group) items in turn so
+// that the items that read the same q and k rows run on one XCD (workgroup i
+// runs on XCD i % 8) and its L2 serves the rows to all of them.
+__global__ void __launch_bounds__(kChunkThreads) gdn_cols_ext_kernel(GdnArgs a) {
+  __shared__ __attribute__((aligned(16))) ColsSmem sm;
+  const int lane = threadIdx.x & (kWave - 1), wv = wave_id();
+  const bool helper = wv >= 4;
+  const int w = wv & 3;                            // wave within its group
+  const int ht = threadIdx.x & (kThreads - 1);     // thread within its group
+  const int g = lane >> 4, n = lane & 15;
+  const int per_key = a.vpk * kColGroups;          // items per (request, key head)
+  const int keys = a.multi[0] * a.hk;
+
+  for (int item = blockIdx.x;; item += gridDim.x) {
+    const int q8 = item >> 3;
+    const int key = q8 / per_key * 8 + (item & 7);
+    if (q8 / per_key * 8 >= keys) break;           // uniform over the workgroup
+    if (key >= keys) continue;
+    const int m = key / a.hk, hk = key - m * a.hk;
+    const int sub = q8 % per_key, h = hk * a.vpk + sub / kColGroups;
+    const int j0 = kCols * (sub % kColGroups);     // first state column
+    const int bi = a.multi[1 + m];
+    const int64_t r = a.req[bi];
+    const int t0 = clamp_row(a, bi), t1 = max(clamp_row(a, bi + 1), t0);
+    const int last = t1 - 1;
+    const int nchunks = (t1 - t0 + kChunk - 1) / kChunk;
+
+    __syncthreads();   // the previous item's buffers are free
+    if (!helper) {
+      float* S = a.ssm + r * a.ssm_ss + (int64_t)h * kDk * kDv + 8 * g * kDv + j0 + 16 * w + n;
+      f32x4 st[8];
+#pragma unroll
+      for (int ti = 0; ti < 8; ++ti)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[ti][e] = S[(32 * (ti >> 1) + 4 * (ti & 1) + e) * kDv];
+      int buf = 0;
+      for (int ci = 0; ci < nchunks; ++ci) {
+        const ColsIn& I = sm.in[buf];
+        buf = buf == kColBufs - 1 ? 0 : buf + 1;
+        __syncthreads();   // chunk ci is in; its output rows' buffer is free
+        // P = K S0 and R = Q S0, k index 8 g + jj <-> state row 32 kk + 8 g + jj:
+        // a lane's operand is one 16-byte chunk of row t (8-byte pieces took the
+        // LDS three times as long).  Four chains (P and R, two m-tiles) take
+        // turns, so that a product never waits for the one before it, and step
+        // kk + 1's operands are read and its state operand split while step kk's
+        // MFMAs run.
+        auto rows_op = [&](const uint32_t (*rows)[128], int mt, int kk, u32x4 (&o)[2])
+                           __attribute__((always_inline)) {
+          const uint32_t* row = rows[16 * mt + n] + 4 * ((4 * kk + g) ^ n);   // t & 15 == n
+          o[0] = *reinterpret_cast<const u32x4*>(row);
+          o[1] = *reinterpret_cast<const u32x4*>(row + 64);
+        };
+        u32x4 op[2][4][2];   // [step parity][k m-tile 0, 1, q m-tile 0, 1][high, low]
+        auto read_ops = [&](int kk) __attribute__((always_inline)) {
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) {
+            rows_op(I.k, mt, kk, op[kk & 1][mt]);
+            rows_op(I.q, mt, kk, op[kk & 1][2 + mt]);
+          }
+        };
+        u32x4 sh[2], sl[2];
+        f32x4 PR[4] = {};
+        read_ops(0);
+        split8(st[0], st[1], sh[0], sl[0]);
+        f32x4 ec[2], dd[2], be[2], vv[2];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          if (kk + 1 < 4) {
+            read_ops(kk + 1);
+          } else {
+            // what X needs beside P
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+              const int t = 16 * mt + 4 * g;
+              ec[mt] = *reinterpret_cast<const f32x4*>(&I.rec[kRecC + t]);
+              dd[mt] = *reinterpret_cast<const f32x4*>(&I.rec[kRecD + t]);
+              be[mt] = *reinterpret_cast<const f32x4*>(&I.rec[kRecBeta + t]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) vv[mt][e] = bf(I.v[t + e][16 * w + n]);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          const u32x4(&o)[4][2] = op[kk & 1];
+          const u32x4 hi = sh[kk & 1], lo = sl[kk & 1];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) PR[c] = mfma_16x16x32(o[c][1], hi, PR[c]);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) PR[c] = mfma_16x16x32(o[c][0], lo, PR[c]);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) PR[c] = mfma_16x16x32(o[c][0], hi, PR[c]);
+          if (kk + 1 < 4) split8(st[2 * kk + 2], st[2 * kk + 3], sh[(kk + 1) & 1], sl[(kk + 1) & 1]);
+#pragma unroll
+          for (int q = 0; q < 12; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // 1 MFMA
+            __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);   // 2 VALU
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // A operand of the state update: the rows of K^T that tile ti = 2 kk + u
+        // holds at the tokens of Delta's k index, read from the token-major k rows
+        // with ds_read_b64_tr_b16, which hands lane i of each 16-lane group element
+        // i % 4 of the 8 bytes addressed by lane 4 k + (i % 16) / 4 as its element
+        // k: lane (g, L) addresses token 4 g + L / 4 (+ 16), dims 32 kk + 8 (L % 4)
+        // + 4 u .. + 3.  Four tiles at a time, the first four read under X.
+        const int ta = 4 * g + (n >> 2), tb = ta + 16;   // tb & 15 == ta & 15
+        const uint32_t* ka = I.k[ta];
+        const uint32_t* kb = I.k[tb];
+        auto read_kt = [&](int ti, u32x4 (&o)[2]) __attribute__((always_inline)) {
+          auto tr = [](const uint32_t* p) __attribute__((always_inline)) {
+            return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                 (lds_i16x4*)(const_cast<uint32_t*>(p))));
+          };
+          const int p = 4 * ((4 * (ti >> 1) + (n & 3)) ^ (ta & 15)) + 2 * (ti & 1);
+          const u32x2 h0 = tr(ka + p), h1 = tr(kb + p), l0 = tr(ka + p + 64), l1 = tr(kb + p + 64);
+          o[0] = u32x4{h0[0], h0[1], h1[0], h1[1]};
+          o[1] = u32x4{l0[0], l0[1], l1[0], l1[1]};
+        };
+        u32x4 kt[2][4][2], tp[2][2];
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          const u32x4* t4 =
+              reinterpret_cast<const u32x4*>(&I.rec[kRecT + (16 * mt + n) * kChunk + 8 * g]);
+          tp[mt][0] = t4[0];
+          tp[mt][1] = t4[1];
+        }
+#pragma unroll
+        for (int ti = 0; ti < 4; ++ti) read_kt(ti, kt[0][ti]);
+        const float cC = I.rec[kRecC + kChunk - 1];
+        // X = beta (v - e^gamma P); Delta = T X (k index 8 g + jj <-> token
+        // 16 (jj / 4) + 4 g + jj % 4)
+        f32x4 X[2], D[2] = {};
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) X[mt][e] = be[mt][e] * (vv[mt][e] - ec[mt][e] * PR[mt][e]);
+        u32x4 xh, xl;
+        split8(X[0], X[1], xh, xl);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) D[mt] = mfma_16x16x32(tp[mt][1], xh, D[mt]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) D[mt] = mfma_16x16x32(tp[mt][0], xl, D[mt]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) D[mt] = mfma_16x16x32(tp[mt][0], xh, D[mt]);
+#pragma unroll
+        for (int ti = 0; ti < 8; ++ti) st[ti] *= cC;
+        // S = e^(gamma_C) S0 + K^T (diag(e^(gamma_C - gamma)) Delta)
+        u32x4 dh, dl, eh, el;
+        split8(D[0] * dd[0], D[1] * dd[1], eh, el);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          if (half == 0) {
+#pragma unroll
+            for (int ti = 0; ti < 4; ++ti) read_kt(4 + ti, kt[1][ti]);
+          }
+#pragma unroll
+          for (int ti = 0; ti < 4; ++ti)
+            st[4 * half + ti] = mfma_16x16x32(kt[half][ti][1], eh, st[4 * half + ti]);
+#pragma unroll
+          for (int ti = 0; ti < 4; ++ti)
+            st[4 * half + ti] = mfma_16x16x32(kt[half][ti][0], el, st[4 * half + ti]);
+#pragma unroll
+          for (int ti = 0; ti < 4; ++ti)
+            st[4 * half + ti] = mfma_16x16x32(kt[half][ti][0], eh, st[4 * half + ti]);
+          if (half == 0) split8(D[0], D[1], dh, dl);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // O = e^gamma R + Bm Delta -> the output rows of this chunk
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          const u32x4* bp = reinterpret_cast<const u32x4*>(&I.rec[kRecB + (16 * mt + n) * kChunk + 8 * g]);
+          const f32x4 O = mma3s(f32x4{}, bp[0], bp[1], dh, dl);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sm.o[ci & 1][16 * mt + 4 * g + e][16 * w + n] =
+                to_bf(fmaf(ec[mt][e], PR[2 + mt][e], O[e]));   // .to(orig_dtype)
+        }
+      }
+      __syncthreads();   // the last chunk's output rows are in
+#pragma unroll
+      for (int ti = 0; ti < 8; ++ti)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[(32 * (ti >> 1) + 4 * (ti & 1) + e) * kDv] = st[ti][e];
+    } else {
+      const int key0 = chunk_key(a, bi);
+      // Chunk ci into its buffer (tokens past the last one re-read the last
+      // token; the record gives them beta = 0 and g = 0).  Helper wave w moves q
+      // and k rows 8 w .. 8 w + 7 (4 + 4 instructions, two rows each), v rows
+      // 8 w .. + 7 (1) and 2 KB of T and Bm (2); wave 2 the rest of the record.
+      const uint8_t* qk_base = reinterpret_cast<const uint8_t*>(a.wqk) + (int64_t)hk * 1024;
+      const uint8_t* v_base = reinterpret_cast<const uint8_t*>(a.ws) +
+                              ((int64_t)2 * a.key_dim + h * kDv + j0) * 2;
+      const uint8_t* rec_base = reinterpret_cast<const uint8_t*>(a.wrec) + (int64_t)h * kRec * 4;
+      auto issue = [&](int ci, int buf) __attribute__((always_inline)) {
+        const int tb = t0 + kChunk * ci;
+        ColsIn& I = sm.in[buf];
+        const int l5 = lane & 31;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const int t = 8 * w + 2 * p + (lane >> 5);
+          const uint32_t row = (uint32_t)min(tb + t, last) * (uint32_t)a.hk * 1024u;
+          const uint32_t cpos = (uint32_t)((l5 & 16) | ((l5 & 15) ^ (t & 15))) * 16u;
+          dma16(qk_base, row + cpos, lds_addr(&I.q[8 * w + 2 * p][0]));
+          dma16(qk_base, row + 512u + cpos, lds_addr(&I.k[8 * w + 2 * p][0]));
+        }
+        const uint32_t rec = (uint32_t)(key0 + ci) * (uint32_t)a.hv * (uint32_t)(kRec * 4);
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          dma16(rec_base, rec + 1024u * (2 * w + p) + 16u * lane,
+                lds_addr(&I.rec[256 * (2 * w + p)]));
+        dma16(v_base,
+              (uint32_t)min(tb + 8 * w + (lane >> 3), last) * (uint32_t)a.conv_dim * 2u +
+                  16u * (lane & 7),
+              lds_addr(&I.v[8 * w][0]));
+        if (w == 2 && lane < 3 * kChunk / 4)
+          dma16(rec_base, rec + 4u * kRecC + 16u * lane, lds_addr(&I.rec[kRecC]));
+      };
+      // The chunk issued before the newest one has landed: only the newest
+      // one's loads (11 per wave, 12 in wave 2; loads return in order) may be in
+      // flight.
+      auto wait_older = [&]() __attribute__((always_inline)) {
+        if (w == 2)
+          asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
+      };
+      // T and Bm of a chunk (fp32 rows of 32) split in place into the state
+      // waves' MFMA operand halves: row floats become, for g = 0 .. 3, the bf16
+      // high parts of columns 4 g + {0..3}, 16 + 4 g + {0..3} (16 bytes) and then
+      // the bf16 roundings of their remainders (16 bytes).  Lane l of helper wave
+      // w takes row 16 w + l / 4 (of T, then Bm), g = l % 4: rows of the 2 KB that
+      // this wave's own DMA brought in, so its vmcnt wait covers them; a wave's
+      // reads precede its writes.
+      auto split_tb = [&](int buf) __attribute__((always_inline)) {
+        static_assert(kRecT == 0 && kRecB == kChunk * kChunk && kRecC == 2 * kChunk * kChunk,
+                      "record layout");
+        float* row = &sm.in[buf].rec[kChunk * (16 * w + (lane >> 2))];
+        const int gg = lane & 3;
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(row + 4 * gg);
+        const f32x4 x1 = *reinterpret_cast<const f32x4*>(row + 16 + 4 * gg);
+        u32x4 hi, lo;
+        split8(x0, x1, hi, lo);
+        wave_lds_sync();
+        u32x4* out = reinterpret_cast<u32x4*>(row) + 2 * gg;
+        out[0] = hi;
+        out[1] = lo;
+      };
+      // Output rows of chunk cj: helper thread (token, part) = (ht / 8, ht % 8)
+      // moves 8 columns.
+      auto write_rows = [&](int cj) __attribute__((always_inline)) {
+        const int te = ht >> 3, c = 8 * (ht & 7), row = t0 + kChunk * cj + te;
+        if (row > last) return;   // padding of the request's last chunk
+        const u32x4 o = *reinterpret_cast<const u32x4*>(&sm.o[cj & 1][te][c]);
+        const int col = h * kDv + j0 + c;
+        u32x2* dst = reinterpret_cast<u32x2*>(a.out + (int64_t)row * a.out_rs + col);
+        dst[0] = u32x2{o[0], o[1]};
+        dst[1] = u32x2{o[2], o[3]};
+        if (a.core) {
+          u32x2* cd = reinterpret_cast<u32x2*>(a.core + (int64_t)row * a.core_rs + col);
+          cd[0] = u32x2{o[0], o[1]};
+          cd[1] = u32x2{o[2], o[3]};
+        }
+      };
+
+      issue(0, 0);
+      if (nchunks > 1) {
+        issue(1, 1);
+        wait_older();
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      split_tb(0);
+      int buf = 0;   // chunk ci's
+      for (int ci = 0; ci < nchunks; ++ci) {
+        const int next = buf == kColBufs - 1 ? 0 : buf + 1;
+        __syncthreads();   // the state waves start chunk ci and are done with chunk ci - 1
+        const bool more = ci + 2 < nchunks;
+        if (ci > 0) write_rows(ci - 1);
+        if (more) issue(ci + 2, next == kColBufs - 1 ? 0 : next + 1);
+        if (ci + 1 < nchunks) {
+          if (more)
+            wait_older();
+          else
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          split_tb(next);
+        }
+        buf = next;
+      }
+      __syncthreads();   // the last chunk's output rows are in
+      write_rows(nchunks - 1);
+    }
+  }
+}
+
+// The gated RMSNorm (rms_norm_gated.py:26-40) of the rows of requests with two
+// or more tokens, in place on the recurrence outputs: a half-wave per (row,
+// value head), 4 dims per lane; out = bf16(norm_w * (o / rms(o)) * silu(z)) with
+// silu(z) = z / (1 + e^-z) from the hardware exp2 and reciprocal (about 1 ulp each
+// in fp32, below the bf16 rounding of the output).  HBM-bound: o and z read, out
+// written.
+__global__ void __launch_bounds__(kThreads) gdn_norm_ext_kernel(GdnArgs a) {
+  const int row = blockIdx.x;
+  const int bi = a.owner[row];
+  if (bi < 0 || clamp_row(a, bi + 1) - clamp_row(a, bi) < 2) return;
+  const int d = 4 * (threadIdx.x & 31);
+  for (int h = threadIdx.x >> 5; h < a.hv; h += kThreads / 32) {
+    uint16_t* orow = a.out + (int64_t)row * a.out_rs + h * kDv + d;
+    const u32x2 ob = *reinterpret_cast<const u32x2*>(orow);
+    const u32x2 zb = __builtin_nontemporal_load(
+        reinterpret_cast<const u32x2*>(a.z + (int64_t)row * a.z_rs + h * kDv + d));
+    const f32x4 wn = *reinterpret_cast<const f32x4*>(a.norm_w + h * kDv + d);
+    const float o[4] = {bf16_lo(ob[0]), bf16_hi(ob[0]), bf16_lo(ob[1]), bf16_hi(ob[1])};
+    const float z[4] = {bf16_lo(zb[0]), bf16_hi(zb[0]), bf16_lo(zb[1]), bf16_hi(zb[1])};
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ss = fmaf(o[k], o[k], ss);
+#pragma unroll
+    for (int x = 16; x >= 1; x >>= 1) ss += __shfl_xor(ss, x, kWave);
+    const float inv = rsqrtf(ss / (float)kDv + a.eps);
+    float y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      y[k] = wn[k] * (o[k] * inv) *
+             (z[k] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-z[k] * kLog2e)));
+    *reinterpret_cast<u32x2*>(orow) = u32x2{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
+  }
+}
+
 // ---------------------------------------------------------------- other head dims
 // Head dims other than 128 (the reference's own test models use 16): one wave
 // per (request, value head) carries the head's dk x dv state in registers,
@@ -1185,6 +1578,22 @@ int64_t gdn_ext_ws_bytes(int64_t n_tokens, int32_t batch, int32_t hk, int32_t hv
 
 namespace {
 
+// Whether the state pass of an extend runs two workgroups per (request, value
+// head): where the prompts (at least ceil((n_tokens - batch) / (max_len - 1)), their
+// number if they are equally long) then still have a CU each, and the longest
+// chain saves (27 ns a token) more than the separate norm launch costs (3 us and
+// 8 ns a token, and 1.5 us for good measure).  The whole call, 48 value heads,
+// whole heads and split: one prompt of 256 tokens 69.8 and 67.4 us, 512 93.9 and
+// 87.0, 2000 237.6 and 198.4; two of 1000 167.8 and 158.8, of 256 83.8 and 85.7.
+// (Either kernel takes any batch; the offsets on the device decide what is done.)
+bool split_columns(int64_t n_tokens, int32_t batch, int32_t max_len, int32_t hv) {
+  if (27LL * max_len < 4500 + 8 * n_tokens || (int64_t)batch + 1 > (int64_t)hv * tfa::kRec)
+    return false;
+  const int64_t extra = std::max<int64_t>(n_tokens - batch, 1);
+  const int64_t prompts = (extra + max_len - 2) / (max_len - 1);
+  return prompts * hv * tfa::kColGroups <= tfa::device_cu_count();
+}
+
 // Validates the arguments shared by the decode and extend entry points and
 // fills the kernel arguments; rows = tokens (extend) or requests (decode).
 int32_t gdn_setup(const char* fn, const void* qkv, int64_t qkv_row_stride, const void* a,
@@ -1262,6 +1671,7 @@ int32_t gdn_setup(const char* fn, const void* qkv, int64_t qkv_row_stride, const
   g->owner = nullptr;
   g->silu_tab = nullptr;
   g->wrec = nullptr;
+  g->multi = nullptr;
   g->ws = static_cast<uint16_t*>(workspace);
   g->out = static_cast<uint16_t*>(out);
   g->out_rs = out_row_stride;
@@ -1447,9 +1857,13 @@ int32_t tf_gdn_extend(const void* qkv, int64_t qkv_row_stride, const void* a, co
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const uint32_t cblocks = (g.conv_dim + kThreads - 1) / kThreads;
   const uint32_t tblocks = (uint32_t)((n_tokens + kConvTokens - 1) / kConvTokens);
+  // The list of multi-token requests lives in the last record slot, which no
+  // chunk uses.
+  if (g.dk == kDk && split_columns(n_tokens, batch_size, max_extend_len, num_v_heads))
+    g.multi = reinterpret_cast<int32_t*>(g.wrec + (n_slots_rec - 1) * num_v_heads * kRec);
   hipLaunchKernelGGL(gdn_owner_kernel,
                      dim3((uint32_t)((std::max<int64_t>(n_tokens, kSiluTab) + kThreads - 1) /
-                                     kThreads)),
+                                     kThreads) + (g.multi ? 1 : 0)),
                      dim3(kThreads), 0, s, g);
   hipLaunchKernelGGL(gdn_conv_ext_kernel,
                      dim3((g.conv_dim / kConvCh + kThreads - 1) / kThreads,
@@ -1503,8 +1917,17 @@ int32_t tf_gdn_extend(const void* qkv, int64_t qkv_row_stride, const void* a, co
     const hipError_t e = hipEventRecord(lane->join, rs);
     if (e != hipSuccess) return side_failure("join event", e);
   }
-  hipLaunchKernelGGL(gdn_chunk_ext_kernel, dim3((int64_t)batch_size * num_v_heads),
-                     dim3(kChunkThreads), 0, s, g);
+  if (g.multi) {
+    const int64_t keys = std::min<int64_t>(batch_size, n_tokens / 2) * num_k_heads;
+    const int64_t items = (keys + 7) / 8 * 8 * g.vpk * kColGroups;
+    const int64_t cap = std::max(device_cu_count() / 8 * 8, 8);
+    hipLaunchKernelGGL(gdn_cols_ext_kernel, dim3((uint32_t)std::min(items, cap)),
+                       dim3(kChunkThreads), 0, s, g);
+    hipLaunchKernelGGL(gdn_norm_ext_kernel, dim3((uint32_t)n_tokens), dim3(kThreads), 0, s, g);
+  } else {
+    hipLaunchKernelGGL(gdn_chunk_ext_kernel, dim3((int64_t)batch_size * num_v_heads),
+                       dim3(kChunkThreads), 0, s, g);
+  }
   if (lane) {
     const hipError_t e = hipStreamWaitEvent(s, lane->join, 0);
     if (e != hipSuccess) return side_failure("join with the side stream", e);
