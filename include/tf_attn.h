@@ -308,8 +308,10 @@ int32_t tf_attn_rows(
  * ({b, kv head, row0, q_start, ext, first 32-key tile, end tile, 1 + partial slot};
  * at most one piece per compute unit), for tf_attn_extend_split with the merge
  * entries [n_merges][8], padded with zeros; n_pieces >= the compute units,
- * n_merges >= half of them, and seq_lens, seq_len_override and rtt_cols are the
- * launch's.
+ * n_merges >= half of them, seq_lens, seq_len_override and rtt_cols are the
+ * launch's, and key_bytes is the size of a token's K and V in the pool (what the
+ * step's streaming rows, given as dec_items also where n_blocks is 0, will read
+ * counts against a split).
  */
 int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* dec_items,
                             const int32_t* dec_rows, int32_t n_dec, int32_t num_q_heads,
@@ -317,7 +319,7 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
                             int32_t* blocks, int32_t n_blocks, int32_t* pieces,
                             int32_t n_pieces, int32_t* merges, int32_t n_merges,
                             const int64_t* seq_lens, int32_t seq_len_override,
-                            int64_t rtt_cols, tf_stream_t stream);
+                            int64_t rtt_cols, int32_t key_bytes, tf_stream_t stream);
 
 /* tf_attn_extend_split: tf_attn_extend (head_dim 256) over the pieces and merge
  * entries of tf_attn_plan_blocks.  workspace: 16-byte aligned scratch of

@@ -49,7 +49,10 @@ def expected(wl, cus):
     mx, length = max(tiles), 0
     if len(work) <= cus and mx >= 24:
         n = next(n for n in range(12, mx + 1) if count(n) <= cus)
-        if n + 24 + 3 + 0.047 * count(n) < 0.92 * (mx + 15):
+        # the decode rows' time in tiles: the split has to win with them after it
+        rows = sum(l for l, e in zip(wl.seq_lens, wl.ext_lens) if e * group <= 64)
+        rows *= 2 * wl.num_kv_heads * 256 * wl.k_pool.element_size() / 9e6
+        if n + 24 + 3 + 0.047 * count(n) + rows < 0.92 * max(mx + 15, rows):
             length = n
     pieces, merges, slot = [], [], 0
     for w, t in zip(work, tiles):
@@ -66,7 +69,8 @@ def expected(wl, cus):
 @pytest.mark.parametrize("seq,ext", [
     ([3000], [100]), ([6100, 1700, 5300], [211, 37, 100]), ([5000], [2000]),
     ([900, 400], [12, 11]), ([4000, 50, 2000], [700, 50, 1]), ([20000], [11]),
-    ([1500] * 20, [200] * 20)])
+    ([1500] * 20, [200] * 20), ([3000] + [2000] * 80, [260] + [1] * 80),
+    ([6000] + [2000] * 20 + [500], [260] + [1] * 20 + [4])])
 @pytest.mark.parametrize("device_plan", [False, True])
 def test_plan(gpu, seq, ext, device_plan):
     wl = case(gpu, seq, ext, seed=len(seq))

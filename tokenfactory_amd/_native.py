@@ -99,7 +99,7 @@ SIGNATURES = {
         _p, _i32, _p, _p, _i32,        # work, n_work, dec_items, dec_rows, n_dec
         _i32, _i32, _i32, _i64,        # heads, row_groups, max_rows
         _p, _i32, _p, _i32, _p, _i32,  # blocks, n_blocks, pieces, n_pieces, merges, n_merges
-        _p, _i32, _i64, _p,            # seq_lens, seq_len_override, rtt_cols, stream
+        _p, _i32, _i64, _i32, _p,      # seq_lens, seq_len_override, rtt_cols, key_bytes, stream
     ]),
     "tf_attn_extend_split": (_i32, [
         _p, _i64,

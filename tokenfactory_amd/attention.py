@@ -28,6 +28,7 @@ import numpy as np
 import torch
 
 from . import _native
+from .fp8_linear import on_stream
 from .planning import EXTEND_TILE_ROWS, plan_decode_items, plan_extend
 
 _KV_DTYPES = {
@@ -190,7 +191,7 @@ class Route:
     captured or reused call's), so launches without work can be left out."""
 
     __slots__ = ("row_groups", "max_rows", "n_blocks", "n_pieces", "n_merges", "split",
-                 "run_extend", "run_rows")
+                 "run_extend", "run_rows", "key_bytes")
 
     def __init__(self, ext_lens, n_tok, n_q, n_kv, head_dim, kv_dtype, n_work, exact,
                  max_len=0, cus=0):
@@ -200,6 +201,7 @@ class Route:
         self.max_rows = SHORT_ROWS
         self.run_extend = self.run_rows = True
         fp8 = kv_dtype == _native.TF_DTYPE_FP8_E4M3
+        self.key_bytes = 2 * n_kv * head_dim * (1 if fp8 else 2)
         if head_dim != 256:
             if fp8 and head_dim % 16:
                 return
@@ -244,14 +246,13 @@ class Route:
         pieces = base + 16 * self.n_blocks
         rows_too = self.row_groups > 0
         _native.call("tf_attn_plan_blocks", work if n_work else None, n_work,
-                     _ptr(items) if rows_too else None, _ptr(rows) if rows_too else None,
-                     n_dec if rows_too else 0, n_q, n_kv, max(self.row_groups, 1),
+                     _ptr(items), _ptr(rows), n_dec, n_q, n_kv, max(self.row_groups, 1),
                      self.max_rows if rows_too else 0, base if self.n_blocks else None,
                      self.n_blocks, pieces if self.n_pieces else None, self.n_pieces,
                      pieces + 32 * self.n_pieces if self.split else None, self.n_merges,
                      batch.seq_lens.data_ptr(),
                      int(batch.max_seq_len) if batch.batch_size == 1 else 0,
-                     batch.req_to_token.shape[1], stream.cuda_stream)
+                     batch.req_to_token.shape[1], self.key_bytes, stream.cuda_stream)
 
 
 class StepPlan:
@@ -660,7 +661,7 @@ class SlotAttentionCall:
                 n_work = self.route.n_pieces
             if self.route.split:
                 # (allocated on the launch's stream, which orders its reuse)
-                with torch.cuda.stream(self.stream):
+                with on_stream(self._fixed_stream):
                     ws = torch.empty(_native.load().tf_attn_extend_split_workspace_bytes(),
                                      dtype=torch.uint8, device=self.q.device)
                 _native.call("tf_attn_extend_split", self.q.data_ptr(), self.q.stride(0),

@@ -217,6 +217,7 @@ struct BlockArgs {
   const int64_t* seq_lens;
   int32_t seq_override;
   int64_t rtt_cols;
+  int32_t key_bytes;      // K and V of one token
   int32_t cus;
 };
 
@@ -228,7 +229,11 @@ struct BlockArgs {
 // tiles + 15 (Q, first slots, output), a piece its tiles + 24 (it also writes
 // 256 KB of partials), the merge 3 + 0.047 per piece.  The shortest piece
 // length that gives no more pieces than CUs is taken when it beats the whole
-// entries by 8 %; short contexts (below about 900 keys) never do.  Measured
+// entries by 8 %; short contexts (below about 900 keys) never do.  The step's
+// streaming rows (decodes, short extends) run beside whole entries, on the CUs
+// these leave, but after pieces that take every CU: their keys' time at 6 TB/s
+// counts in full against the split (86 decodes on 100 to 4k keys beside 2 prompts
+// of 260 tokens on 1k to 3k: 175 us whole, 203 split).  Measured
 // (24 / 4 heads): 3 requests of 37 to 211 new tokens on 1.5k to 6k keys, 36
 // entries of up to 180 tiles: 252 us whole, 48 + 14 (merge) in 252 pieces.  One
 // of 2000 tokens on 3000, 188 entries of 95 to 156 tiles, stays whole (the plan
@@ -243,17 +248,22 @@ struct SplitSmem {
   int32_t piece;              // tiles per piece (0: no split)
 };
 
+__device__ __forceinline__ int64_t context_len(const BlockArgs& a, int b) {
+  const int64_t len = a.seq_override > 0 ? (int64_t)a.seq_override : a.seq_lens[b];
+  return min(max(len, (int64_t)0), a.rtt_cols);
+}
+
 // Tiles of 32 keys that the entry's rows see.
 __device__ __forceinline__ int entry_tiles(const BlockArgs& a, const int32_t* wk) {
-  int64_t len = a.seq_override > 0 ? (int64_t)a.seq_override : a.seq_lens[wk[0]];
-  if (len > a.rtt_cols) len = a.rtt_cols;
+  const int64_t len = context_len(a, wk[0]);
   const int64_t last = min<int64_t>((int64_t)wk[2] + kExtendItemRows, (int64_t)wk[4] * a.group) - 1;
   const int64_t kend = min(len, len - wk[4] + last / a.group + 1);
   return kend > 0 ? (int)((kend + 31) / 32) : 0;
 }
 
 // Tiles per piece for n entries, by wave 0 (every lane gets it; 0: no split).
-__device__ int piece_tiles(const SplitSmem& sm, int n, int cus) {
+// rows: the streaming rows' time, in tiles.
+__device__ int piece_tiles(const SplitSmem& sm, int n, int cus, float rows) {
   const int lane = threadIdx.x & (kWave - 1);
   auto wave_sum = [&](int v) {
 #pragma unroll
@@ -279,8 +289,8 @@ __device__ int piece_tiles(const SplitSmem& sm, int n, int cus) {
     const int mid = (lo + hi) >> 1;
     if (pieces(mid) <= cus) hi = mid; else lo = mid + 1;
   }
-  const float split = (float)hi + kPieceCost + kMergeCost + kMergePiece * (float)pieces(hi);
-  return split < 0.92f * ((float)mx + kEntryCost) ? hi : 0;
+  const float split = (float)hi + kPieceCost + kMergeCost + kMergePiece * (float)pieces(hi) + rows;
+  return split < 0.92f * fmaxf((float)mx + kEntryCost, rows) ? hi : 0;
 }
 
 __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
@@ -289,6 +299,7 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
   const int tid = threadIdx.x;
   const int R = a.unit_rows, G = a.group;
   int64_t at = 0;   // blocks so far
+  int64_t keys = 0;   // of the streaming rows
   auto emit = [&](int n, int64_t i0, const RowItem& first) {
     for (int k = 0; k < n; ++k)
       if (i0 + k < a.n_blocks)
@@ -306,6 +317,10 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
     const int64_t before = block_scan(n, wsum, total);
     emit(n, at + before, it);
     at += total;
+    if (a.merges) {
+      (void)block_scan(it.b < 0 ? 0 : context_len(a, it.b), wsum, total);
+      keys += total;
+    }
   }
   int64_t kept = 0;   // pieces so far
   for (int base = 0; base < a.n_work; base += kPlanThreads) {
@@ -324,6 +339,11 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
     const int64_t before = block_scan(n, wsum, total);
     emit(n, at + before, it);
     at += total;
+    if (a.merges) {
+      const bool first = n > 0 && wk[2] == 0;
+      (void)block_scan(first ? context_len(a, wk[0]) : 0, wsum, total);
+      keys += total;
+    }
     const bool keep = rows > 0 && !to_blocks;
     int64_t n_keep;
     const int64_t k0 = kept + block_scan(keep ? 1 : 0, wsum, n_keep);
@@ -341,7 +361,8 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
   if (a.merges && kept <= kSplitMax) {
     __syncthreads();
     if (tid < kWave) {
-      const int len = piece_tiles(sm, (int)kept, a.cus);
+      // a tile takes about 1.5 us, 9 MB at 6 TB/s
+      const int len = piece_tiles(sm, (int)kept, a.cus, (float)keys * (float)a.key_bytes / 9e6f);
       if (tid == 0) sm.piece = len;
     }
     __syncthreads();
@@ -549,7 +570,7 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
                             int32_t* blocks, int32_t n_blocks, int32_t* pieces,
                             int32_t n_pieces, int32_t* merges, int32_t n_merges,
                             const int64_t* seq_lens, int32_t seq_len_override,
-                            int64_t rtt_cols, tf_stream_t stream) {
+                            int64_t rtt_cols, int32_t key_bytes, tf_stream_t stream) {
   using namespace tfa;
   clear_error();
   if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads)
@@ -562,7 +583,7 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
       !aligned16(merges) || n_merges < 0)
     return fail(TF_ERR_INVALID, "plan_blocks: null or misaligned pointer or negative count");
   const int32_t cus = device_cu_count();
-  if (merges && (n_pieces < cus || n_merges < cus / 2 || rtt_cols < 1 ||
+  if (merges && (n_pieces < cus || n_merges < cus / 2 || rtt_cols < 1 || key_bytes < 0 ||
                  (!seq_lens && seq_len_override <= 0)))
     return fail(TF_ERR_INVALID, "plan_blocks: a split needs the lengths and room for %d pieces "
                 "and %d merges", cus, cus / 2);
@@ -584,6 +605,7 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
   a.seq_lens = seq_lens;
   a.seq_override = seq_len_override;
   a.rtt_cols = rtt_cols;
+  a.key_bytes = key_bytes;
   a.cus = cus;
   hipLaunchKernelGGL(blocks_kernel, dim3(1), dim3(kPlanThreads), 0,
                      reinterpret_cast<hipStream_t>(stream), a);
