@@ -308,7 +308,8 @@ int32_t tf_attn_rows(
  * ({b, kv head, row0, q_start, ext, first 32-key tile, end tile, 1 + partial slot};
  * at most one piece per compute unit), for tf_attn_extend_split with the merge
  * entries [n_merges][8], padded with zeros; n_pieces >= the compute units,
- * n_merges >= half of them, seq_lens, seq_len_override and rtt_cols are the
+ * n_merges >= 1 (entries that it has no room for stay whole: the number of
+ * entries, or half of the compute units, is always enough), seq_lens, seq_len_override and rtt_cols are the
  * launch's, and key_bytes is the size of a token's K and V in the pool (what the
  * step's streaming rows, given as dec_items also where n_blocks is 0, will read
  * counts against a split).

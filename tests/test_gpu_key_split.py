@@ -162,3 +162,27 @@ def test_captured_split_step_replays(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert_attn_close(call.out, restatement(wl), what=f"replay {i}")
+
+
+def test_plan_without_room_for_merges_stays_whole(gpu):
+    """tf_attn_plan_blocks with fewer merge entries than the split needs."""
+    from tokenfactory_amd import _native
+    wl = case(gpu, [6100, 1700, 5300], [211, 37, 100], seed=3)
+    call = call_of(wl)
+    call.run_plan()
+    call._plan_lists()
+    _, merges = lists(call)
+    r, need = call.route, int((merges[:, 4] > 0).sum())
+    assert need > 1
+    for room in (need, need - 1):
+        got = torch.full((8 * (r.n_pieces + room),), -1, dtype=torch.int32, device=gpu)
+        _native.call("tf_attn_plan_blocks", call._meta.data_ptr(), call.n_work, None, None, 0,
+                     24, 4, 1, 0, None, 0, got.data_ptr(), r.n_pieces,
+                     got.data_ptr() + 32 * r.n_pieces, room, wl.batch.seq_lens.data_ptr(), 0,
+                     wl.batch.req_to_token.shape[1], r.key_bytes,
+                     torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        got = got.cpu().numpy()
+        cut = (got[:8 * r.n_pieces].reshape(-1, 8)[:, 7] > 0).sum()
+        assert (cut > 0) == (room == need)
+        assert (got[8 * r.n_pieces:].reshape(-1, 8)[:, 4] > 0).sum() == (need if cut else 0)

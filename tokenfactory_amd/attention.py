@@ -183,7 +183,14 @@ class Route:
     (``tf_attn_plan_blocks`` decides from the lengths on the device): ``split``
     says that it may, i.e. there is at most one entry per CU and a context of at
     least ``SPLIT_KEYS`` keys (a piece shorter than 12 tiles of 32 keys never
-    pays).
+    pays).  Where the plan then keeps the entries whole, the merge launch and the
+    kernel's other instance cost about 4 us (10 decodes beside a prompt of 440
+    tokens on 850: 73 and 77 us); of a mixed step the host knows only the longest
+    context of all, so the split is considered where what it can save if an extend
+    has that context (1.5 us per 32 keys beyond 768), times the extends' share of
+    the batch, exceeds that: L - 768 >= 86 batch / extends.  (7 decodes beside a
+    prompt of 300 on 5k: 255 us whole, 103 split; 75 beside one, contexts below
+    1.1k: 83 whole, 86 considered.)
 
     ``row_groups``: groups of 16 rows per unit, 0 = the streaming kernel takes no
     blocks.  ``n_blocks`` / ``n_pieces`` / ``n_merges``: capacities of the device
@@ -217,12 +224,14 @@ class Route:
             unit = 16 * self.row_groups
             self.n_blocks = bsz * max(-(-SHORT_ROWS // unit), -(-group // unit))
             self.n_pieces = n_work
-        long_entries = sum(n_kv * -(-e * group // EXTEND_TILE_ROWS) for e in ext_lens
-                           if e > 1 and e * group > SHORT_ROWS)
-        if n_work and 0 < long_entries <= cus and max_len >= SPLIT_KEYS:
+        long_ = [e for e in ext_lens if e > 1 and e * group > SHORT_ROWS]
+        long_entries = sum(n_kv * -(-e * group // EXTEND_TILE_ROWS) for e in long_)
+        if n_work and 0 < long_entries <= cus and max_len >= SPLIT_KEYS \
+                and len(long_) * (max_len - 768) >= 86 * bsz:
             self.split = True
             self.n_pieces = cus if exact else max(n_work, cus)
-            self.n_merges = cus // 2
+            # (an empty merge entry still costs its workgroups' launch)
+            self.n_merges = min(cus // 2, long_entries) if exact else cus // 2
         if exact:
             n_short, n_dec = len(short), sum(1 for e in ext_lens if e == 1)
             self.run_extend = n_short + n_dec < bsz

@@ -374,7 +374,8 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
       const int64_t p0 = block_scan(n, wsum, total);
       const int64_t s0 = block_scan(n > 1 ? n : 0, wsum, slots);
       const int64_t m0 = block_scan(n > 1 ? 1 : 0, wsum, n_merge);
-      if (tid < kept) {
+      // (more merges than the caller has room for: the entries stay whole)
+      if (n_merge <= a.n_merges && tid < kept) {
         int32_t wk[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) wk[q] = a.work[8 * (int64_t)sm.src[tid] + q];
@@ -386,7 +387,7 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
           pc[6] = n > 1 ? (int)((int64_t)t * (k + 1) / n) : 0;
           pc[7] = n > 1 ? (int32_t)(s0 + k + 1) : 0;
         }
-        if (n > 1 && m0 < a.n_merges) {
+        if (n > 1) {
           int32_t* mg = a.merges + 8 * m0;
 #pragma unroll
           for (int q = 0; q < 5; ++q) mg[q] = wk[q];
@@ -395,7 +396,10 @@ __global__ void __launch_bounds__(kPlanThreads) blocks_kernel(BlockArgs a) {
           mg[7] = 0;
         }
       }
-      kept = total;
+      if (n_merge <= a.n_merges)
+        kept = total;
+      else
+        n_merge = 0;
     }
   }
   if (a.merges)
@@ -583,10 +587,10 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
       !aligned16(merges) || n_merges < 0)
     return fail(TF_ERR_INVALID, "plan_blocks: null or misaligned pointer or negative count");
   const int32_t cus = device_cu_count();
-  if (merges && (n_pieces < cus || n_merges < cus / 2 || rtt_cols < 1 || key_bytes < 0 ||
+  if (merges && (n_pieces < cus || n_merges < 1 || rtt_cols < 1 || key_bytes < 0 ||
                  (!seq_lens && seq_len_override <= 0)))
     return fail(TF_ERR_INVALID, "plan_blocks: a split needs the lengths and room for %d pieces "
-                "and %d merges", cus, cus / 2);
+                "and 1 merge", cus);
   BlockArgs a;
   a.work = work;
   a.n_work = n_work;
