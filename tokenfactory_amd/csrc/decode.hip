@@ -987,10 +987,15 @@ int launch_rows(const DecodeArgs& a, const DecodePlan& p, int phases, hipStream_
   }
   if (phases & kPhaseMerge) {
     // kWaves waves per (unit, head) row when the units average more than
-    // three partials each, else one (measured: see decode_merge_kernel).  With
+    // three partials each, else one (measured: see decode_merge_kernel), and one
+    // where that would be more than two workgroups per CU (86 requests on a grid
+    // of 768, about three partials each: 11.2 us wide, 6.3 narrow).  With
     // many units most are not split: one workgroup per unit then, so that it
     // finds that out once.
-    const bool wide = (int64_t)p.n_blocks > 2 * p.n_units;
+    constexpr int kWideRows = kMergeWaves / kWaves;
+    const bool wide = (int64_t)p.n_blocks > 2 * p.n_units &&
+                      p.n_units * ((p.rows_used + kWideRows - 1) / kWideRows) <=
+                          2 * device_cu_count();
     const int per_wg = wide ? kMergeWaves / kWaves : kMergeWaves;
     const bool many = p.n_units >= 2 * p.n_blocks;
     const dim3 grid((unsigned)p.n_units, many ? 1u : (unsigned)((p.rows_used + per_wg - 1) / per_wg));
