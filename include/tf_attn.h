@@ -279,8 +279,9 @@ int32_t tf_attn_plan_device(const int64_t* extend_lens, int32_t batch_size,
  * the request's ext * G (row = t * G + h, token t sees keys up to
  * seq_lens[b] - ext + t); b = -1 is padding.  NULL: item i is request i with one
  * token at q row i (at most 2048), every head of it.  row_groups: 1 without
- * blocks; 1 or 2 (2 at head dims other than 256) with them.  The other arguments are tf_attn_decode's;
- * workspace: tf_attn_rows_workspace_bytes of the same sizes, 16-byte aligned.
+ * blocks; 1 or 2 (2 at head dims other than 256) with them.  The other arguments
+ * are tf_attn_decode's; workspace: tf_attn_rows_workspace_bytes of the same
+ * sizes, 16-byte aligned.
  */
 int64_t tf_attn_rows_workspace_bytes(int32_t has_blocks, int32_t n_items, int32_t row_groups,
                                      int32_t num_q_heads, int32_t num_kv_heads,

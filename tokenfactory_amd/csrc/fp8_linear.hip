@@ -23,9 +23,9 @@
 // SIMD) or 8 waves (256 columns x 256 or 192 rows, two slices in LDS, two waves
 // per SIMD), chosen with the split over K by gemm_plan.  One launch takes up to
 // four weight matrices of the same input (a layer's projections), so a narrow
-// matrix fills the rounds of a wide one.  Each MFMA starts from zero and its product is folded into the
-// fp32 accumulator with that block's scale, acc += p * s, one FMA per
-// accumulator element per 128 of K; a row's folds run between the next row's
+// matrix fills the rounds of a wide one.  Each MFMA starts from zero and its
+// product is folded into the fp32 accumulator with that block's scale,
+// acc += p * s, one FMA per accumulator element per 128 of K; a row's folds run between the next row's
 // MFMAs, and each row's operand is read from LDS two rows ahead.  Per
 // 128-wide K slice the workgroup stages the weight tile (64 WN rows), the
 // activation tile (32 MT rows) and the column scales straight from global
