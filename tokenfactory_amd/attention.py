@@ -41,7 +41,8 @@ _workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
 
 
 def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
-    """Decode split-partial scratch, one per (device, stream), grown on demand."""
+    """Decode split-partial scratch, one per (device, stream), grown on demand
+    (the caller makes ``stream`` current: the allocator orders reuse by it)."""
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     with _ws_lock:
         ws = _workspaces.get(key)
@@ -441,12 +442,14 @@ class SlotAttentionCall:
         if kv_dtype == _native.TF_DTYPE_FP8_E4M3:
             if k_scale is None or v_scale is None:
                 raise ValueError("an fp8 KV pool needs k_scale and v_scale")
-            k_scale = k_scale.to(device=q.device, dtype=torch.float32).reshape(1).contiguous()
-            v_scale = v_scale.to(device=q.device, dtype=torch.float32).reshape(1).contiguous()
+            with on_stream(stream):   # conversions run, and live, where they are read
+                k_scale = k_scale.to(device=q.device, dtype=torch.float32).reshape(1).contiguous()
+                v_scale = v_scale.to(device=q.device, dtype=torch.float32).reshape(1).contiguous()
         else:
             k_scale = v_scale = None
         if q.stride(2) != 1 or q.stride(1) != head_dim:
-            q = q.contiguous()
+            with on_stream(stream):
+                q = q.contiguous()
         if out is None:
             out = torch.empty((n_tok, n_q, head_dim), dtype=q.dtype, device=q.device)
         elif out.shape != q.shape or out.dtype != q.dtype or out.stride(2) != 1 \
@@ -530,8 +533,9 @@ class SlotAttentionCall:
             self.n_work = _native.plan_device_capacity(n_tok, bsz, n_q, n_kv)
             self.n_dec = bsz
             self._ext_t = ext_t
-            self._meta = torch.empty(self.n_work * 8 + 2 * bsz + 4, dtype=torch.int32,
-                                     device=q.device)
+            with on_stream(stream):
+                self._meta = torch.empty(self.n_work * 8 + 2 * bsz + 4, dtype=torch.int32,
+                                         device=q.device)
             base = self._meta.data_ptr() + 4 * self.n_work * 8
             self._items = _DevPtr(base)
             self._rows = _DevPtr(base + 4 * bsz)
@@ -562,7 +566,10 @@ class SlotAttentionCall:
                                exact=not self.device_plan, max_len=self.max_len,
                                cus=_cu_count(q.device))
             if self.route.planned and self.n_work:
-                self._lists = self.route.alloc(q.device)
+                # (allocated on the launches' stream, which writes and reads it: a
+                # dropped call's memory then goes back to that stream's pool)
+                with on_stream(stream):
+                    self._lists = self.route.alloc(q.device)
         if (self.decode_workgroups == 0 and self.n_work and self.n_dec and self.route.run_extend
                 and max(ext_lens) > 1 and min(ext_lens) == 1):
             # A mixed step's decode kernel runs beside the extend kernel, whose
@@ -585,7 +592,8 @@ class SlotAttentionCall:
             nbytes = _native.decode_workspace_bytes(self.n_dec, n_q, n_kv, head_dim,
                                                     self.max_len, self.decode_workgroups)
         if nbytes:
-            self.ws = _workspace(q.device, self._stream_handle, nbytes)
+            with on_stream(stream):
+                self.ws = _workspace(q.device, self._stream_handle, nbytes)
 
     @property
     def stream(self) -> torch.cuda.Stream:
