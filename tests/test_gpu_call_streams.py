@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from tests.helpers import small_case
-from tokenfactory_amd import workloads
+from tokenfactory_amd import slot_based_attention, workloads
 from tokenfactory_amd.attention import SlotAttentionCall
 
 pytestmark = pytest.mark.gpu
@@ -66,5 +66,31 @@ def test_inputs_converted_on_the_launch_stream(gpu):
     for ptr, n, dtype in spans:
         for _ in range(4):
             assert torch.empty(n, dtype=dtype, device=gpu).fill_(float("nan")).data_ptr() != ptr
+    s.synchronize()
+    assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("planned_by", ["other", "own"])
+def test_dropped_batch_leaves_no_memory_to_its_first_stream(gpu, planned_by):
+    """The step plan kept on a batch is read by every stream that calls with the
+    batch: its memory is not reused before the last of them is done."""
+    wl = small_case([900, 300, 3000], [4, 1, 100], hq=24, hkv=4, d=256, seed=7, device=gpu,
+                    dtype=torch.bfloat16)
+    run = lambda: slot_based_attention(wl.q, wl.k_pool, wl.v_pool, wl.batch, scaling=wl.scale)
+    want = run().clone()
+    plan, = wl.batch._tf_attn_step_plans.values()
+    if planned_by == "own":   # made on this stream, first planned and read by the other
+        plan._planned_on = plan._event = None
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(50_000_000)   # the stream is busy while the batch goes away
+        out = run()
+    spans = [(t.data_ptr(), t.numel()) for t in (plan.meta, plan.lists)]
+    del plan
+    wl.batch._tf_attn_step_plans.clear()
+    other = [torch.empty(n, dtype=torch.int32, device=gpu).fill_(77) for _, n in spans
+             for _ in range(4)]
+    assert not {t.data_ptr() for t in other} & {p for p, _ in spans}
     s.synchronize()
     assert torch.equal(out, want)

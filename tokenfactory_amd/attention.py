@@ -302,6 +302,7 @@ class StepPlan:
         self.status = _DevPtr(base + 8 * bsz)
         self.device = device
         self._lock = threading.Lock()
+        self._users = {_native.current_stream(device)}   # streams that own or have used the lists
         self._planned_on: Optional[torch.cuda.Stream] = None
         self._event: Optional[torch.cuda.Event] = None
 
@@ -309,6 +310,12 @@ class StepPlan:
         """Plan on ``stream`` if no call has yet; else order ``stream`` after
         the plan."""
         with self._lock:
+            if stream.cuda_stream not in self._users:
+                # (a batch dropped while this stream still reads them)
+                self._users.add(stream.cuda_stream)
+                for t in (self.meta, self.lists):
+                    if t is not None:
+                        t.record_stream(stream)
             if self._planned_on is None:
                 _native.call("tf_attn_plan_device", self.ext_t.data_ptr(), self.batch_size,
                              self.n_q, self.n_kv, 1, self.meta.data_ptr(), self.n_work,
