@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from tests.helpers import small_case
-from tokenfactory_amd import slot_based_attention, workloads
+from tokenfactory_amd import attention, slot_based_attention, workloads
 from tokenfactory_amd.attention import SlotAttentionCall
 
 pytestmark = pytest.mark.gpu
@@ -30,7 +30,7 @@ def test_dropped_call_leaves_no_memory_to_other_streams(gpu, seq, ext, d, device
     s.wait_stream(torch.cuda.current_stream())
     out = torch.empty_like(wl.q)
     call = calls(wl, device_plan=device_plan, stream=s, out=out)
-    held = {n: t for n, t in (("lists", call._lists), ("meta", call._meta), ("ws", call.ws))
+    held = {n: t for n, t in (("lists", call._lists), ("meta", call._meta), ("ws", call._scratch()))
             if t is not None}
     spans = {n: (t.data_ptr(), t.data_ptr() + t.numel() * t.element_size(), t.numel(), t.dtype)
              for n, t in held.items()}
@@ -94,3 +94,44 @@ def test_dropped_batch_leaves_no_memory_to_its_first_stream(gpu, planned_by):
     assert not {t.data_ptr() for t in other} & {p for p, _ in spans}
     s.synchronize()
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("kept", [False, True])
+@pytest.mark.parametrize("seq,ext,d", [([700, 900], [1, 1], 128), ([900, 1500], [4, 10], 256),
+                                       ([2000, 900], [1, 1], 256),
+                                       ([3000, 2000, 50], [100, 1, 1], 256)])   # overlapped
+def test_captured_call_owns_its_scratch(gpu, seq, ext, d, kept):
+    """Replays write neither the stream's shared scratch nor what became of it
+    after a later call on the same stream needed more."""
+    kw = dict(hq=24, hkv=4, d=d, dtype=torch.bfloat16, device=gpu)
+    wl = small_case(seq, ext, seed=d, **kw)
+    run = lambda: slot_based_attention(wl.q, wl.k_pool, wl.v_pool, wl.batch, scaling=wl.scale)
+    want = run().clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        call = calls(wl, device_plan=max(ext) > 1)
+        call.run()   # a warm-up on the capturing stream
+    s.synchronize()
+    with torch.cuda.graph(graph, stream=s):
+        out = call.run() if kept else run()
+    keep = call.ws if kept else None
+    key = (gpu.index, s.cuda_stream)
+    shared = attention._workspaces[key]
+    if kept:
+        assert keep.data_ptr() != shared.data_ptr()
+    shared.fill_(0x5a)
+    for i in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), f"replay {i}"
+        assert (shared == 0x5a).all(), f"replay {i} wrote the shared scratch"
+        with torch.cuda.stream(s):   # eager work on the stream, with more scratch
+            attention._workspace(gpu, s.cuda_stream, shared.numel() + (1 << 20))
+            calls(wl, decode_workgroups=600 + 100 * i).run()
+        torch.cuda.synchronize()
+        shared = attention._workspaces[key].fill_(0x5a)
+        torch.cuda.synchronize()

@@ -514,7 +514,9 @@ class SlotAttentionCall:
         self.route = None
         self._lists = None
         self._lists_planned = False   # of a host-planned call (its lengths are fixed)
-        self.ws = None
+        self.ws = None                # split scratch of the last launch
+        self._ws_bytes = 0
+        self._ws_stream = None        # whose shared scratch self.ws is (None: a graph's own)
         self._n_rows_items = 0   # items of the tf_attn_rows launch (0: tf_attn_decode)
         if n_tok == 0:
             return
@@ -598,9 +600,7 @@ class SlotAttentionCall:
         elif self.n_dec and self.route.run_rows:
             nbytes = _native.decode_workspace_bytes(self.n_dec, n_q, n_kv, head_dim,
                                                     self.max_len, self.decode_workgroups)
-        if nbytes:
-            with on_stream(stream):
-                self.ws = _workspace(q.device, self._stream_handle, nbytes)
+        self._ws_bytes = nbytes
 
     @property
     def stream(self) -> torch.cuda.Stream:
@@ -653,9 +653,27 @@ class SlotAttentionCall:
         n = self.n_work * 8 + 2 * self.n_dec
         return tuple(int(x) for x in self._meta[n:n + 3].cpu())
 
-    def _decode(self, entry: str, stream: Optional[torch.cuda.Stream] = None) -> None:
-        ws = self.ws
-        handle = stream.cuda_stream if stream is not None else self._stream_handle
+    def _scratch(self) -> Optional[torch.Tensor]:
+        """Split scratch of a launch: its stream's shared one, or, under graph
+        capture, one of its own from the graph's memory.  (The shared one is
+        replaced when a later call needs more: a graph that held its address would
+        replay into memory given away.)"""
+        if not self._ws_bytes:
+            return None
+        with on_stream(self._fixed_stream):
+            if torch.cuda.is_current_stream_capturing():
+                self.ws, self._ws_stream = torch.empty(self._ws_bytes, dtype=torch.uint8,
+                                                       device=self.q.device), None
+            elif self._ws_stream != self._stream_handle:
+                self._ws_stream = self._stream_handle
+                self.ws = _workspace(self.q.device, self._ws_stream, self._ws_bytes)
+        return self.ws
+
+    def _decode(self, entry: str, side: Optional[torch.cuda.Stream] = None) -> None:
+        # (a merge launched by itself reads what the partial launch before it left;
+        # beside the extend launch, the caller took the scratch before that)
+        ws = self.ws if side is not None or entry == "tf_attn_decode_merge" else self._scratch()
+        handle = side.cuda_stream if side is not None else self._stream_handle
         if self._n_rows_items:
             if entry == "tf_attn_decode_merge":
                 return   # part of the rows launch
@@ -722,6 +740,7 @@ class SlotAttentionCall:
             main, side = self.stream, _side_stream(self.q.device)
             fork, join = _fork_join_events(self.q.device, main)
             fork.record(main)
+            self._scratch()   # before the extend launch frees its own to this stream's pool
             self.run_extend()
             side.wait_event(fork)
             self._decode("tf_attn_decode", side)
