@@ -326,7 +326,9 @@ int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* 
 /* tf_attn_extend_split: tf_attn_extend (head_dim 256) over the pieces and merge
  * entries of tf_attn_plan_blocks.  workspace: 16-byte aligned scratch of
  * tf_attn_extend_split_workspace_bytes() (fp32 partials of a piece per compute
- * unit of the current device; no initialisation needed).
+ * unit of the current device; no initialisation needed).  The lengths may differ
+ * from those at planning: the last piece of an entry takes every key from its
+ * first tile on, and a piece without keys counts for nothing.
  */
 int64_t tf_attn_extend_split_workspace_bytes(void);
 

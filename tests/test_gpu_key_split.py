@@ -164,6 +164,50 @@ def test_captured_split_step_replays(gpu):
         assert_attn_close(call.out, restatement(wl), what=f"replay {i}")
 
 
+@pytest.mark.parametrize("phases", [False, True])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_lengths_that_change_after_planning(gpu, fp8, phases):
+    """A plan kept on a batch, or on a call whose phases run one by one, with other
+    seq_lens in place: contexts beyond the planned pieces, and contexts that leave
+    pieces and whole entries without keys."""
+    mk = lambda seq, seed: workloads.build("split", seq, [90, 40], num_q_heads=24, num_kv_heads=4,
+                                           head_dim=256, pool_slots=16384, device=gpu, seed=seed,
+                                           max_reqs=8, kv_fp8=fp8)
+    live = mk([3000, 2000], 1)
+    width = 8000
+    table = torch.full((8, width), -1, dtype=torch.long, device=gpu)
+    table[:, :live.batch.req_to_token.shape[1]] = live.batch.req_to_token
+    live.batch.req_to_token = table
+    call = call_of(live)
+    kw = dict(scaling=live.scale, k_scale=live.k_scale, v_scale=live.v_scale)
+    run = lambda: slot_based_attention(live.q, live.k_pool, live.v_pool, live.batch, **kw)
+    first = (call.run_extend(), call.out)[1] if phases else run()
+    assert_attn_close(first, restatement(live), what="as planned")
+    r = (call if phases else live.batch._tf_attn_step_plans.popitem()[1]).route
+    assert r.split
+    if not phases:
+        run()   # (planned again, kept on the batch)
+    for i, seq in enumerate(([7000, 5000], [2980, 150], [100, 41], [700, 6000])):
+        wl = mk(seq, 20 + i)
+        table.fill_(-1)
+        w = wl.batch.req_to_token.shape[1]
+        table[:, :w] = wl.batch.req_to_token
+        for x, y in ((live.q, wl.q), (live.k_pool, wl.k_pool), (live.v_pool, wl.v_pool),
+                     (live.batch.seq_lens, wl.batch.seq_lens),
+                     (live.batch.req_pool_indices, wl.batch.req_pool_indices)):
+            x.copy_(y)
+        if fp8:
+            live.k_scale.copy_(wl.k_scale)
+            live.v_scale.copy_(wl.v_scale)
+        # scratch that holds anything but finite numbers
+        torch.empty(1 << 26, dtype=torch.float32, device=gpu).fill_(float("nan"))
+        torch.cuda.synchronize()
+        print(f"[split] lengths {seq} after the plan", flush=True)
+        out = (call.run_extend(), call.out)[1] if phases else run()
+        torch.cuda.synchronize()
+        assert_attn_close(out, restatement(wl), what=f"L={seq}")
+
+
 def test_plan_without_room_for_merges_stays_whole(gpu):
     """tf_attn_plan_blocks with fewer merge entries than the split needs."""
     from tokenfactory_amd import _native

@@ -513,7 +513,7 @@ class SlotAttentionCall:
         self._status = None
         self.route = None
         self._lists = None
-        self._lists_planned = False   # of a host-planned call (its lengths are fixed)
+        self._lists_planned = False   # of a host-planned call (its extend lengths are fixed)
         self.ws = None                # split scratch of the last launch
         self._ws_bytes = 0
         self._ws_stream = None        # whose shared scratch self.ws is (None: a graph's own)

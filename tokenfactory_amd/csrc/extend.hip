@@ -396,6 +396,10 @@ __device__ __forceinline__ bool softmax_tile(const f32x16& s, Row& row, float sl
   return __ballot(grow) != 0;
 }
 
+// The reference maximum that a piece's rows start with: its first tiles may hold
+// no key a row sees, and any score raises it.
+constexpr float kNoKeys = -1e30f;
+
 // kSplit: the work list may hold pieces of entries (an instance of its own: as
 // one kernel, large prefills took 0.4 % and mixed steps 2 % longer).
 template <bool FP8, bool kSplit>
@@ -420,6 +424,9 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
   if (ext <= 0) return;   // padding entry of a device-built work list
   // A piece of a split entry takes key tiles [wk[5], wk[6]) and writes slot
   // wk[7] - 1 of the partials; positions below are relative to its first key.
+  // The tiles come from the lengths at planning, the keys from the lengths now:
+  // the last piece (the next entry of the list starts at tile 0) takes every key
+  // from its first one on, and a piece left without keys writes empty partials.
   const int part = kSplit ? wk[7] : 0;
   const int key0 = part ? kBN * wk[5] : 0;
   int64_t len = a.seq_override > 0 ? (int64_t)a.seq_override : a.seq_lens[b];
@@ -427,7 +434,7 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
   const int L = (int)len - key0;
   const int P = L - ext;
   const int rows_total = ext * G;
-  if (L <= 0 || row0 >= rows_total) return;
+  if (row0 >= rows_total) return;
 
   const int64_t rrow = clamp_i64(a.rpi[b], 0, a.rtt_rows - 1);
   const int64_t* rtt = a.rtt + rrow * a.rtt_stride + key0;
@@ -443,8 +450,14 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
   // is finite after tile 0).
   const int blk_last_row = min(row0 + kExtendItemRows, rows_total) - 1;
   const int keys = min(L, P + blk_last_row / G + 1);
-  const int kend = part ? min(keys, kBN * (wk[6] - wk[5])) : keys;
-  if (kend <= 0) return;
+  const bool inner = kSplit && part && blockIdx.x + 1 < gridDim.x && wk[8 + 5] > 0;
+  const int kend = inner ? min(keys, kBN * (wk[6] - wk[5])) : keys;
+  if (L <= 0 || kend <= 0) {
+    if (kSplit && part && tid < kExtendItemRows)
+      reinterpret_cast<float2*>(a.part_ml)[(int64_t)(part - 1) * kExtendItemRows + tid] =
+          float2{kNoKeys, 0.f};
+    return;
+  }
   const int n_tiles = (kend + kBN - 1) / kBN;
   const int last = n_tiles - 1;
   const int w_first = row0 + kRowsPerWave * w;
@@ -540,9 +553,7 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
 #pragma unroll
   for (int kk = 0; kk < 16; ++kk) asm volatile("" ::"v"(qf[kk]));
 
-  // (a piece's first tiles may hold no key a row sees: its maximum starts at a
-  // finite value that any score raises)
-  Row row{part ? -1e30f : -INFINITY, 0.f, 0.f};
+  Row row{part ? kNoKeys : -INFINITY, 0.f, 0.f};
   f32x16 acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = f32x16{};
@@ -744,6 +755,11 @@ __global__ void __launch_bounds__(kThreads) extend_merge_kernel(ExtendArgs a, co
   const int rows_total = ext * G;
   const int first = mg[2] + kRowsPerWave * blockIdx.y;
   if (ext <= 0 || first >= rows_total) return;
+  // (an entry without a key now: not written, as by the extend kernel)
+  const int64_t len = min(a.seq_override > 0 ? (int64_t)a.seq_override : a.seq_lens[mg[0]],
+                          a.rtt_cols);
+  const int last_row = min(mg[2] + kExtendItemRows, rows_total) - 1;
+  if (len <= 0 || len - ext + last_row / G + 1 <= 0) return;
   const int hk = mg[1], q_start = mg[3], slot0 = mg[5], n_pieces = mg[6];
   const int lane = threadIdx.x & 63, mt = wave_id();
   const int g = lane >> 5, n = lane & 31;
@@ -776,8 +792,9 @@ __global__ void __launch_bounds__(kThreads) extend_merge_kernel(ExtendArgs a, co
       if (p + k >= n_pieces) break;
       const float a2 = fast_exp2(ml[k].x - mn);
       l += ml[k].y * a2;
+      // (a piece without keys for the row may not have written its O)
 #pragma unroll
-      for (int rq = 0; rq < 4; ++rq) acc[rq] += o[k][rq] * a2;
+      for (int rq = 0; rq < 4; ++rq) acc[rq] += ml[k].y == 0.f ? f32x4{} : o[k][rq] * a2;
     }
     m = mn;
   }
