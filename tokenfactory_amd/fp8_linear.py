@@ -237,12 +237,31 @@ def block_fp8_linear(x: torch.Tensor, weight: torch.Tensor,
 
 
 def _plain(linear, kind) -> bool:
-    """Whether calling ``linear`` runs ``kind.forward`` and nothing else (no
-    subclass, replaced forward or hook)."""
+    """Whether calling ``linear`` runs ``kind.forward`` on plain tensors and nothing
+    else (no subclass of the module or of its weight, replaced forward or hook)."""
     return (type(linear) is kind and "forward" not in linear.__dict__
+            and type(linear.weight) in (nn.Parameter, torch.Tensor)
             and not (linear._forward_hooks or linear._forward_pre_hooks
                      or linear._backward_hooks or linear._backward_pre_hooks
                      or nn.modules.module._has_any_global_hook()))
+
+
+def _narrow_pair(x: torch.Tensor, first: nn.Module, second: nn.Module) -> bool:
+    """Whether ``tf_narrow_linear2`` takes the pair.  (The modules may be anything
+    that can be called: nothing of them is read before they are known to be plain.)"""
+    if not (_plain(first, nn.Linear) and _plain(second, nn.Linear)):
+        return False
+    n, k = first.weight.shape
+    if torch.is_grad_enabled() and (x.requires_grad or first.weight.requires_grad
+                                    or second.weight.requires_grad):
+        return False
+    if (torch.is_autocast_enabled() or not x.is_cuda or x.dim() != 2
+            or x.dtype != torch.bfloat16 or x.shape[0] == 0 or n > 64 or k % 32
+            or x.shape[1] != k or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16):
+        return False
+    return all(m.bias is None and m.weight.shape == (n, k) and m.weight.dtype == torch.bfloat16
+               and m.weight.device == x.device and m.weight.is_contiguous()
+               and m.weight.data_ptr() % 16 == 0 for m in (first, second))
 
 
 def narrow_linears(x: torch.Tensor, first: nn.Linear, second: nn.Linear):
@@ -252,17 +271,9 @@ def narrow_linears(x: torch.Tensor, first: nn.Linear, second: nn.Linear):
     Linears that are more than plain bf16 ``nn.Linear`` calls without a bias, that
     autograd is to record or autocast to cast, or whose sizes the kernel does not
     take are called one by one (``amax_partials`` is then None)."""
-    n, k = first.weight.shape
-    grad = torch.is_grad_enabled() and (x.requires_grad or first.weight.requires_grad
-                                        or second.weight.requires_grad)
-    if (grad or torch.is_autocast_enabled() or not x.is_cuda or x.dim() != 2
-            or x.dtype != torch.bfloat16 or x.shape[0] == 0 or n > 64 or k % 32
-            or x.shape[1] != k or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16
-            or not all(_plain(m, nn.Linear) and m.bias is None and m.weight.shape == (n, k)
-                       and m.weight.dtype == torch.bfloat16 and m.weight.device == x.device
-                       and m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 0
-                       for m in (first, second))):
+    if not _narrow_pair(x, first, second):
         return first(x), second(x), None
+    n, k = first.weight.shape
     rows = x.shape[0]
     outs = [torch.empty((rows, n), dtype=torch.bfloat16, device=x.device) for _ in range(2)]
     blocks = _native.load().tf_narrow_linear2_blocks(rows)
