@@ -46,6 +46,7 @@
 
 #include <mutex>
 
+#include "attn_row.h"
 #include "tf_common.h"
 #include "tf_internal.h"
 
@@ -85,6 +86,7 @@ struct DecodeArgs {
   uint32_t* amax;       // optional: raised to max |out| (bf16 bits), amax_commit
   float* ws_ml;
   float* ws_o;
+  int32_t* odd;       // OTHER: per unit that one workgroup owns, whether its O is not finite
   int32_t n_blocks;   // P: workgroups of the streaming kernel
 };
 
@@ -400,6 +402,27 @@ __device__ __forceinline__ void pv(const VBuf<C>& vb, const u32x2 (&pt)[C::NG],
   }
 }
 
+__device__ __forceinline__ bool not_finite(const f32x4& v) {
+  float y = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y = fmaf(v[e], 0.f, y);
+  return y != y;
+}
+
+// Whether any of the lane's accumulators is NaN or infinite.
+template <class C>
+__device__ __forceinline__ bool any_odd(const WaveState<C>& st) {
+  f32x4 x[2] = {};   // (eight short chains)
+#pragma unroll
+  for (int q = 0; q < C::NG; ++q)
+#pragma unroll
+    for (int i = 0; i < C::kAcc; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[i & 1][e] = fmaf(st.acc[q][i][e], 0.f, x[i & 1][e]);
+  const float y = (x[0][0] + x[0][1] + x[0][2] + x[0][3]) + (x[1][0] + x[1][1] + x[1][2] + x[1][3]);
+  return y != y;
+}
+
 // Item i of the call: query rows row0 .. (row = t * G + h: token t of the
 // request's ext new tokens, head h of the kv head's group) of request b, whose
 // first token is q row qrow.  A negative b marks a padding entry of a
@@ -641,6 +664,13 @@ decode_kernel(DecodeArgs a) {
 
     if (w == 0) {
       const bool whole = t0 == 0 && t1 == Ti;
+      if constexpr (C::OTHER) {
+        // NaN or infinite V values: see decode_merge_kernel.
+        if (whole) {
+          const bool odd = __ballot(any_odd<C>(st)) != 0;
+          if (lane == 0) a.odd[(int64_t)item * units_per_item + j] = odd;
+        }
+      }
       uint32_t om = 0;
 #pragma unroll
       for (int q = 0; q < C::NG; ++q) {
@@ -680,6 +710,13 @@ decode_kernel(DecodeArgs a) {
 // this takes 6.1, 7.3 and 4.9 us.  Eight waves per workgroup: with four, the
 // amax atomics (one per workgroup on one word) took 1.7 us more at B = 16, with
 // sixteen a launch starts 2 us later.
+// NaN or infinite V values at other head dims (OTHER): an MFMA multiplies every V
+// row of a tile with every query row's p, zero for keys the row does not see
+// (later tokens, repeats past the last key), and the low part of a visible key's
+// p may be zero or negative.  A row whose O is not finite is done again here,
+// over the keys it sees: O is looked at once per row or whole unit (a test of
+// each tile's V in the streaming kernel took 2 to 40 % of it; the rows done again
+// there cost it 3 %, in scalar registers).
 // Units of an empty request (L = 0) get zeros, as the reference's fully masked
 // scaled_dot_product_attention returns them (torch's safe softmax: a row with
 // no visible key is all zeros).
@@ -739,7 +776,8 @@ decode_merge_kernel(DecodeArgs a) {
     const int P = (int)min<int64_t>(a.n_blocks, N);   // as in the streaming kernel
     b0 = owner_of(p, N, P);
     b1 = owner_of(p + Ti - 1, N, P);
-    if (b0 == b1) return;   // written directly by the streaming kernel
+    // one owner: written directly by the streaming kernel
+    if (b0 == b1 && !(C::OTHER && a.odd[u])) return;
   }
 
   const int D = C::OTHER ? a.head_dim : C::DP;
@@ -760,7 +798,7 @@ decode_merge_kernel(DecodeArgs a) {
       gv = ld_g8(a.gate + (int64_t)qrow * a.gate_stride + (int64_t)hq * a.gate_hstride + 4 * lane);
     float m = -INFINITY, l = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (write) {
+    if (write && b0 != b1) {
       for (int bb = b0 + w % WPR; bb <= b1; bb += WPR * kMergeAhead) {
         f32x4 o[kMergeAhead];
         float2 ml[kMergeAhead];
@@ -811,6 +849,28 @@ decode_merge_kernel(DecodeArgs a) {
           l = l * a1 + l2 * a2;
           m = mn;
         }
+      }
+    }
+    if constexpr (C::OTHER) {
+      if (write && (b0 == b1 || __ballot(lane_in && not_finite(acc)))) {
+        const int len = item_len(a, im);
+        const int seen = C::BLK ? len - im.ext + t + 1 : len;
+        const int row_bytes = C::FP8 ? D : 2 * D;
+        RowState rs;
+        attend_row<C::FP8>(
+            rs, a.q + (int64_t)qrow * a.q_stride + (int64_t)hq * D,
+            reinterpret_cast<uint32_t*>(&so[w][0]), D,
+            a.rtt + clamp_i64(a.rpi[im.b], 0, a.rtt_rows - 1) * a.rtt_stride, 0, seen,
+            a.pool_slots, a.seq_override > 0, a.k_pool + (int64_t)hk * row_bytes,
+            a.v_pool + (int64_t)hk * row_bytes, (int64_t)a.hkv * row_bytes,
+            a.scale_log2 * (C::FP8 ? a.k_scale[0] : 1.f), lane);
+        om = max(om, write_row(rs, seen > 0 ? vscale / rs.l : 0.f, D,
+                               a.out + (int64_t)qrow * a.out_stride + (int64_t)hq * D,
+                               a.gate ? a.gate + (int64_t)qrow * a.gate_stride +
+                                            (int64_t)hq * a.gate_hstride
+                                      : nullptr,
+                               lane));
+        write = false;
       }
     }
     if (write) {
@@ -879,19 +939,20 @@ int make_decode_plan(int32_t n_items, int32_t num_q_heads, int32_t num_kv_heads,
   p->generic = false;
   // One persistent workgroup (4 waves) per CU measured fastest on MI355X.
   p->n_blocks = num_workgroups > 0 ? num_workgroups : device_cu_count();
-  plan_units(n_items, num_kv_heads, (group + 15) / 16, 16, group < 16 ? group : 16, kD, p);
+  plan_units(n_items, num_kv_heads, (group + 15) / 16, 16, group < 16 ? group : 16, kD,
+             false, p);
   return TF_OK;
 }
 
 void plan_units(int32_t n_items, int32_t num_kv_heads, int32_t n_hgroups, int32_t unit_rows,
-                int32_t rows_used, int32_t row_floats, DecodePlan* p) {
+                int32_t rows_used, int32_t row_floats, bool marked, DecodePlan* p) {
   p->n_hgroups = n_hgroups;
   p->rows_used = rows_used;
   p->n_units = (int64_t)n_items * num_kv_heads * n_hgroups;
   const int64_t rows = (p->n_units + p->n_blocks) * unit_rows;
   p->ml_bytes = (rows * 2 * 4 + 255) / 256 * 256;
   p->o_bytes = rows * row_floats * 4;
-  p->total_bytes = p->ml_bytes + p->o_bytes;
+  p->total_bytes = p->ml_bytes + p->o_bytes + (marked ? p->n_units * 4 : 0);
 }
 
 }  // namespace tfa
@@ -973,6 +1034,7 @@ void set_args(DecodeArgs* a, const void* q, int64_t q_row_stride, const void* k_
   char* ws = static_cast<char*>(workspace);
   a->ws_ml = reinterpret_cast<float*>(ws);
   a->ws_o = reinterpret_cast<float*>(ws + p.ml_bytes);
+  a->odd = reinterpret_cast<int32_t*>(ws + p.ml_bytes + p.o_bytes);
   a->n_blocks = p.n_blocks;
 }
 
@@ -1117,7 +1179,7 @@ int make_rows_plan(bool blocks, int32_t n_items, int32_t row_groups, int32_t num
   r->p.n_blocks = num_workgroups > 0 ? num_workgroups : device_cu_count() * (narrow ? 2 : 1);
   plan_units(n_items < kMaxItems ? n_items : kMaxItems, num_kv_heads,
              blocks ? 1 : (group + rows - 1) / rows, rows, blocks || group > rows ? rows : group,
-             r->narrow ? 128 : kD, &r->p);
+             r->narrow ? 128 : kD, head_dim != kD, &r->p);
   if (r->p.n_units > INT32_MAX) return fail(TF_ERR_INVALID, "rows: too many units");
   return TF_OK;
 }
