@@ -183,3 +183,21 @@ def test_fp8_gemm_workspace_queries_agree():
     assert nbytes > 0 and nbytes % (4 * 48 * (1024 + 256 + 132)) == 0
     assert lib.tf_fp8_linears_workspace_bytes(48, mats, 5, 5120) < 0
     assert lib.tf_fp8_linears_workspace_bytes(48, mats, 1, 5100) < 0
+
+
+@pytest.mark.parametrize("hq,hkv,d,kv_dtype", [(64, 8, 128, 0), (64, 16, 192, 0), (32, 8, 128, 1),
+                                               (24, 4, 256, 0), (24, 4, 256, 1), (8, 8, 64, 0)])
+def test_rows_workspace_is_bounded_by_the_grid(hq, hkv, d, kv_dtype):
+    """A workgroup leaves at most two partials: however many blocks a step has, the
+    scratch of tf_attn_rows holds two units of rows per workgroup (fp32 O, maximum
+    and sum) and a word per unit."""
+    kv = (_native.TF_DTYPE_BF16, _native.TF_DTYPE_FP8_E4M3)[kv_dtype]
+    width = 128 if d <= 128 and not kv_dtype else 256
+    cus = _native.rows_workspace_bytes(True, 1 << 20, 2, hq, hkv, d, kv, 0)
+    for grid in (1, 7, 256, 768):
+        sizes = [_native.rows_workspace_bytes(True, n, 2, hq, hkv, d, kv, grid)
+                 for n in (1, 3, 64, 700, 2048, 5000, 1 << 20)]
+        assert sizes == sorted(sizes)
+        assert sizes[-1] <= 2 * grid * 32 * (4 * width + 8) + 256 + 4 * 2048 * hkv
+    # the default grid: one workgroup per CU, two of the 128-dim kernel
+    assert cus <= 2 * 512 * 32 * (4 * 128 + 8) + 256 + 4 * 2048 * hkv

@@ -87,6 +87,16 @@ def test_strided_q_out_gate_and_amax(gpu):
         assert int(amax) == int(fused.abs().max().view(torch.int16))
 
 
+@pytest.mark.parametrize("d", [256, 128, 200])
+@pytest.mark.parametrize("workgroups", [1, 3, 7, 40, 100, 513])
+def test_units_cut_anywhere(gpu, d, workgroups):
+    """Grids with fewer and with more workgroups than units, whose ranges start and
+    end inside units: first, inner and last units of a workgroup."""
+    wl = case(gpu, [30, 700, 9, 300, 90, 33], [2, 5, 3, 1, 2, 6], 8, 2, d, d)
+    got = run(wl, decode_workgroups=workgroups)
+    assert_attn_close(got, restatement(wl), what=f"{workgroups} workgroups")
+
+
 def expected_lists(ext_lens, group, hkv, unit, max_rows):
     starts = np.concatenate([[0], np.cumsum(ext_lens)[:-1]]).tolist()
     blocks = [(b, starts[b], 1, r) for b, e in enumerate(ext_lens) if e == 1

@@ -13,8 +13,10 @@
 //   whatever the length mix. A workgroup walks its range as segments (one unit
 //   each); 4 waves take interleaved tiles of a segment. A unit owned entirely by
 //   one workgroup is written as final bf16 output; otherwise each owner stores
-//   an fp32 partial (O, max, sum) at index b + u (unique, < P + units) and a
-//   second small kernel merges them.
+//   an fp32 partial (O, max, sum) and a second small kernel merges them.  Only a
+//   workgroup's first and last unit can be shared: its partials are at slots 2 b
+//   and 2 b + 1, or at b + u (unique, < P + units) where that takes fewer (and in
+//   tf_attn_decode, whose workspace has that size).
 //   The whole GQA head group of a kv head shares every K/V row read from HBM.
 // Per segment: the slot ids of up to 2048 tokens at a time (int64 req_to_token
 // entries clamped to the pool) are staged in LDS with coalesced loads, and the
@@ -88,6 +90,7 @@ struct DecodeArgs {
   float* ws_o;
   int32_t* odd;       // OTHER: per unit that one workgroup owns, whether its O is not finite
   int32_t n_blocks;   // P: workgroups of the streaming kernel
+  bool by_owner;      // partial slots: two per workgroup (else one per workgroup and unit)
 };
 
 // The kernels' shape (NG = 1 or 2: four groups of 256 dims spill).  DP: head dims in a row's tile (256, or 128 for head dims
@@ -112,6 +115,7 @@ struct Cfg {
   static constexpr int kSteps = DP / 32;               // 32-dim MFMA steps of QK^T
   static constexpr int kRows = 16 * NG;                // query rows per unit
   static constexpr int kRowFloats = DP;                // a partial row's O
+  static constexpr bool kByOwner = OTHER || BLK;       // DecodeArgs::by_owner may be set
 };
 
 template <class C>
@@ -540,7 +544,7 @@ decode_kernel(DecodeArgs a) {
     item = lo;
   }
 
-  while (x < x_end) {
+  for (int part_at = 0; x < x_end; part_at = 1) {   // 0: the workgroup's first unit
     // ---- locate the segment: unit (item, j), tiles [t0, t1)
     while ((int64_t)units_per_item * sm.ipre[item + 1] <= x) ++item;
     const int Ti = sm.ipre[item + 1] - sm.ipre[item];
@@ -682,7 +686,9 @@ decode_kernel(DecodeArgs a) {
           om = max(om, write_output<C>(a, qrow, hq, g, st, q, vscale));
         } else {
           // Partial of unit u = item * units_per_item + j from this workgroup.
-          const int64_t part = (int64_t)blockIdx.x + (int64_t)item * units_per_item + j;
+          const int64_t part = C::kByOwner && a.by_owner
+                                   ? 2 * (int64_t)blockIdx.x + part_at
+                                   : (int64_t)blockIdx.x + (int64_t)item * units_per_item + j;
           const int64_t pr = part * C::kRows + 16 * q + n;
           f32x4* po = reinterpret_cast<f32x4*>(a.ws_o + pr * C::kRowFloats) + g * C::kAcc;
 #pragma unroll
@@ -745,6 +751,7 @@ decode_merge_kernel(DecodeArgs a) {
   const int first = blockIdx.y * kRows, stride = gridDim.y * kRows;
   if (im.b < 0 || first >= n_rows) return;   // padding
 
+  const bool odd = C::OTHER && a.odd[u];   // (under the reductions; of whole units only)
   // Tiles before this item and in total (block reductions over items).
   const int Ti = item_tiles<C>(a, item);
   int before = 0, total = 0;
@@ -770,14 +777,16 @@ decode_merge_kernel(DecodeArgs a) {
     total += red[1][k];
   }
   int b0 = 0, b1 = -1;   // an empty context: zeros
+  bool inside = false;   // the unit starts inside the first owner's range
   if (Ti > 0) {
     const int64_t N = (int64_t)units_per_item * total;
     const int64_t p = (int64_t)units_per_item * before + (int64_t)j * Ti;
     const int P = (int)min<int64_t>(a.n_blocks, N);   // as in the streaming kernel
     b0 = owner_of(p, N, P);
+    inside = b0 * N / P < p;
     b1 = owner_of(p + Ti - 1, N, P);
     // one owner: written directly by the streaming kernel
-    if (b0 == b1 && !(C::OTHER && a.odd[u])) return;
+    if (b0 == b1 && !odd) return;
   }
 
   const int D = C::OTHER ? a.head_dim : C::DP;
@@ -804,7 +813,10 @@ decode_merge_kernel(DecodeArgs a) {
         float2 ml[kMergeAhead];
 #pragma unroll
         for (int k = 0; k < kMergeAhead; ++k) {
-          const int64_t pr = ((int64_t)min(bb + WPR * k, b1) + u) * C::kRows + n;
+          const int bk = min(bb + WPR * k, b1);
+          const int64_t slot =
+              C::kByOwner && a.by_owner ? 2 * (int64_t)bk + (inside && bk == b0 ? 1 : 0) : (int64_t)bk + u;
+          const int64_t pr = slot * C::kRows + n;
           o[k] = reinterpret_cast<const f32x4*>(
               a.ws_o + pr * C::kRowFloats)[C::DP == 256 ? lane : lane & 31];
           ml[k] = reinterpret_cast<const float2*>(a.ws_ml)[pr];
@@ -940,16 +952,19 @@ int make_decode_plan(int32_t n_items, int32_t num_q_heads, int32_t num_kv_heads,
   // One persistent workgroup (4 waves) per CU measured fastest on MI355X.
   p->n_blocks = num_workgroups > 0 ? num_workgroups : device_cu_count();
   plan_units(n_items, num_kv_heads, (group + 15) / 16, 16, group < 16 ? group : 16, kD,
-             false, p);
+             false, false, p);
   return TF_OK;
 }
 
 void plan_units(int32_t n_items, int32_t num_kv_heads, int32_t n_hgroups, int32_t unit_rows,
-                int32_t rows_used, int32_t row_floats, bool marked, DecodePlan* p) {
+                int32_t rows_used, int32_t row_floats, bool by_owner, bool marked,
+                DecodePlan* p) {
   p->n_hgroups = n_hgroups;
   p->rows_used = rows_used;
   p->n_units = (int64_t)n_items * num_kv_heads * n_hgroups;
-  const int64_t rows = (p->n_units + p->n_blocks) * unit_rows;
+  p->by_owner = by_owner && p->n_units > p->n_blocks;
+  const int64_t slots = p->n_blocks + (p->by_owner ? p->n_blocks : p->n_units);
+  const int64_t rows = slots * unit_rows;
   p->ml_bytes = (rows * 2 * 4 + 255) / 256 * 256;
   p->o_bytes = rows * row_floats * 4;
   p->total_bytes = p->ml_bytes + p->o_bytes + (marked ? p->n_units * 4 : 0);
@@ -1036,6 +1051,7 @@ void set_args(DecodeArgs* a, const void* q, int64_t q_row_stride, const void* k_
   a->ws_o = reinterpret_cast<float*>(ws + p.ml_bytes);
   a->odd = reinterpret_cast<int32_t*>(ws + p.ml_bytes + p.o_bytes);
   a->n_blocks = p.n_blocks;
+  a->by_owner = p.by_owner;
 }
 
 // Launches the streaming kernel and / or the merge of one call.
@@ -1179,7 +1195,7 @@ int make_rows_plan(bool blocks, int32_t n_items, int32_t row_groups, int32_t num
   r->p.n_blocks = num_workgroups > 0 ? num_workgroups : device_cu_count() * (narrow ? 2 : 1);
   plan_units(n_items < kMaxItems ? n_items : kMaxItems, num_kv_heads,
              blocks ? 1 : (group + rows - 1) / rows, rows, blocks || group > rows ? rows : group,
-             r->narrow ? 128 : kD, head_dim != kD, &r->p);
+             r->narrow ? 128 : kD, blocks || head_dim != kD, head_dim != kD, &r->p);
   if (r->p.n_units > INT32_MAX) return fail(TF_ERR_INVALID, "rows: too many units");
   return TF_OK;
 }

@@ -34,15 +34,17 @@ struct DecodePlan {
   int32_t rows_used;    // query rows of a unit that can be real
   int64_t n_units;      // items * kv_heads * n_hgroups
   int64_t ml_bytes, o_bytes, total_bytes;  // split partials: (max, sum) and O
+  bool by_owner;        // partial slots: two per workgroup, not one per workgroup and unit
   bool generic;         // head_dim != 256: the one-wave-per-row kernel, no workspace
 };
 int make_decode_plan(int32_t n_items, int32_t num_q_heads, int32_t num_kv_heads,
                      int32_t head_dim, int32_t max_seq_len, int32_t num_workgroups,
                      DecodePlan* plan);
-// Units and split workspace of a plan whose n_blocks is set (marked: with a word
-// per unit).
+// Units and split workspace of a plan whose n_blocks is set (by_owner: partials of
+// at most two units per workgroup; marked: with a word per unit).
 void plan_units(int32_t n_items, int32_t num_kv_heads, int32_t n_hgroups, int32_t unit_rows,
-                int32_t rows_used, int32_t row_floats, bool marked, DecodePlan* plan);
+                int32_t rows_used, int32_t row_floats, bool by_owner, bool marked,
+                DecodePlan* plan);
 
 // Extend kernel arguments (validated by tf_attn_extend).  Work items cover
 // kExtendItemRows flattened (token, q-head-of-group) rows each.
