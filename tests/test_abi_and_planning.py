@@ -190,7 +190,7 @@ def test_fp8_gemm_workspace_queries_agree():
 def test_rows_workspace_is_bounded_by_the_grid(hq, hkv, d, kv_dtype):
     """A workgroup leaves at most two partials: however many blocks a step has, the
     scratch of tf_attn_rows holds two units of rows per workgroup (fp32 O, maximum
-    and sum) and a word per unit."""
+    and sum), a word per block and one per unit."""
     kv = (_native.TF_DTYPE_BF16, _native.TF_DTYPE_FP8_E4M3)[kv_dtype]
     width = 128 if d <= 128 and not kv_dtype else 256
     cus = _native.rows_workspace_bytes(True, 1 << 20, 2, hq, hkv, d, kv, 0)
@@ -198,6 +198,6 @@ def test_rows_workspace_is_bounded_by_the_grid(hq, hkv, d, kv_dtype):
         sizes = [_native.rows_workspace_bytes(True, n, 2, hq, hkv, d, kv, grid)
                  for n in (1, 3, 64, 700, 2048, 5000, 1 << 20)]
         assert sizes == sorted(sizes)
-        assert sizes[-1] <= 2 * grid * 32 * (4 * width + 8) + 256 + 4 * 2048 * hkv
+        assert sizes[-1] <= 2 * grid * 32 * (4 * width + 8) + 256 + 4 * (2049 + 2048 * hkv)
     # the default grid: one workgroup per CU, two of the 128-dim kernel
-    assert cus <= 2 * 512 * 32 * (4 * 128 + 8) + 256 + 4 * 2048 * hkv
+    assert cus <= 2 * 512 * 32 * (4 * 128 + 8) + 256 + 4 * (2049 + 2048 * hkv)

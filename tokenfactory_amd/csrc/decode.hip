@@ -88,6 +88,7 @@ struct DecodeArgs {
   uint32_t* amax;       // optional: raised to max |out| (bf16 bits), amax_commit
   float* ws_ml;
   float* ws_o;
+  int32_t* ipre;      // row plans: the streaming kernel's tile prefix, for the merge
   int32_t* odd;       // OTHER: per unit that one workgroup owns, whether its O is not finite
   int32_t n_blocks;   // P: workgroups of the streaming kernel
   bool by_owner;      // partial slots: two per workgroup (else one per workgroup and unit)
@@ -115,7 +116,7 @@ struct Cfg {
   static constexpr int kSteps = DP / 32;               // 32-dim MFMA steps of QK^T
   static constexpr int kRows = 16 * NG;                // query rows per unit
   static constexpr int kRowFloats = DP;                // a partial row's O
-  static constexpr bool kByOwner = OTHER || BLK;       // DecodeArgs::by_owner may be set
+  static constexpr bool kRowPlan = OTHER || BLK;       // DecodeArgs::by_owner and ipre are set
 };
 
 template <class C>
@@ -519,6 +520,8 @@ decode_kernel(DecodeArgs a) {
   const int n = lane & 15;
 
   item_prefix<C>(a, sm.ipre, sm.wsum);
+  if (C::kRowPlan && blockIdx.x == 0)
+    for (int i = tid; i <= a.n_items; i += kWaves * kWave) a.ipre[i] = sm.ipre[i];
   const int units_per_item = a.hkv * a.n_hg;
   const int64_t N = (int64_t)units_per_item * sm.ipre[a.n_items];
   // With P <= N every workgroup's range is non-empty, so the owners of a unit
@@ -686,7 +689,7 @@ decode_kernel(DecodeArgs a) {
           om = max(om, write_output<C>(a, qrow, hq, g, st, q, vscale));
         } else {
           // Partial of unit u = item * units_per_item + j from this workgroup.
-          const int64_t part = C::kByOwner && a.by_owner
+          const int64_t part = C::kRowPlan && a.by_owner
                                    ? 2 * (int64_t)blockIdx.x + part_at
                                    : (int64_t)blockIdx.x + (int64_t)item * units_per_item + j;
           const int64_t pr = part * C::kRows + 16 * q + n;
@@ -751,30 +754,36 @@ decode_merge_kernel(DecodeArgs a) {
   const int first = blockIdx.y * kRows, stride = gridDim.y * kRows;
   if (im.b < 0 || first >= n_rows) return;   // padding
 
-  const bool odd = C::OTHER && a.odd[u];   // (under the reductions; of whole units only)
-  // Tiles before this item and in total (block reductions over items).
-  const int Ti = item_tiles<C>(a, item);
-  int before = 0, total = 0;
-  for (int i = tid; i < a.n_items; i += kMergeWaves * kWave) {
-    const int t = item_tiles<C>(a, i);
-    total += t;
-    if (i < item) before += t;
-  }
+  const bool odd = C::OTHER && a.odd[u];   // (of whole units only)
+  // Tiles before this item, of it and in total.
+  int before = 0, Ti = 0, total = 0;
+  if constexpr (C::kRowPlan) {
+    before = a.ipre[item];
+    Ti = a.ipre[item + 1] - before;
+    total = a.ipre[a.n_items];
+  } else {   // block reductions over items
+    Ti = item_tiles<C>(a, item);
+    for (int i = tid; i < a.n_items; i += kMergeWaves * kWave) {
+      const int t = item_tiles<C>(a, i);
+      total += t;
+      if (i < item) before += t;
+    }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    before += __shfl_xor(before, off, kWave);
-    total += __shfl_xor(total, off, kWave);
-  }
-  if (lane == 0) {
-    red[0][w] = before;
-    red[1][w] = total;
-  }
-  __syncthreads();
-  before = total = 0;
+    for (int off = 32; off > 0; off >>= 1) {
+      before += __shfl_xor(before, off, kWave);
+      total += __shfl_xor(total, off, kWave);
+    }
+    if (lane == 0) {
+      red[0][w] = before;
+      red[1][w] = total;
+    }
+    __syncthreads();
+    before = total = 0;
 #pragma unroll
-  for (int k = 0; k < kMergeWaves; ++k) {
-    before += red[0][k];
-    total += red[1][k];
+    for (int k = 0; k < kMergeWaves; ++k) {
+      before += red[0][k];
+      total += red[1][k];
+    }
   }
   int b0 = 0, b1 = -1;   // an empty context: zeros
   bool inside = false;   // the unit starts inside the first owner's range
@@ -815,7 +824,7 @@ decode_merge_kernel(DecodeArgs a) {
         for (int k = 0; k < kMergeAhead; ++k) {
           const int bk = min(bb + WPR * k, b1);
           const int64_t slot =
-              C::kByOwner && a.by_owner ? 2 * (int64_t)bk + (inside && bk == b0 ? 1 : 0) : (int64_t)bk + u;
+              C::kRowPlan && a.by_owner ? 2 * (int64_t)bk + (inside && bk == b0 ? 1 : 0) : (int64_t)bk + u;
           const int64_t pr = slot * C::kRows + n;
           o[k] = reinterpret_cast<const f32x4*>(
               a.ws_o + pr * C::kRowFloats)[C::DP == 256 ? lane : lane & 31];
@@ -952,22 +961,22 @@ int make_decode_plan(int32_t n_items, int32_t num_q_heads, int32_t num_kv_heads,
   // One persistent workgroup (4 waves) per CU measured fastest on MI355X.
   p->n_blocks = num_workgroups > 0 ? num_workgroups : device_cu_count();
   plan_units(n_items, num_kv_heads, (group + 15) / 16, 16, group < 16 ? group : 16, kD,
-             false, false, p);
+             false, p);
   return TF_OK;
 }
 
 void plan_units(int32_t n_items, int32_t num_kv_heads, int32_t n_hgroups, int32_t unit_rows,
-                int32_t rows_used, int32_t row_floats, bool by_owner, bool marked,
-                DecodePlan* p) {
+                int32_t rows_used, int32_t row_floats, bool row_plan, DecodePlan* p) {
   p->n_hgroups = n_hgroups;
   p->rows_used = rows_used;
   p->n_units = (int64_t)n_items * num_kv_heads * n_hgroups;
-  p->by_owner = by_owner && p->n_units > p->n_blocks;
+  p->by_owner = row_plan && p->n_units > p->n_blocks;
   const int64_t slots = p->n_blocks + (p->by_owner ? p->n_blocks : p->n_units);
   const int64_t rows = slots * unit_rows;
   p->ml_bytes = (rows * 2 * 4 + 255) / 256 * 256;
   p->o_bytes = rows * row_floats * 4;
-  p->total_bytes = p->ml_bytes + p->o_bytes + (marked ? p->n_units * 4 : 0);
+  p->total_bytes = p->ml_bytes + p->o_bytes;
+  if (row_plan) p->total_bytes += 4 * (n_items + 1 + p->n_units);   // tile prefix, unit marks
 }
 
 }  // namespace tfa
@@ -1049,7 +1058,8 @@ void set_args(DecodeArgs* a, const void* q, int64_t q_row_stride, const void* k_
   char* ws = static_cast<char*>(workspace);
   a->ws_ml = reinterpret_cast<float*>(ws);
   a->ws_o = reinterpret_cast<float*>(ws + p.ml_bytes);
-  a->odd = reinterpret_cast<int32_t*>(ws + p.ml_bytes + p.o_bytes);
+  a->ipre = reinterpret_cast<int32_t*>(ws + p.ml_bytes + p.o_bytes);
+  a->odd = a->ipre + n_items + 1;
   a->n_blocks = p.n_blocks;
   a->by_owner = p.by_owner;
 }
@@ -1195,7 +1205,7 @@ int make_rows_plan(bool blocks, int32_t n_items, int32_t row_groups, int32_t num
   r->p.n_blocks = num_workgroups > 0 ? num_workgroups : device_cu_count() * (narrow ? 2 : 1);
   plan_units(n_items < kMaxItems ? n_items : kMaxItems, num_kv_heads,
              blocks ? 1 : (group + rows - 1) / rows, rows, blocks || group > rows ? rows : group,
-             r->narrow ? 128 : kD, blocks || head_dim != kD, head_dim != kD, &r->p);
+             r->narrow ? 128 : kD, blocks || head_dim != kD, &r->p);
   if (r->p.n_units > INT32_MAX) return fail(TF_ERR_INVALID, "rows: too many units");
   return TF_OK;
 }

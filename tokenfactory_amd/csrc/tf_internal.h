@@ -40,11 +40,10 @@ struct DecodePlan {
 int make_decode_plan(int32_t n_items, int32_t num_q_heads, int32_t num_kv_heads,
                      int32_t head_dim, int32_t max_seq_len, int32_t num_workgroups,
                      DecodePlan* plan);
-// Units and split workspace of a plan whose n_blocks is set (by_owner: partials of
-// at most two units per workgroup; marked: with a word per unit).
+// Units and split workspace of a plan whose n_blocks is set (row_plan: of
+// tf_attn_rows, except its 256-dim calls without blocks, which are tf_attn_decode's).
 void plan_units(int32_t n_items, int32_t num_kv_heads, int32_t n_hgroups, int32_t unit_rows,
-                int32_t rows_used, int32_t row_floats, bool by_owner, bool marked,
-                DecodePlan* plan);
+                int32_t rows_used, int32_t row_floats, bool row_plan, DecodePlan* plan);
 
 // Extend kernel arguments (validated by tf_attn_extend).  Work items cover
 // kExtendItemRows flattened (token, q-head-of-group) rows each.
