@@ -151,6 +151,28 @@ def test_more_blocks_than_one_launch_takes(gpu):
     check(two, "2500 rows of 64 heads")
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("groups,ext,pre", [
+    (0, [10] * 66, 30), (1, [4] * 130 + [1] * 3 + [70], 25), (0, [7] * 300 + [1] * 280, 20),
+    (1, [2] * 5 + [1] * 40, 200), (2, [5] * 16, 900)])
+def test_every_way_of_short_extends(gpu, groups, ext, pre, fp8):
+    """The extend kernel, units of 16 and of 32 rows, as the rule chooses them, and
+    a device-planned call (whose lists have room for other lengths)."""
+    hq, hkv = 24, 4
+    seq = [e + pre + i % 7 for i, e in enumerate(ext)]
+    wl = case(gpu, seq, ext, hq, hkv, 256, len(ext), fp8)
+    calls = [SlotAttentionCall(wl.q, wl.k_pool, wl.v_pool, wl.batch, scaling=wl.scale,
+                               k_scale=wl.k_scale, v_scale=wl.v_scale, device_plan=dev)
+             for dev in (False, True)]
+    if not fp8:
+        assert calls[0].route.row_groups == groups
+    outs = [run(wl)] + [c.run() for c in calls]
+    torch.cuda.synchronize()
+    ref = restatement(wl)
+    for out in outs:
+        assert_attn_close(out, ref, what=f"{len(ext)} requests")
+
+
 def test_captured_step_replays_over_other_routes(gpu):
     """Replays over batches with the same T and B whose requests fall on either
     side of SHORT_ROWS: every replay against the oracle."""

@@ -21,6 +21,7 @@ by phase. Only ROCm device tensors are accepted; there is no CPU path.
 """
 from __future__ import annotations
 
+import math
 import threading
 from typing import Dict, Optional, Tuple
 
@@ -165,20 +166,69 @@ SHORT_ROWS = 64      # query rows per kv head up to which an extend takes the st
 MAX_ROW_ITEMS = 2048
 
 
+def _n_units(ext: int, group: int, unit: int) -> int:
+    """Blocks of ``unit`` rows of a request with ``ext`` new tokens (none spans two
+    work entries of 256 rows, which are whole units)."""
+    return -(-ext * group // unit)
+
+
+# Streaming kernel, one workgroup per CU: us per unit and us per 16 keys of it, in
+# units of 16 and of 32 rows, for bf16 and for fp8 pools.
+_UNIT_US = {False: ((8.0, 0.80), (20.0, 0.82)), True: ((11.5, 0.33), (26.0, 0.53))}
+
+
+def _row_groups(short, n_dec: int, group: int, n_kv: int, fp8: bool, max_len: int,
+                cus: int) -> int:
+    """Groups of 16 rows per unit (1 or 2) for a step's short extends (and then its
+    decodes) as row blocks, or 0: extend kernel, beside the decode kernel.
+
+    The times of the three ways, in us, from the numbers of units and entries and
+    from the longest context, the one length that the host knows (contexts are
+    taken to be 0.65 of it on average): a unit's rows stream its keys once, so 17 to
+    32 rows are one unit of 32 where the keys decide and two of 16 where the units'
+    own cost does (short contexts, or decodes beside them, whose few rows leave a
+    unit of 32 empty; fp8 keys cost half the bytes and the same arithmetic); the
+    extend kernel takes 1.4 us per 32 keys and nine such steps per entry, in rounds of
+    one entry per CU.  Beside decodes it runs on a second stream, for which the host
+    alone takes 58 us.
+    Measured (24 / 4 heads of 256, us: extend kernel, units of 16, of 32):
+    20 requests of 2 to 4 tokens on 1k to 8k keys 346, 108, 82; 64 of 5 on 1k to 8k
+    365, 386, 232; 64 of 6 365, 563, 416; 64 of 10 on 1k to 2k 126, 289, 180; 256 of
+    8 on 500 to 1500 308, 563, 438; 128 of 4 on 100 to 300 49, 85, 78; 64 decodes
+    beside one of 3 tokens 246, 202, 206, beside 16 of 3 or 4 338, 306, 277; 900
+    decodes beside 200 of 4 on 100 to 500 350, 394, 472; 8 decodes of 65k fp8 beside
+    one of 4 230, 185, 271."""
+    per_cu = n_kv / (cus or 256)
+    tiles = 0.65 * max_len / 16
+    cost = [f + a * tiles for f, a in _UNIT_US[fp8]]
+    rows = [12 + per_cu * c * (sum(_n_units(e, group, u) for e in short)
+                               + n_dec * _n_units(1, group, u))
+            for c, u in zip(cost, (16, 32))]
+    rounds = len(short) * per_cu
+    rounds = rounds if rounds > 4 else math.ceil(rounds)
+    ext = rounds * 1.4 * (0.9 * max_len / 32 + 9)
+    dec = per_cu * cost[0] * n_dec * _n_units(1, group, 16)
+    other = 5 + max(ext, dec) + 0.35 * min(ext, dec)
+    if n_dec:
+        other = max(other + 5, 58)
+    if other <= min(rows):
+        return 0
+    return 1 if rows[0] <= rows[1] else 2
+
+
 class Route:
     """Which kernels a step's rows take, from what the host knows of it.
 
     At head_dim 256 decode rows run the streaming kernel and extends the extend
     kernel, except that requests with few new tokens (2 <= ext, ext * G <=
     ``SHORT_ROWS`` query rows per kv head, e.g. up to 10 tokens at G = 6) are row
-    blocks of the streaming kernel too: its work is spread evenly over the CUs,
-    where the extend kernel gives a request one workgroup per kv head with 256
-    rows to fill (20 requests of 2 to 4 tokens on 1k to 8k keys: 347 us there,
-    84 us here).  At other head dims every row runs the streaming kernel (2
-    prompts of 100 to 400 tokens beside 12 decodes, 32 / 8 heads of 128: 1660 us
-    on the one-wave-per-row kernel, 88 us here); fp8 pools need a head dim that
-    is a multiple of 16, whose rows keep the 16-byte alignment of its loads, and
-    stay on the one-wave-per-row kernel otherwise.
+    blocks of the streaming kernel too where ``_row_groups`` finds that faster: its
+    work is spread evenly over the CUs, where the extend kernel gives a request
+    one workgroup per kv head with 256 rows to fill.  At other head dims every row
+    runs the streaming kernel (2 prompts of 100 to 400 tokens beside 12 decodes,
+    32 / 8 heads of 128: 1660 us on the one-wave-per-row kernel, 95 us here); fp8
+    pools need a head dim that is a multiple of 16, whose rows keep the 16-byte
+    alignment of its loads, and stay on the one-wave-per-row kernel otherwise.
 
     Extend entries that leave CUs idle are cut over their keys
     (``tf_attn_plan_blocks`` decides from the lengths on the device): ``split``
@@ -216,27 +266,38 @@ class Route:
             self.max_rows = 1 << 62
             self.row_groups = 2 if n_work else 1   # blocks whenever the step is planned
             unit = 16 * self.row_groups
-            self.n_blocks = n_tok * group // unit + (n_work // n_kv if n_work else 0) + bsz
+            if exact:
+                self.n_blocks = sum(_n_units(e, group, unit) for e in ext_lens)
+            else:
+                self.n_blocks = n_tok * group // unit + (n_work // n_kv if n_work else 0) + bsz
             self.run_extend = False
             return
+        n_dec = sum(1 for e in ext_lens if e == 1)
         short = [e for e in ext_lens if e > 1 and e * group <= SHORT_ROWS]
         if short:
-            self.row_groups = 1 if max(short) * group <= 16 else 2
+            self.row_groups = _row_groups(short, n_dec, group, n_kv, fp8, max_len, cus)
+        if self.row_groups:
             unit = 16 * self.row_groups
-            self.n_blocks = bsz * max(-(-SHORT_ROWS // unit), -(-group // unit))
+            if exact:
+                self.n_blocks = sum(_n_units(e, group, unit) for e in short) \
+                    + n_dec * _n_units(1, group, unit)
+            else:
+                self.n_blocks = bsz * max(-(-SHORT_ROWS // unit), -(-group // unit))
             self.n_pieces = n_work
         long_ = [e for e in ext_lens if e > 1 and e * group > SHORT_ROWS]
         long_entries = sum(n_kv * -(-e * group // EXTEND_TILE_ROWS) for e in long_)
+        # (not where the extend kernel has short extends too: they fill it)
         if n_work and 0 < long_entries <= cus and max_len >= SPLIT_KEYS \
+                and (self.row_groups or not short) \
                 and len(long_) * (max_len - 768) >= 86 * bsz:
             self.split = True
             self.n_pieces = cus if exact else max(n_work, cus)
             # (an empty merge entry still costs its workgroups' launch)
             self.n_merges = min(cus // 2, long_entries) if exact else cus // 2
         if exact:
-            n_short, n_dec = len(short), sum(1 for e in ext_lens if e == 1)
-            self.run_extend = n_short + n_dec < bsz
-            self.run_rows = n_short + n_dec > 0
+            n_rows = n_dec + (len(short) if self.row_groups else 0)
+            self.run_extend = n_rows < bsz
+            self.run_rows = n_rows > 0
             if not self.run_extend:
                 self.n_pieces = 0
 
