@@ -54,7 +54,7 @@ def test_other_modules_are_called(make, place):
     x = torch.randn(5, 64)
     pair = [nn.Linear(64, 8, bias=False), nn.Linear(64, 8, bias=False)]
     pair[place] = make()
-    assert not _narrow_pair(x, *pair)
+    assert _narrow_pair(x, *pair) is None
     first, second, partials = narrow_linears(x, *pair)
     assert partials is None
     assert torch.equal(first, pair[0](x)) and torch.equal(second, pair[1](x))

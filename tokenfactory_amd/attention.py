@@ -721,13 +721,19 @@ class SlotAttentionCall:
         replay into memory given away.)"""
         if not self._ws_bytes:
             return None
-        with on_stream(self._fixed_stream):
-            if torch.cuda.is_current_stream_capturing():
-                self.ws, self._ws_stream = torch.empty(self._ws_bytes, dtype=torch.uint8,
-                                                       device=self.q.device), None
-            elif self._ws_stream != self._stream_handle:
-                self._ws_stream = self._stream_handle
-                self.ws = _workspace(self.q.device, self._ws_stream, self._ws_bytes)
+        if self._fixed_stream is None:
+            return self._scratch_of_current()
+        with torch.cuda.stream(self._fixed_stream):
+            return self._scratch_of_current()
+
+    def _scratch_of_current(self) -> torch.Tensor:
+        if torch.cuda.is_current_stream_capturing():
+            self.ws, self._ws_stream = torch.empty(self._ws_bytes, dtype=torch.uint8,
+                                                   device=self.q.device), None
+            return self.ws
+        handle = _native.current_stream(self.q.device)
+        if self._ws_stream != handle:
+            self._ws_stream, self.ws = handle, _workspace(self.q.device, handle, self._ws_bytes)
         return self.ws
 
     def _decode(self, entry: str, side: Optional[torch.cuda.Stream] = None) -> None:

@@ -240,28 +240,32 @@ def _plain(linear, kind) -> bool:
     """Whether calling ``linear`` runs ``kind.forward`` on plain tensors and nothing
     else (no subclass of the module or of its weight, replaced forward or hook)."""
     return (type(linear) is kind and "forward" not in linear.__dict__
-            and type(linear.weight) in (nn.Parameter, torch.Tensor)
+            and type(linear._parameters.get("weight")) is nn.Parameter
             and not (linear._forward_hooks or linear._forward_pre_hooks
                      or linear._backward_hooks or linear._backward_pre_hooks
                      or nn.modules.module._has_any_global_hook()))
 
 
-def _narrow_pair(x: torch.Tensor, first: nn.Module, second: nn.Module) -> bool:
-    """Whether ``tf_narrow_linear2`` takes the pair.  (The modules may be anything
-    that can be called: nothing of them is read before they are known to be plain.)"""
+def _narrow_pair(x: torch.Tensor, first: nn.Module, second: nn.Module):
+    """The weights of the pair if ``tf_narrow_linear2`` takes it, else None.  (The
+    modules may be anything that can be called: nothing of them is read before they
+    are known to be plain.)"""
     if not (_plain(first, nn.Linear) and _plain(second, nn.Linear)):
-        return False
-    n, k = first.weight.shape
-    if torch.is_grad_enabled() and (x.requires_grad or first.weight.requires_grad
-                                    or second.weight.requires_grad):
-        return False
+        return None
+    pair = w0, w1 = first.weight, second.weight
+    n, k = w0.shape
+    if torch.is_grad_enabled() and (x.requires_grad or w0.requires_grad or w1.requires_grad):
+        return None
     if (torch.is_autocast_enabled() or not x.is_cuda or x.dim() != 2
             or x.dtype != torch.bfloat16 or x.shape[0] == 0 or n > 64 or k % 32
-            or x.shape[1] != k or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16):
-        return False
-    return all(m.bias is None and m.weight.shape == (n, k) and m.weight.dtype == torch.bfloat16
-               and m.weight.device == x.device and m.weight.is_contiguous()
-               and m.weight.data_ptr() % 16 == 0 for m in (first, second))
+            or x.shape[1] != k or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16
+            or first.bias is not None or second.bias is not None):
+        return None
+    for w in pair:
+        if (w.shape != (n, k) or w.dtype != torch.bfloat16 or w.device != x.device
+                or not w.is_contiguous() or w.data_ptr() % 16):
+            return None
+    return pair
 
 
 def narrow_linears(x: torch.Tensor, first: nn.Linear, second: nn.Linear):
@@ -271,17 +275,18 @@ def narrow_linears(x: torch.Tensor, first: nn.Linear, second: nn.Linear):
     Linears that are more than plain bf16 ``nn.Linear`` calls without a bias, that
     autograd is to record or autocast to cast, or whose sizes the kernel does not
     take are called one by one (``amax_partials`` is then None)."""
-    if not _narrow_pair(x, first, second):
+    pair = _narrow_pair(x, first, second)
+    if pair is None:
         return first(x), second(x), None
-    n, k = first.weight.shape
+    n, k = pair[0].shape
     rows = x.shape[0]
     outs = [torch.empty((rows, n), dtype=torch.bfloat16, device=x.device) for _ in range(2)]
     blocks = _native.load().tf_narrow_linear2_blocks(rows)
     partials = None
     if 0 < blocks <= _native.TF_FP8_QUANT_WORKSPACE_BYTES // 4:
         partials = torch.empty((blocks,), dtype=torch.int32, device=x.device)
-    _native.call("tf_narrow_linear2", _ptr(x), x.stride(0), rows, k, _ptr(first.weight),
-                 _ptr(second.weight), n, _ptr(outs[0]), _ptr(outs[1]), n, _ptr(partials),
+    _native.call("tf_narrow_linear2", _ptr(x), x.stride(0), rows, k, _ptr(pair[0]),
+                 _ptr(pair[1]), n, _ptr(outs[0]), _ptr(outs[1]), n, _ptr(partials),
                  _stream_ptr(None, x.device))
     return outs[0], outs[1], partials
 
