@@ -380,3 +380,23 @@ def test_narrow_linears_call_what_is_not_plain(gpu):
     lins[1].requires_grad_(True)
     out = fl.narrow_linears(x, *lins)
     assert out[2] is None and out[1].requires_grad
+
+
+@pytest.mark.parametrize("k", [2048, 3072])
+def test_narrow_linears_of_many_rows(gpu, k):
+    """On either side of the line above which the modules run: the same products,
+    and FP8 linears that find the input's amax by themselves."""
+    rows = fl.NARROW_MAX_ELEMS // k
+    x = torch.randn((rows + 1, k), device=gpu, dtype=torch.bfloat16)
+    lins = [torch.nn.Linear(k, 6, bias=False, dtype=torch.bfloat16, device=gpu)
+            .requires_grad_(False) for _ in range(2)]
+    lin = fl.Fp8Linear(k, 128).to(gpu)
+    lin.quantize_from(torch.randn((128, k), device=gpu) * k ** -0.5)
+    for n, shared in ((rows, True), (rows + 1, False)):
+        first, second, amax = fl.narrow_linears(x[:n], *lins)
+        assert (amax is not None) == shared
+        for got, m in zip((first, second), lins):
+            # one bf16 rounding (2^-9) and fp32 sums of k terms of about 1/sqrt(k) each
+            ref = x[:n][-2000:].double() @ m.weight.double().t()
+            assert torch.allclose(got[-2000:].double(), ref, rtol=2 ** -8, atol=1e-5)
+        assert torch.equal(fl.fp8_linears(x[:n], [lin], amax)[0], lin(x[:n]))

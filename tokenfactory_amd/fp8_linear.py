@@ -246,6 +246,15 @@ def _plain(linear, kind) -> bool:
                      or nn.modules.module._has_any_global_hook()))
 
 
+# Elements of x up to which the gate projections share a launch.  Above, the
+# library's two products and a pass for max |x| are faster: its kernel re-reads x for
+# each 32 columns of either weight, from memory once x outgrows the caches
+# (hidden 5120, 48 + 48 columns, us shared / two products + pass: 4000 rows 37 / 51,
+# 5000 53 / 53, 8000 73 / 56, 16000 142 / 91; hidden 8192, 64 + 64: 3000 62 / 69,
+# 5000 93 / 63; hidden 2048, 32 + 32: 12000 32 / 51).
+NARROW_MAX_ELEMS = 24 << 20
+
+
 def _narrow_pair(x: torch.Tensor, first: nn.Module, second: nn.Module):
     """The weights of the pair if ``tf_narrow_linear2`` takes it, else None.  (The
     modules may be anything that can be called: nothing of them is read before they
@@ -257,8 +266,8 @@ def _narrow_pair(x: torch.Tensor, first: nn.Module, second: nn.Module):
     if torch.is_grad_enabled() and (x.requires_grad or w0.requires_grad or w1.requires_grad):
         return None
     if (torch.is_autocast_enabled() or not x.is_cuda or x.dim() != 2
-            or x.dtype != torch.bfloat16 or x.shape[0] == 0 or n > 64 or k % 32
-            or x.shape[1] != k or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16
+            or x.dtype != torch.bfloat16 or not 0 < x.numel() <= NARROW_MAX_ELEMS or n > 64
+            or k % 32 or x.shape[1] != k or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16
             or first.bias is not None or second.bias is not None):
         return None
     for w in pair:
