@@ -14,7 +14,7 @@ import torch.nn.functional as F
 from tests.helpers import assert_attn_close, restatement, small_case
 from tests.test_gpu_gate import assert_bits_match, module_gate
 from tokenfactory_amd import _native, slot_based_attention, workloads
-from tokenfactory_amd.attention import SHORT_ROWS, Route, SlotAttentionCall
+from tokenfactory_amd.attention import SHORT_ROWS, TINY_CONTEXT, Route, SlotAttentionCall
 
 pytestmark = pytest.mark.gpu
 
@@ -67,6 +67,46 @@ def test_other_head_dims(gpu, d, fp8):
     dim is not a multiple of 16 stays on the one-wave-per-row kernel."""
     check(case(gpu, [90, 400, 7, 1900, 64], [90, 1, 3, 1, 20], 8, 2, d, d, fp8), "mixed")
     check(case(gpu, [500, 31], [1, 1], 20, 1, d, d, fp8), "decode, G = 20")
+
+
+@pytest.mark.parametrize("d,fp8", [(64, False), (128, False), (128, True), (72, False)])
+@pytest.mark.parametrize("longest", [1, TINY_CONTEXT, TINY_CONTEXT + 1])
+def test_tiny_contexts(gpu, d, fp8, longest):
+    """Decodes on either side of TINY_CONTEXT, eager; a step captured on tiny contexts
+    replays on long ones."""
+    seq = [longest, 1, max(longest - 1, 1)]
+    wl = case(gpu, seq, [1] * 3, 8, 2, d, d, fp8)
+    check(wl, f"longest {longest}")
+    gate = module_gate(wl, d)
+    amax = torch.zeros(1, dtype=torch.int32, device=gpu)
+    fused = run(wl, gate=gate, out_amax=amax)
+    want = (run(wl) * F.silu(gate)).float()
+    # one bf16 ulp of silu (at most 2^-7 relative) and the product's two roundings
+    # (2^-9 each), as in assert_bits_match, whose count of differing elements
+    # (one in a thousand) needs more elements than these few rows have
+    assert ((fused.float() - want).abs() <= 3 * 2.0 ** -8 * want.abs()).all()
+    assert int(amax) == int(fused.abs().max().view(torch.int16))
+    long = workloads.build("rows", [600, 3, 77], [1] * 3, num_q_heads=8, num_kv_heads=2, head_dim=d,
+                           pool_slots=wl.k_pool.shape[0] + 2000, device=gpu, seed=d, kv_fp8=fp8)
+    table = torch.full_like(long.batch.req_to_token, -1)
+    wl.k_pool, wl.v_pool, wl.batch.req_to_token = long.k_pool, long.v_pool, table
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = run(wl)
+    wl.q.copy_(long.q)
+    table.copy_(long.batch.req_to_token)
+    wl.batch.req_pool_indices.copy_(long.batch.req_pool_indices)
+    wl.batch.seq_lens.copy_(long.batch.seq_lens)
+    if fp8:
+        wl.k_scale.copy_(long.k_scale)
+        wl.v_scale.copy_(long.v_scale)
+    for i in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_attn_close(out, restatement(long), what=f"replay {i}")
 
 
 def test_strided_q_out_gate_and_amax(gpu):
