@@ -201,3 +201,19 @@ def test_rows_workspace_is_bounded_by_the_grid(hq, hkv, d, kv_dtype):
         assert sizes[-1] <= 2 * grid * 32 * (4 * width + 8) + 256 + 4 * (2049 + 2048 * hkv)
     # the default grid: one workgroup per CU, two of the 128-dim kernel
     assert cus <= 2 * 512 * 32 * (4 * 128 + 8) + 256 + 4 * (2049 + 2048 * hkv)
+
+
+@pytest.mark.parametrize("source,message", [
+    (f"int tf_attn_abi_version(void) {{ return {_native.ABI_VERSION - 1}; }}",
+     f"ABI version {_native.ABI_VERSION - 1}, expected {_native.ABI_VERSION}"),
+    (f"int tf_attn_abi_version(void) {{ return {_native.ABI_VERSION}; }}", "has no tf_"),
+    ("int other(void) { return 0; }", "has no tf_attn_abi_version"),
+])
+def test_a_library_of_another_version_is_refused_as_such(tmp_path, source, message):
+    """Before its missing entry points are looked up."""
+    (tmp_path / "old.c").write_text(source + "\n")
+    lib = tmp_path / "libold.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(tmp_path / "old.c")],
+                   check=True)
+    with pytest.raises(_native.NativeLibraryError, match=message):
+        _native.load(lib)

@@ -14,7 +14,7 @@ from typing import Optional
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libtf_attn.so"
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 TF_DTYPE_BF16 = 0
 TF_DTYPE_FP8_E4M3 = 1
@@ -250,13 +250,20 @@ def load(path: Optional[Path] = None) -> ctypes.CDLL:
             lib = ctypes.CDLL(str(target))
         except OSError as exc:
             raise NativeLibraryError(f"cannot load {target}: {exc}") from exc
-        for name, (res, args) in SIGNATURES.items():
-            fn = getattr(lib, name)
-            fn.restype = res
-            fn.argtypes = args
-        ver = lib.tf_attn_abi_version()
+        # (the version first: a library of another one may lack entry points)
+        version = getattr(lib, "tf_attn_abi_version", None)
+        if version is None:
+            raise NativeLibraryError(f"{target} has no tf_attn_abi_version")
+        version.restype, version.argtypes = SIGNATURES["tf_attn_abi_version"]
+        ver = version()
         if ver != ABI_VERSION:
             raise NativeLibraryError(f"{target}: ABI version {ver}, expected {ABI_VERSION}")
+        for name, (res, args) in SIGNATURES.items():
+            fn = getattr(lib, name, None)
+            if fn is None:
+                raise NativeLibraryError(f"{target} has no {name}")
+            fn.restype = res
+            fn.argtypes = args
         if path is None:
             _lib = lib
         return lib

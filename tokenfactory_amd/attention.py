@@ -162,6 +162,12 @@ def _plan_event(device: torch.device, stream: torch.cuda.Stream) -> torch.cuda.E
 
 
 SPLIT_KEYS = 896     # shortest context whose extend entries may be split over keys
+# Longest context up to which a decode step at another head dim than 256 runs the
+# one-wave-per-row kernel: one launch without a merge, but one key after another
+# (16 / 4 heads of 64, 8 requests: 16 keys 7.2 us and 10.5 with the streaming
+# kernel, 32 keys 9.7 and 12.0, 64 keys 16.0 and 12.3; 32 / 8 of 128 the same).  Not in
+# a captured step, whose replays may have other lengths.
+TINY_CONTEXT = 40
 SHORT_ROWS = 64      # query rows per kv head up to which an extend takes the streaming kernel
 MAX_ROW_ITEMS = 2048
 
@@ -266,10 +272,9 @@ class Route:
             self.max_rows = 1 << 62
             self.row_groups = 2 if n_work else 1   # blocks whenever the step is planned
             unit = 16 * self.row_groups
-            if exact:
-                self.n_blocks = sum(_n_units(e, group, unit) for e in ext_lens)
-            else:
-                self.n_blocks = n_tok * group // unit + (n_work // n_kv if n_work else 0) + bsz
+            if n_work:   # (a step that is not planned has no list)
+                self.n_blocks = (sum(_n_units(e, group, unit) for e in ext_lens) if exact else
+                                 n_tok * group // unit + n_work // n_kv + bsz)
             self.run_extend = False
             return
         n_dec = sum(1 for e in ext_lens if e == 1)
@@ -578,6 +583,7 @@ class SlotAttentionCall:
         self.ws = None                # split scratch of the last launch
         self._ws_bytes = 0
         self._ws_stream = None        # whose shared scratch self.ws is (None: a graph's own)
+        self._tiny = False
         self._n_rows_items = 0   # items of the tf_attn_rows launch (0: tf_attn_decode)
         if n_tok == 0:
             return
@@ -655,6 +661,7 @@ class SlotAttentionCall:
                 raise NotImplementedError(f"decode: {bsz} requests in one call (at most "
                                           f"{MAX_ROW_ITEMS})")
             self._n_rows_items = self.route.n_blocks if has_blocks else bsz
+            self._tiny = head_dim != 256 and not self.n_work and self.max_len <= TINY_CONTEXT
             nbytes = _native.rows_workspace_bytes(has_blocks, self._n_rows_items,
                                                   self.route.row_groups, n_q, n_kv, head_dim,
                                                   kv_dtype, self.decode_workgroups)
@@ -744,6 +751,13 @@ class SlotAttentionCall:
         if self._n_rows_items:
             if entry == "tf_attn_decode_merge":
                 return   # part of the rows launch
+            if self._tiny and self._ws_stream is not None:
+                _native.call("tf_attn_decode", self.q.data_ptr(), self.q.stride(0),
+                             *self._pool_args, None, None, self.n_dec, self.n_q, self.n_kv,
+                             self.head_dim, self.scaling, self.out.data_ptr(),
+                             self.out.stride(0), None, 0, self.max_len, 0,
+                             *self._epilogue_args, handle)
+                return
             self._host_lists()
             _native.call("tf_attn_rows", self.q.data_ptr(), self.q.stride(0), *self._pool_args,
                          _ptr(self._lists), self._n_rows_items, self.route.row_groups,

@@ -49,7 +49,7 @@ int device_cu_count() {
 
 extern "C" {
 
-int32_t tf_attn_abi_version(void) { return 12; }
+int32_t tf_attn_abi_version(void) { return 13; }
 
 const char* tf_attn_last_error(void) { return tfa::g_err; }
 
