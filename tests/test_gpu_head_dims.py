@@ -96,6 +96,40 @@ def test_fused_gate(gpu, d):
     assert_bits_match(fused, plain * F.silu(gate), f"gate D={d}")
 
 
+@pytest.mark.parametrize("d", [64, 128, 200])
+@pytest.mark.parametrize("ext", [[1, 1], [40, 1]])
+def test_probabilities_keep_their_24_bits(gpu, d, ext):
+    """Two keys whose weights p differ by about 2^-14 of them and whose values cancel:
+    the output is the difference.  A probability in two bf16 parts is off by up to
+    2^-18, a sixteenth of the difference."""
+    wl = small_case([e + 60 for e in ext], ext, hq=8, hkv=1, d=d, seed=d, device=gpu,
+                    dtype=torch.bfloat16)
+    n = wl.q.shape[0]
+    wl.k_pool.zero_()
+    wl.v_pool.zero_()
+    wl.q.zero_()
+    g = torch.Generator().manual_seed(d)
+    x = (0.3 + 1.2 * torch.rand((n, 8), generator=g)).to(torch.bfloat16)
+    e = (2.0 ** -14 * (1 + torch.rand((n, 8), generator=g))).to(torch.bfloat16)
+    wl.q[..., 0], wl.q[..., 1] = x.to(gpu), e.to(gpu)
+    for r, length in zip(wl.rows, wl.seq_lens):
+        slots = wl.batch.req_to_token[r, :length]
+        wl.k_pool[slots, 0, 0] = -200                  # no weight
+        wl.k_pool[slots[0], 0, 0] = 0                  # the largest score: 0
+        wl.k_pool[slots[5:7], 0, 0] = -1               # scores -x and -x - e
+        wl.k_pool[slots[6], 0, 1] = -1
+        wl.v_pool[slots[5]], wl.v_pool[slots[6]] = 1, -1
+    wl.scale = 1.0
+    out = run(wl).double().cpu()
+    x, e = x.double(), e.double()
+    pa, pb = torch.exp(-x), torch.exp(-x - e)
+    want = ((pa - pb) / (1 + pa + pb))[..., None]
+    # of a difference of 2^-14: each exponent's rounding (2^-25 of up to 2 log2 e) and each
+    # exp2's ulp (2^-24), and the output's bf16 rounding
+    tol = 2 * (2.0 ** -24 * 1.5 + 2.0 ** -24) / 2.0 ** -14 + 2.0 ** -8
+    assert ((out / want - 1).abs() <= tol).all(), (out / want - 1).abs().max()
+
+
 def test_rejects_head_dims_that_are_not_multiples_of_8(gpu):
     wl = small_case([10], [1], hq=4, hkv=1, d=36, seed=1, device=gpu, dtype=torch.bfloat16)
     with pytest.raises(NotImplementedError):

@@ -94,14 +94,14 @@ struct DecodeArgs {
   bool by_owner;      // partial slots: two per workgroup (else one per workgroup and unit)
 };
 
-// The kernels' shape (NG = 1 or 2: four groups of 256 dims spill).  DP: head dims in a row's tile (256, or 128 for head dims
-// up to 128); NG: groups of 16 query rows a unit holds; OTHER: head dims that do
-// not fill the tile (chunks past the head dim are read as zeros and not
-// written) and probabilities split into bf16 high and low parts, which the PV
-// product takes one after the other (about 2^-17 relative error: the kernel these
-// head dims ran before kept them in fp32).  BLK: items are row blocks
-// (DecodeArgs::blocks); else one token each, and every row sees every key of
-// its item.
+// The kernels' shape.  DP: head dims in a row's tile (256, or 128 for head dims up
+// to 128); NG: groups of 16 query rows a unit holds (1 or 2: four groups of 256 dims
+// spill); OTHER: head dims that do not fill the tile (chunks past the head dim are
+// read as zeros and not written) and probabilities split into three bf16 parts, all
+// of their 24 bits, which the PV product takes one after the other, smallest first
+// (the kernel these head dims ran before kept them in fp32; two parts are off by up
+// to 2^-18 and 1 to 5 % faster).  BLK: items are row blocks (DecodeArgs::blocks);
+// else one token each, and every row sees every key of its item.
 template <int DP_, bool FP8_, int NG_, bool OTHER_, bool BLK_>
 struct Cfg {
   static constexpr int DP = DP_;
@@ -328,11 +328,12 @@ __device__ __forceinline__ void k_frags(const u32x4* ks, int g, int n, u32x4 (&k
 // S^T = K Q^T for the tile, then the online-softmax update of group q's row n,
 // whose visible tokens are those below lim (chunk-local); returns the tile's
 // probabilities packed as the PV B operand (P^T, 4 tokens per lane), pl their
-// low parts (OTHER).
+// lower parts, smallest first (OTHER).
 template <class C>
 __device__ __forceinline__ u32x2 qk_softmax(const u32x4 (&kf)[C::kSteps],
                                             const u32x4 (&qf)[C::kSteps], int it, int lim, int g,
-                                            float sl2, WaveState<C>& st, int q, u32x2& pl) {
+                                            float sl2, WaveState<C>& st, int q,
+                                            u32x2 (&pl)[2]) {
   f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kk = 0; kk < C::kSteps; ++kk) sacc = mfma_16x16x32(kf[kk], qf[kk], sacc);
@@ -364,21 +365,30 @@ __device__ __forceinline__ u32x2 qk_softmax(const u32x4 (&kf)[C::kSteps],
     for (int i = 0; i < C::kAcc; ++i) st.acc[q][i] *= alpha;
   }
   const u32x2 ph = {pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
-  if (C::OTHER)
-    pl = u32x2{pack_bf16(p[0] - bf16_lo(ph[0]), p[1] - bf16_hi(ph[0])),
-               pack_bf16(p[2] - bf16_lo(ph[1]), p[3] - bf16_hi(ph[1]))};
+  if (C::OTHER) {   // (the differences are exact)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] -= r & 1 ? bf16_hi(ph[r >> 1]) : bf16_lo(ph[r >> 1]);
+    pl[1] = u32x2{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] -= r & 1 ? bf16_hi(pl[1][r >> 1]) : bf16_lo(pl[1][r >> 1]);
+    pl[0] = u32x2{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
+  }
   return ph;
 }
 
 // O^T += V^T P^T for the tile, every group.
 template <class C>
 __device__ __forceinline__ void pv(const VBuf<C>& vb, const u32x2 (&pt)[C::NG],
-                                   const u32x2 (&pl)[C::NG], WaveState<C>& st, int n_groups) {
+                                   const u32x2 (&pl)[C::NG][2], WaveState<C>& st,
+                                   int n_groups) {
   auto mma = [&](int i, u32x2 va) {
 #pragma unroll
     for (int q = 0; q < C::NG; ++q) {
       if (C::NG > 1 && q >= n_groups) break;
-      if (C::OTHER) st.acc[q][i] = mfma_16x16x16(va, pl[q], st.acc[q][i]);
+      if (C::OTHER) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) st.acc[q][i] = mfma_16x16x16(va, pl[q][k], st.acc[q][i]);
+      }
       st.acc[q][i] = mfma_16x16x16(va, pt[q], st.acc[q][i]);
     }
   };
@@ -626,7 +636,7 @@ decode_kernel(DecodeArgs a) {
         VBuf<C> vb;
         const int32_t* slots = sm.u.loop.slots;
         u32x4* ks = sm.u.loop.kstage[w];
-        auto scores = [&](int it, u32x2 (&pt)[C::NG], u32x2 (&pl)[C::NG]) {
+        auto scores = [&](int it, u32x2 (&pt)[C::NG], u32x2 (&pl)[C::NG][2]) {
           u32x4 kf[C::kSteps];
           k_frags<C>(ks, g, n, kf);
 #pragma unroll
@@ -636,10 +646,11 @@ decode_kernel(DecodeArgs a) {
         #pragma unroll
               for (int kk = 0; kk < C::kSteps; ++kk) qf[kk] = sm.qfrag[q][kk][lane];
             }
-            pt[q] = qk_softmax<C>(kf, qf, it, C::BLK ? min(n_loc, seen[q] - c0) : n_loc, g, sl2, st, q, pl[q]);
+            const int lim = C::BLK ? min(n_loc, seen[q] - c0) : n_loc;
+            pt[q] = qk_softmax<C>(kf, qf, it, lim, g, sl2, st, q, pl[q]);
           }
         };
-        u32x2 pt[C::NG], pl[C::NG];
+        u32x2 pt[C::NG], pl[C::NG][2];
         issue_rows<C>(kb.k, slots, it, n_loc, g, n, kbase, slot_bytes, n_chunks);
         issue_rows<C>(vb.v, slots, it, n_loc, g, n, vbase, slot_bytes, n_chunks);
         for (; it + kWaves < n_tiles; it += kWaves) {
