@@ -199,9 +199,10 @@ def test_extend_matches_oracle(gpu, lens, hk, hv):
 @pytest.mark.parametrize("lens", [[237], [236], [1, 300, 1], [1, 31, 512], [512, 512],
                                   [3] * 20 + [600] + [2] * 20 + [1] * 5])
 def test_split_columns_match_oracle(gpu, lens):
-    """Few long prompts (two workgroups per value head) at the rule's edge, beside
-    short requests, and with more (request, head) items than workgroups; the
-    second call of each case, with half the lengths, is the other kernel's."""
+    """Few long prompts (two workgroups per value head; 236 tokens are one below the
+    rule's edge), beside short requests, and with more (request, head) items than
+    workgroups.  The second call of a case has half the lengths: whole heads for
+    [237], [1, 300, 1] and [512, 512]."""
     test_extend_matches_oracle(gpu, lens, 4, 12)
 
 

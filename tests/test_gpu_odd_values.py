@@ -76,3 +76,25 @@ def test_gate_and_amax_with_odd_values(gpu):
     assert not fin.all() and torch.equal(fused.isfinite(), fin)
     assert ((fused - want).abs()[fin] <= 2 ** -7 * want.abs()[fin] + 1e-6).all()
     assert int(amax) == int(fused.to(torch.bfloat16).abs().view(torch.int16).max())
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("seq,ext", [([700, 90], [1, 1]), ([400, 900], [4, 10]),
+                                     ([1600, 300], [60, 1]), ([2000], [30])])
+def test_visible_values_pass_through_merges(gpu, seq, ext, fp8):
+    """At 256 dims: NaN and infinite V values that every row of a request sees, through
+    units cut over workgroups, row blocks and split extend entries."""
+    wl = workloads.build("odd", seq, ext, num_q_heads=12, num_kv_heads=2, head_dim=256,
+                         pool_slots=4096, device=gpu, seed=sum(seq), kv_fp8=fp8)
+    values = [math.nan] if fp8 else [math.nan, math.inf, -math.inf]
+    for b, n in enumerate(seq):
+        for i, v in enumerate(values):
+            slot = int(wl.batch.req_to_token[wl.rows[b], 3 + 17 * i])
+            pool = wl.v_pool.view(torch.uint8) if fp8 else wl.v_pool
+            odd = torch.full((1,), v, device=gpu)
+            pool[slot, 0, 5 + 100 * i] = (odd.to(torch.float8_e4m3fn).view(torch.uint8) if fp8
+                                          else odd.to(torch.bfloat16))[0]
+    ref = torch.from_numpy(brute(wl, dense=True)).float()
+    print(f"[odd] D=256 L={seq} ext={ext} fp8={fp8}", flush=True)
+    for workgroups in (0, 40):
+        check(run(wl, decode_workgroups=workgroups), ref, f"{workgroups} workgroups")

@@ -13,8 +13,8 @@ import torch.nn.functional as F
 
 from tests.helpers import assert_attn_close, restatement, small_case
 from tests.test_gpu_gate import assert_bits_match, module_gate
-from tokenfactory_amd import _native, slot_based_attention, workloads
-from tokenfactory_amd.attention import SHORT_ROWS, TINY_CONTEXT, Route, SlotAttentionCall
+from tokenfactory_amd import slot_based_attention, workloads
+from tokenfactory_amd.attention import MAX_ROW_ITEMS, SHORT_ROWS, TINY_CONTEXT, SlotAttentionCall
 
 pytestmark = pytest.mark.gpu
 
@@ -177,18 +177,24 @@ def test_block_lists(gpu, d, lens, device_plan):
     assert (gp[len(pieces):] == 0).all()
 
 
-def test_more_blocks_than_one_launch_takes(gpu):
+@pytest.mark.parametrize("exts,hq,hkv,d", [
+    ([1100, 700, 1, 900], 64, 4, 64),            # 1351 blocks: one launch
+    ([2500], 64, 1, 32),                         # 5000: three
+    ([1] * 2060 + [40, 7] * 4, 8, 2, 64),        # 2084: decodes and extends past the 2048th
+])
+def test_more_blocks_than_one_launch_takes(gpu, exts, hq, hkv, d):
     """Above 2048 blocks the rows kernel is launched over parts of the list."""
-    lens = [1100, 700, 1, 900]
-    wl = small_case([e + 30 for e in lens], lens, hq=64, hkv=4, d=64, seed=3, device=gpu,
-                    dtype=torch.bfloat16)
-    r = Route(lens, sum(lens), 64, 4, 64, _native.TF_DTYPE_BF16, 4 * 177, exact=True)
-    assert r.n_blocks > 512
-    check(wl, "many blocks")
-    calls = SlotAttentionCall(wl.q, wl.k_pool, wl.v_pool, wl.batch, scaling=wl.scale)
-    calls.run()
-    two = case(gpu, [2500 + 1], [2500], 64, 1, 32, 9)
-    check(two, "2500 rows of 64 heads")
+    wl = case(gpu, [e + i % 5 for i, e in enumerate(exts)], exts, hq, hkv, d, len(exts))
+    call = SlotAttentionCall(wl.q, wl.k_pool, wl.v_pool, wl.batch, scaling=wl.scale)
+    out = call.run()
+    torch.cuda.synchronize()
+    blocks = call._lists.cpu().numpy()[:4 * call.route.n_blocks].reshape(-1, 4)
+    real = int((blocks[:, 0] >= 0).sum())
+    assert real == call.route.n_blocks == sum(-(-e * (hq // hkv) // 32) for e in exts)
+    assert (real > MAX_ROW_ITEMS) == (len(exts) != 4)
+    if len(exts) > 4:
+        assert (blocks[MAX_ROW_ITEMS:, 2] == 1).any() and (blocks[MAX_ROW_ITEMS:, 2] > 1).any()
+    assert torch.equal(check(wl, f"{real} blocks"), out)
 
 
 @pytest.mark.parametrize("fp8", [False, True])
