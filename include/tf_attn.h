@@ -310,10 +310,10 @@ int32_t tf_attn_rows(
  * at most one piece per compute unit), for tf_attn_extend_split with the merge
  * entries [n_merges][8], padded with zeros; n_pieces >= the compute units,
  * n_merges >= 1 (entries that it has no room for stay whole: the number of
- * entries, or half of the compute units, is always enough), seq_lens, seq_len_override and rtt_cols are the
- * launch's, and key_bytes is the size of a token's K and V in the pool (what the
- * step's streaming rows, given as dec_items also where n_blocks is 0, will read
- * counts against a split).
+ * entries, or half of the compute units, is always enough), seq_lens,
+ * seq_len_override and rtt_cols are the launch's, and key_bytes is the size of a
+ * token's K and V in the pool (what the step's streaming rows, given as dec_items
+ * also where n_blocks is 0, will read counts against a split).
  */
 int32_t tf_attn_plan_blocks(const int32_t* work, int32_t n_work, const int32_t* dec_items,
                             const int32_t* dec_rows, int32_t n_dec, int32_t num_q_heads,
@@ -456,10 +456,10 @@ int32_t tf_qk_norm_rope_kv_write(const void* q, int64_t q_token_stride, int64_t 
  * out: bf16 [m, n], row stride out_row_stride elements (a multiple of 4),
  * 8-byte aligned.
  * workspace (optional, NULL allowed): when the output tiles alone leave most
- * compute units idle the call splits K over several workgroups per tile if it gets tf_fp8_block_gemm_workspace_bytes(m,
- * n, k) bytes of 16-byte aligned scratch (fp32 partials, no initialisation
- * needed; the partials are summed in a fixed order, so results do not depend
- * on timing).  Without it (or when the size query returns 0) one workgroup
+ * compute units idle the call splits K over several workgroups per tile if it gets
+ * tf_fp8_block_gemm_workspace_bytes(m, n, k) bytes of 16-byte aligned scratch (fp32
+ * partials, no initialisation needed; the partials are summed in a fixed order, so
+ * results do not depend on timing).  Without it (or when the size query returns 0) one workgroup
  * covers each output tile.
  */
 #define TF_FP8_QUANT_WORKSPACE_BYTES 4096

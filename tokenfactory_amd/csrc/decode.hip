@@ -41,7 +41,7 @@
 // rows of any request at head dims other than 256.  Up to two groups of 16 rows
 // share every K / V tile a wave loads, each row masked at its own last key; the
 // group's softmax state and 64 (or 32) output dims per lane are all that grows.
-// 20 requests of 2 to 4 tokens on 1k to 8k keys stream 362 MB in 78 us.
+// 20 requests of 2 to 4 tokens on 1k to 8k keys stream 362 MB in 76 us.
 // The merge lives in its own launch so the streaming kernel needs no
 // device-scope fence (on gfx950 those write back and invalidate the XCD's L2).
 #include <math.h>
@@ -276,8 +276,13 @@ __device__ __forceinline__ uint32_t write_output(const DecodeArgs& a, int qrow, 
 // Issue the loads of tile `it` (chunk tokens it*16 .. it*16+15, clamped to the
 // chunk's last token so every address is a valid row): lane (g, n) reads chunk
 // n (+ 16 s) of the rows of tokens 4g + j, the same row-contiguous pattern for
-// K (the MFMA layout is produced through LDS) and V.  The rows are streamed
-// once, so the loads are nontemporal.  n_chunks: chunks of a row (OTHER).
+// K (the MFMA layout is produced through LDS) and V.  The loads are nontemporal:
+// one-token units stream every row once.  Blocks of one request read its rows
+// again, each for itself, and plain loads serve those better (2 prompts beside 12
+// decodes at 128 dims 94.8 and 84.2 us, 20 requests of 6 tokens at 256 153 and 143),
+// but cost steps of many rows that are read once more (64 decodes beside 3 tokens
+// 211 and 240, 64 requests of 5 tokens 232 and 256).  n_chunks: chunks of a row
+// (OTHER).
 template <class C>
 __device__ __forceinline__ void issue_rows(u32x4 (&x)[4][C::kS], const int32_t* slots, int it,
                                            int n_loc, int g, int n, const uint8_t* base,
@@ -834,8 +839,9 @@ decode_merge_kernel(DecodeArgs a) {
 #pragma unroll
         for (int k = 0; k < kMergeAhead; ++k) {
           const int bk = min(bb + WPR * k, b1);
-          const int64_t slot =
-              C::kRowPlan && a.by_owner ? 2 * (int64_t)bk + (inside && bk == b0 ? 1 : 0) : (int64_t)bk + u;
+          const int64_t slot = C::kRowPlan && a.by_owner
+                                   ? 2 * (int64_t)bk + (inside && bk == b0 ? 1 : 0)
+                                   : (int64_t)bk + u;
           const int64_t pr = slot * C::kRows + n;
           o[k] = reinterpret_cast<const f32x4*>(
               a.ws_o + pr * C::kRowFloats)[C::DP == 256 ? lane : lane & 31];
@@ -1097,7 +1103,8 @@ int launch_rows(const DecodeArgs& a, const DecodePlan& p, int phases, hipStream_
                           2 * device_cu_count();
     const int per_wg = wide ? kMergeWaves / kWaves : kMergeWaves;
     const bool many = p.n_units >= 2 * p.n_blocks;
-    const dim3 grid((unsigned)p.n_units, many ? 1u : (unsigned)((p.rows_used + per_wg - 1) / per_wg));
+    const dim3 grid((unsigned)p.n_units,
+                    many ? 1u : (unsigned)((p.rows_used + per_wg - 1) / per_wg));
     const dim3 block(kMergeWaves * kWave);
     if (wide)
       hipLaunchKernelGGL((decode_merge_kernel<C, kWaves>), grid, block, 0, s, a);
@@ -1173,7 +1180,8 @@ int decode_launch(const void* q, int64_t q_row_stride, const void* k_pool, const
            rtt_rows, rtt_row_stride, rtt_cols, req_pool_indices, seq_lens, seq_len_override,
            n_items, num_q_heads, num_kv_heads, head_dim, scale, out, out_row_stride, workspace,
            gate, gate_row_stride, gate_head_stride, out_amax, p);
-  if (kv_dtype == TF_DTYPE_FP8_E4M3) return launch_rows<Cfg<256, true, 1, false, false>>(a, p, phases, s);
+  if (kv_dtype == TF_DTYPE_FP8_E4M3)
+    return launch_rows<Cfg<256, true, 1, false, false>>(a, p, phases, s);
   return launch_rows<Cfg<256, false, 1, false, false>>(a, p, phases, s);
 }
 

@@ -682,7 +682,8 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
     // row's reference maximum (log2 units) and sum.
     const float l = row.l + __shfl_xor(row.l, 32, kWave);
     if (w_first < rows_total) {
-      f32x4* po = reinterpret_cast<f32x4*>(a.part_o) + ((int64_t)(part - 1) * kWaves + w) * 32 * kWave + lane;
+      f32x4* po = reinterpret_cast<f32x4*>(a.part_o) +
+                  ((int64_t)(part - 1) * kWaves + w) * 32 * kWave + lane;
 #pragma unroll
       for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
@@ -748,7 +749,8 @@ __global__ void __launch_bounds__(kThreads) extend_mfma_kernel(ExtendArgs a) {
 constexpr int kMergeAhead = 4;
 
 template <bool FP8>
-__global__ void __launch_bounds__(kThreads) extend_merge_kernel(ExtendArgs a, const int32_t* merges) {
+__global__ void __launch_bounds__(kThreads)
+extend_merge_kernel(ExtendArgs a, const int32_t* merges) {
   __shared__ __attribute__((aligned(16))) uint8_t rows[kTileBytes];
   const int32_t* mg = merges + 8 * (int64_t)blockIdx.x;
   const int ext = mg[4], G = a.group;

@@ -25,9 +25,9 @@
 // four weight matrices of the same input (a layer's projections), so a narrow
 // matrix fills the rounds of a wide one.  Each MFMA starts from zero and its
 // product is folded into the fp32 accumulator with that block's scale,
-// acc += p * s, one FMA per accumulator element per 128 of K; a row's folds run between the next row's
-// MFMAs, and each row's operand is read from LDS two rows ahead.  Per
-// 128-wide K slice the workgroup stages the weight tile (64 WN rows), the
+// acc += p * s, one FMA per accumulator element per 128 of K; a row's folds run
+// between the next row's MFMAs, and each row's operand is read from LDS two rows
+// ahead.  Per 128-wide K slice the workgroup stages the weight tile (64 WN rows), the
 // activation tile (32 MT rows) and the column scales straight from global
 // memory into LDS (global_load_lds_dwordx4 / global_load_lds_dword), STAGES - 1
 // slices ahead of the MFMAs, a few instructions per row of MFMAs.  Tiles are
@@ -452,7 +452,8 @@ fp8_gemm_kernel(GemmArgs a) {
       for (int tm = 0; tm < MT; ++tm) {
         const int m = m0 + xrow + 16 * tm;
         if (m < a.M)
-          *reinterpret_cast<f32x4*>(a.part + ((int64_t)split * a.M + m) * a.n_cols + mat.c0 + n) = acc[tm][tn];
+          *reinterpret_cast<f32x4*>(a.part + ((int64_t)split * a.M + m) * a.n_cols + mat.c0 +
+                                    n) = acc[tm][tn];
       }
     }
     return;
@@ -820,7 +821,8 @@ int32_t tf_fp8_linears(const void* x, int64_t x_row_stride, const uint32_t* amax
   if (need < 0) return (int32_t)need;
   if (m == 0) return TF_OK;
   if (!workspace || !aligned16(workspace) || workspace_bytes < need)
-    return fail(TF_ERR_INVALID, "fp8_linears: workspace of %lld bytes (needs %lld, 16-byte aligned)",
+    return fail(TF_ERR_INVALID,
+                "fp8_linears: workspace of %lld bytes (needs %lld, 16-byte aligned)",
                 (long long)workspace_bytes, (long long)need);
   if (amax_partials && ((reinterpret_cast<uintptr_t>(amax_partials) & 3u) || n_partials < 1 ||
                         n_partials > kQuantMaxBlocks))

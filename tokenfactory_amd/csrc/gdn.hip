@@ -1198,7 +1198,8 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_cols_ext_kernel(GdnArgs a) 
           for (int c = 0; c < 4; ++c) PR[c] = mfma_16x16x32(o[c][0], lo, PR[c]);
 #pragma unroll
           for (int c = 0; c < 4; ++c) PR[c] = mfma_16x16x32(o[c][0], hi, PR[c]);
-          if (kk + 1 < 4) split8(st[2 * kk + 2], st[2 * kk + 3], sh[(kk + 1) & 1], sl[(kk + 1) & 1]);
+          if (kk + 1 < 4)
+            split8(st[2 * kk + 2], st[2 * kk + 3], sh[(kk + 1) & 1], sl[(kk + 1) & 1]);
 #pragma unroll
           for (int q = 0; q < 12; ++q) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // 1 MFMA
@@ -1278,7 +1279,8 @@ __global__ void __launch_bounds__(kChunkThreads) gdn_cols_ext_kernel(GdnArgs a) 
         // O = e^gamma R + Bm Delta -> the output rows of this chunk
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
-          const u32x4* bp = reinterpret_cast<const u32x4*>(&I.rec[kRecB + (16 * mt + n) * kChunk + 8 * g]);
+          const u32x4* bp =
+              reinterpret_cast<const u32x4*>(&I.rec[kRecB + (16 * mt + n) * kChunk + 8 * g]);
           const f32x4 O = mma3s(f32x4{}, bp[0], bp[1], dh, dl);
 #pragma unroll
           for (int e = 0; e < 4; ++e)
