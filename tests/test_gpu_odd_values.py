@@ -62,20 +62,25 @@ def test_rows_depend_on_the_keys_they_see(gpu, d, fp8, where):
     check(run(wl, decode_workgroups=3), ref, "3 workgroups: whole units")
 
 
-def test_gate_and_amax_with_odd_values(gpu):
+@pytest.mark.parametrize("workgroups", [0, 2])
+@pytest.mark.parametrize("value", [math.inf, math.nan])
+def test_gate_and_amax_with_odd_values(gpu, value, workgroups):
+    """Of units cut over workgroups and of whole ones: out_amax comes from the outputs
+    alone."""
     wl = small_case([40, 100], [4, 1], hq=8, hkv=2, d=128, seed=3, device=gpu,
                     dtype=torch.bfloat16)
-    wl.v_pool[int(wl.batch.req_to_token[wl.rows[0], 39]), 0, 5] = math.inf
+    wl.v_pool[int(wl.batch.req_to_token[wl.rows[0], 39]), 0, 5] = value
     gate = torch.randn_like(wl.q)
     amax = torch.zeros(1, dtype=torch.int32, device=gpu)
-    plain = run(wl)
-    fused = run(wl, gate=gate, out_amax=amax)
+    plain = run(wl, decode_workgroups=workgroups)
+    fused = run(wl, gate=gate, out_amax=amax, decode_workgroups=workgroups)
     g = gate.float().cpu()
     want = plain * torch.nn.functional.silu(g)
     fin = want.isfinite()
     assert not fin.all() and torch.equal(fused.isfinite(), fin)
-    assert ((fused - want).abs()[fin] <= 2 ** -7 * want.abs()[fin] + 1e-6).all()
-    assert int(amax) == int(fused.to(torch.bfloat16).abs().view(torch.int16).max())
+    # one bf16 ulp of silu and the product's two roundings (tests/test_gpu_gate.py)
+    assert ((fused - want).abs()[fin] <= 3 * 2 ** -8 * want.abs()[fin]).all()
+    assert int(amax) == 0x7f80 if value == math.inf else int(amax) > 0x7f80
 
 
 @pytest.mark.parametrize("fp8", [False, True])

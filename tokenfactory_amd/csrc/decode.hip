@@ -688,10 +688,12 @@ decode_kernel(DecodeArgs a) {
     if (w == 0) {
       const bool whole = t0 == 0 && t1 == Ti;
       if constexpr (C::OTHER) {
-        // NaN or infinite V values: see decode_merge_kernel.
+        // NaN or infinite V values: the merge does such a unit's rows again, and
+        // writes them and their amax (see decode_merge_kernel).
         if (whole) {
           const bool odd = __ballot(any_odd<C>(st)) != 0;
           if (lane == 0) a.odd[(int64_t)item * units_per_item + j] = odd;
+          if (odd) continue;
         }
       }
       uint32_t om = 0;
