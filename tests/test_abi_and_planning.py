@@ -217,3 +217,12 @@ def test_a_library_of_another_version_is_refused_as_such(tmp_path, source, messa
                    check=True)
     with pytest.raises(_native.NativeLibraryError, match=message):
         _native.load(lib)
+
+
+def test_current_stream_without_the_raw_handle(monkeypatch):
+    """A torch that lacks the private accessor gets the handle from the Stream."""
+    import torch
+    stream = type("S", (), {"cuda_stream": 0x70})()
+    monkeypatch.setattr(_native, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: stream)
+    assert _native.current_stream(torch.device("cuda", 0)) == 0x70

@@ -283,11 +283,17 @@ def call(name: str, *args) -> int:
     return rc
 
 
+# (private to torch; a build without it pays for the Stream object)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def current_stream(device) -> int:
     """The handle of ``device``'s current stream (0 = the default stream), without
     the ``torch.cuda.Stream`` object that ``torch.cuda.current_stream`` makes
     (about 2 us per launch)."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def plan_device_capacity(total_tokens, batch_size, num_q_heads, num_kv_heads) -> int:

@@ -340,7 +340,8 @@ class StepPlan:
 
     A model step runs every full-attention layer over the same batch
     (``decoder_layer.py:68-69`` calls the attention once per layer), so the
-    lists do not change between layers; ``slot_based_attention`` keeps one
+    lists do not change between layers (nor with ``seq_lens``: a split entry's
+    pieces follow the lengths at launch); ``slot_based_attention`` keeps one
     ``StepPlan`` per (device, T, q heads, kv heads, head dim, pool dtype) on the
     batch object itself.  Calls on another stream than the planning one wait for
     the plan (an event recorded on the planning stream)."""
@@ -476,7 +477,10 @@ class _DevPtr:
 
 class SlotAttentionCall:
     """One planned ``_slot_based_attention`` step: validated arguments, uploaded
-    work lists and workspace, ready to launch (repeatedly) on ``stream``.
+    work lists and workspace, ready to launch (repeatedly) on ``stream``.  The
+    tensors that the kernels read (q, pools, ``req_to_token``, ``req_pool_indices``,
+    ``seq_lens``) may change in place between launches; the extend lengths may not,
+    except under ``device_plan``, which reads them from ``extend_lens_tensor``.
 
     ``run()`` enqueues every kernel of the step. For timing, ``run_extend()``,
     ``run_decode_partial()`` and ``run_decode_merge()`` enqueue the individual
